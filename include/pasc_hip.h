@@ -343,7 +343,10 @@ typedef struct {
                                 polish.block == 0 derives it from main (chunk / 2) */
 } pasc_launch_shape;
 
-/* Pin the launch shapes of later solves (the iterate is kept). */
+/* Pin the launch shapes of later solves (the iterate is kept).  Without a pinned shape a 1-D
+ * problem whose iterate and data fit on the chip (about 1.5 million steps at K = 3 in FP64, 3
+ * million in the FP32 phase) runs its iterations in one persistent launch instead, which has no
+ * shape to choose; a pinned shape is always run. */
 int pasc_set_launch_shape(pasc_problem *p, const pasc_launch_shape *shape);
 
 /* ---- autotuner ----

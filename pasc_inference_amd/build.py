@@ -31,6 +31,9 @@ def _units():
         for nt in (64, 128, 256, 512):
             units.append((os.path.join(CSRC, "pass_inst.hip"), f"pass_{s}_{nt}.o",
                           [f"-DPASS_S={s}", f"-DPASS_NT={nt}"]))
+        for nw in (4, 8):
+            units.append((os.path.join(CSRC, "loop_inst.hip"), f"loop_{s}_{nw}.o",
+                          [f"-DPASS_S={s}", f"-DLOOP_NW={nw}"]))
         units.append((os.path.join(CSRC, "grid_inst.hip"), f"grid_{s}.o", [f"-DPASS_S={s}"]))
         units.append((os.path.join(CSRC, "img_inst.hip"), f"img_{s}.o", [f"-DPASS_S={s}"]))
     units.append((os.path.join(CSRC, "engine.hip"), "engine.o", []))

@@ -1155,7 +1155,9 @@ int pasc_set_launch_shape(pasc_problem *p, const pasc_launch_shape *shape) {
     if (!p || !shape) return fail(PASC_ERR_ARG, "set_launch_shape: NULL argument");
     int rc = use_device(p->ctx);
     if (rc) return rc;
-    return set_shape(p->e, shape);
+    rc = set_shape(p->e, shape);
+    if (rc == PASC_OK) p->e.shape_pinned = true;
+    return rc;
 }
 
 int pasc_autotune(pasc_problem *p, const char *cache_path, pasc_launch_shape *shape) {

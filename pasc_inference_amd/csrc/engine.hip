@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "img_kernels.h"
+#include "loop_kernels.h"
 #include "spg_kernels.h"
 #include "step_kernels.h"
 #include "util_kernels.h"
@@ -46,6 +47,11 @@ int launch_pass_grid_float(int K, const GridArgs &a, int grid, hipStream_t s);
 int launch_pass_grid_double(int K, const GridArgs &a, int grid, hipStream_t s);
 int launch_pass_img_float(int K, const ImgArgs &a, int grid, int pd, hipStream_t s);
 int launch_pass_img_double(int K, const ImgArgs &a, int grid, int pd, hipStream_t s);
+
+int launch_loop_1d_float_4_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
+int launch_loop_1d_float_8_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
+int launch_loop_1d_double_4_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
+int launch_loop_1d_double_8_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
 
 // Images (T == 1 on the implicit 4-neighbour grid, whole rows, fewer than 2^31 nodes, every
 // instance's K rows within 4 GiB: the pass addresses them with 32-bit byte offsets) run the
@@ -584,8 +590,127 @@ static int img_data_terms(Engine &e, const void *x, S *q) {
     return PASC_OK;
 }
 
+// The persistent loop of a phase (loop_kernels.h): how many workgroups of how many waves with how
+// many steps per lane, or nwg = 0 when the problem does not run it.
+struct LoopPlan {
+    int nwg = 0, nw = 0, chunk = 0, tpw = 0, ntiles = 0;
+    int64_t epoch_words = 0;
+};
+
+template <typename S, int K, int CH>
+static bool loop_shape(int64_t T, int n_cu, LoopPlan &pl) {
+    using L = LoopShape<S, K, CH>;
+    const int64_t nt = (T + L::TILE - 1) / L::TILE;
+    const int64_t tpw = std::max<int64_t>((nt + n_cu - 1) / n_cu, LOOP_WAVES_MIN);
+    if (L::lds_bytes((int)std::min<int64_t>(tpw, 1 << 20)) > LOOP_LDS_BYTES) return false;
+    pl.tpw = (int)std::min(tpw, nt);
+    pl.ntiles = (int)nt;
+    pl.nwg = (int)((nt + pl.tpw - 1) / pl.tpw);
+    pl.nw = pl.tpw <= LOOP_WAVES_MIN ? LOOP_WAVES_MIN : LOOP_WAVES_MAX;
+    pl.chunk = CH;
+    pl.epoch_words = L::epoch_words(pl.nwg);
+    return true;
+}
+
+// The shorter chunk while every wave has one tile and a SIMD of its own, else the longer one
+// (fewer halo steps per owned step).
+template <typename S, int K>
+static void loop_shapes(int64_t T, int n_cu, LoopPlan &pl) {
+    constexpr bool f64 = sizeof(S) == 8;
+    if constexpr (loop_has_chunk(f64, K, 2)) {
+        LoopPlan two;
+        if (loop_shape<S, K, 2>(T, n_cu, two) &&
+            (two.tpw <= LOOP_WAVES_MIN || !loop_has_chunk(f64, K, 4))) {
+            pl = two;
+            return;
+        }
+    }
+    if constexpr (loop_has_chunk(f64, K, 4)) loop_shape<S, K, 4>(T, n_cu, pl);
+}
+
+static LoopPlan loop_plan(const Engine &e, bool f64) {
+    LoopPlan pl;
+    if (e.n_inst != 1 || e.stencil != STENCIL_TIME || e.profile || e.shape_pinned) return pl;
+    const InstDesc &d = e.h_desc[0];
+    const int n_cu = std::max(e.ctx->n_cu, 1);
+    switch (d.K) {
+#define PASC_LK(KK)                                        \
+    case KK:                                               \
+        if (f64) loop_shapes<double, KK>(d.T, n_cu, pl);   \
+        else loop_shapes<float, KK>(d.T, n_cu, pl);        \
+        break;
+        PASC_LK(1) PASC_LK(2) PASC_LK(3) PASC_LK(4) PASC_LK(5) PASC_LK(6) PASC_LK(7) PASC_LK(8)
+#undef PASC_LK
+    }
+    return pl;
+}
+
+// Runs a phase's passes in the persistent loop; *ran = false when the problem does not qualify or
+// the launch is refused (the tiled passes then go on from the state as it is).
+static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, bool *ran) {
+    *ran = false;
+    const LoopPlan pl = loop_plan(e, ph.f64);
+    if (pl.nwg == 0) return PASC_OK;
+    hipStream_t s = S_(e);
+    const int64_t cap = std::max<int64_t>(1, LOOP_EXCHANGE_BYTES / (8 * pl.epoch_words));
+    const int epochs = (int)std::min<int64_t>(std::min(max_passes, LOOP_EPOCHS_MAX), cap);
+    void *ex;
+    int rc = scratch(e, sizeof(double) * (size_t)pl.epoch_words * (epochs + 1), &ex);
+    if (rc) return rc;
+    const bool g64 = ph.f64 && e.precision == PASC_FP32_BULK;
+    int32_t *flags = e.h_nactive;
+    while (passes < max_passes) {
+        const int n = std::min(epochs, max_passes - passes);
+        const int64_t words = pl.epoch_words * (n + 1);
+        hipLaunchKernelGGL(fill_u64, dim3((unsigned)std::min<int64_t>((words + 255) / 256, 1024)),
+                           dim3(256), 0, s, (uint64_t *)ex, words, PART_EMPTY);
+        HIP_TRY(hipGetLastError());
+        LoopArgs a{};
+        a.p.gamma0 = g64 ? e.d_gamma64[0] : e.d_gamma[0];
+        a.p.gamma1 = g64 ? e.d_gamma64[1] : e.d_gamma[1];
+        a.p.x = ph.f64 ? e.d_x64 : e.d_x32;
+        a.p.b = ph.f64 ? e.d_b64 : e.d_b32;
+        a.p.desc = e.d_desc;
+        a.p.state = e.d_state;
+        a.p.kkt_every = ph.kkt_every;
+        a.p.need_f = ph.sp.fx_identity ? 0 : 1;
+        a.p.sp = ph.sp;
+        a.ex = (double *)ex;
+        a.flags = flags;
+        a.ntiles = pl.ntiles;
+        a.tpw = pl.tpw;
+        a.epochs = n;
+        // a residual that no stop test reads is only reported: it is formed for the last iterate
+        a.kkt_last = !ph.sp.fp32_phase && ph.kkt_every <= 1 && !(ph.sp.stop_mask & PASC_STOP_KKT);
+        flags[0] = 1;
+        flags[1] = 0;
+        const int K = e.h_desc[0].K;
+        const bool small = pl.nw == LOOP_WAVES_MIN;
+        if (ph.f64)
+            rc = small ? launch_loop_1d_double_4_(K, a, pl.nwg, pl.chunk, s) : launch_loop_1d_double_8_(K, a, pl.nwg, pl.chunk, s);
+        else
+            rc = small ? launch_loop_1d_float_4_(K, a, pl.nwg, pl.chunk, s) : launch_loop_1d_float_8_(K, a, pl.nwg, pl.chunk, s);
+        if (rc) {
+            (void)hipGetLastError();
+            return PASC_OK;
+        }
+        HIP_TRY(hipStreamSynchronize(s));
+        if (flags[1]) return fail(PASC_ERR_HIP, "the workgroups of the persistent loop lost each other");
+        passes += n;
+        if (!flags[0]) break;
+    }
+    *ran = true;
+    return PASC_OK;
+}
+
 static int run_phase(Engine &e, const PhaseCfg &ph, const pasc_spg_params &p, int max_passes) {
     hipStream_t s = S_(e);
+    int passes = 0;
+    {
+        bool ran;
+        const int rc0 = run_loop(e, ph, passes, max_passes, &ran);
+        if (rc0 || ran) return rc0;
+    }
     if (e.cur_phase != (ph.f64 ? 1 : 0) || tile_len(e, ph.f64) != e.cur_tile) {
         int rc0 = engine_retile(e, ph.f64);
         if (rc0) return rc0;
@@ -624,7 +749,6 @@ static int run_phase(Engine &e, const PhaseCfg &ph, const pasc_spg_params &p, in
     GraphGuard gg;
     EventsGuard eg;
     std::vector<hipEvent_t> &evs = eg.ev;
-    int passes = 0;
     int rc = PASC_OK;
     while (passes < max_passes) {
         const int n = std::min(every, max_passes - passes);

@@ -156,6 +156,7 @@ struct Engine {
                                          // fused step (DONE_BYTES, single problems only)
     int32_t *h_nactive = nullptr;        // pinned mirror
     PassShape sh[2];                     // [0] FP32 phase of FP32-bulk, [1] every FP64 pass
+    bool shape_pinned = false;           // the caller pinned sh: the tiled passes run it
     int grid_cap = 0;                    // persistent grid cap (0: 32 blocks per CU)
     int cur_tile = 0;                    // time steps per tile the partial slots are sized for
     int cur_phase = -1;                  // shape index the partial slots are sized for

@@ -132,16 +132,23 @@ __device__ __forceinline__ void exchange_edges(const C (&v)[K][CH], C *lds, C (&
     lds_barrier();
 }
 
-template <typename C>
-__device__ __forceinline__ C lap_half(C v, C vm, C vp, int64_t t, int64_t T, bool interior) {
-    // half of row t of A0 (blockgraphsparse.cpp:60-89) in difference form:
-    // (v_t - v_{t-1})[t>0] + (v_t - v_{t+1})[t<T-1]; the callers scale by 2*alpha (the factor
-    // 2 is exact, so (2 alpha) * s equals alpha * (2 s) bit for bit, one multiply fewer)
-    if (interior) return (v - vm) + (v - vp);
-    C a = C(0);
-    if (t > 0) a += v - vm;
-    if (t < T - 1) a += v - vp;
-    return a;
+// Half of the rows [t0, t0 + CH) of A0 (blockgraphsparse.cpp:60-89) in difference form,
+// (v_t - v_{t-1})[t>0] - (v_{t+1} - v_t)[t<T-1]; the callers scale by 2*alpha (the factor 2 is
+// exact, so (2 alpha) * s equals alpha * (2 s) bit for bit, one multiply fewer).  Each edge's
+// difference is formed once and serves both of its ends.
+template <typename C, int CH>
+__device__ __forceinline__ void lap_half(const C (&v)[CH], C vl, C vr, int64_t t0, int64_t T,
+                                         bool interior, C (&l)[CH]) {
+    C e[CH + 1];
+    e[0] = v[0] - vl;
+#pragma unroll
+    for (int c = 1; c < CH; c++) e[c] = v[c] - v[c - 1];
+    e[CH] = vr - v[CH - 1];
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        const int64_t t = t0 + c;
+        l[c] = (interior || t > 0 ? e[c] : C(0)) - (interior || t < T - 1 ? e[c + 1] : C(0));
+    }
 }
 
 // One tile of the fused pass.  INT: every step of the tile, halos included, lies in [1, T-2]
@@ -255,6 +262,180 @@ __device__ __forceinline__ void stage_read(const S *stage, int r, C (&v)[CH]) {
     }
 }
 
+// Sums of one thread's owned steps in the compute type, entering the FP64 slot sums once per tile.
+template <typename C>
+struct LevelSums {
+    C dd = C(0), off = C(0), f = C(0), kkt = C(0), dad = C(0);
+};
+
+// The last row of gamma_{i-1} rebuilt from the stored ones (zero at steps outside [0, T)).
+template <typename C, int K, int CH, bool INT>
+__device__ __forceinline__ void rebuild_last_row(int64_t t0, int64_t T, C (&G)[K][CH]) {
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        C r = C(1);
+#pragma unroll
+        for (int k = 0; k < K - 1; k++) r -= G[k][c];
+        const bool valid = INT || (t0 + c >= 0 && t0 + c < T);
+        G[K - 1][c] = valid ? (r > C(0) ? r : C(0)) : C(0);
+    }
+}
+
+// The data term q = bscale*(x - theta_k)^2 of a thread's chunk (zero where obs is false).
+template <typename C, int K, int CH>
+__device__ __forceinline__ void chunk_data_term(const C (&theta)[K], C bscale, const C (&X)[CH],
+                                                const bool (&obs)[CH], C (&Q)[K][CH]) {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const C th = theta[k];
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const C dx = X[c] - th;
+            Q[k][c] = obs[c] ? bscale * dx * dx : C(0);
+        }
+    }
+}
+
+// The three levels of a thread's chunk [t0, t0 + CH) in registers: G holds gamma_{i-1} (K rows),
+// Q the data term; G1 receives gamma_i and p the sums of the chunk when it is owned.  exch(v,
+// left, right) gets the neighbouring threads' edge values; next() runs once G and Q are in
+// registers.  Shared by the tiled pass and the persistent loop, so that both form every step
+// with the same arithmetic.
+template <typename S, typename C, int K, int CH, bool INT, typename Exch, typename Next>
+__device__ __forceinline__ void pass_levels(const TileCtx<S, C, K> &cx, int64_t t0, bool owner,
+                                            const C (&Q)[K][CH], const C (&G)[K][CH], Exch exch,
+                                            Next next, C (&G1)[K][CH], LevelSums<C> &p) {
+    const int64_t T = cx.T;
+    const C alpha2 = C(2) * cx.alpha;
+    const C s_kkt = cx.s_kkt;
+    const C a_apply = cx.a_apply;
+    const C b_apply = cx.b_apply;
+    const C a_dir = cx.a_dir;
+    const bool first = cx.first;
+    const bool need_f = cx.need_f;
+    // every step of the chunk is interior (both time neighbours exist): no boundary selects
+    const bool interior = INT || (t0 >= 1 && t0 + CH <= T - 1);
+    const bool want_kkt = cx.want_kkt;
+
+    // The levels have no branch inside their loops over the chunk (the options branch once per
+    // level, the sums of steps that are not owned are dropped by selects at the end): the chains
+    // of the CH steps are independent and hide each other's latency, which one or two waves per
+    // SIMD do not.
+    // level 1: gamma_i = gamma_{i-1} + beta_{i-1} (P(gamma_{i-1} - alpha_{i-1} g_{i-1}) - gamma_{i-1})
+    {
+        C gl[K], gr[K];
+        exch(G, gl, gr);
+        next();
+        if (first) {
+#pragma unroll
+            for (int c = 0; c < CH; c++) {
+                C y[K];
+#pragma unroll
+                for (int k = 0; k < K; k++) y[k] = G[k][c];
+                project_simplex<K, C>(y);
+#pragma unroll
+                for (int k = 0; k < K; k++) G1[k][c] = y[k];
+            }
+        } else {
+            C lap[K][CH];
+#pragma unroll
+            for (int k = 0; k < K; k++)
+                lap_half<C, CH>(G[k], gl[k], gr[k], t0, T, interior, lap[k]);
+#pragma unroll
+            for (int c = 0; c < CH; c++) {
+                C y[K];
+#pragma unroll
+                for (int k = 0; k < K; k++) {
+                    const C g = alpha2 * lap[k][c] + Q[k][c];
+                    y[k] = G[k][c] - a_apply * g;
+                }
+                project_simplex<K, C>(y);
+#pragma unroll
+                for (int k = 0; k < K; k++) G1[k][c] = G[k][c] + b_apply * (y[k] - G[k][c]);
+            }
+        }
+    }
+    // level 2: g_i, d_i = P(gamma_i - alpha_i g_i) - gamma_i, and on the owned steps |d|^2, the
+    // off-support term of <g,d>, f_i and the KKT residual of gamma_i
+    C Dd[K][CH];
+    {
+        C gl[K], gr[K], g[K][CH];
+        exch(G1, gl, gr);
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            lap_half<C, CH>(G1[k], gl[k], gr[k], t0, T, interior, g[k]);
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const int64_t t = t0 + c;
+            C y[K], z[K];
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                g[k][c] = alpha2 * g[k][c] + Q[k][c];
+                y[k] = G1[k][c] - a_dir * g[k][c];
+                z[k] = y[k];
+            }
+            const C tau = project_simplex<K, C>(z);
+            // <g, d> = -(|d|^2 + sum_{k off the support} (tau - y_k) gamma_k) / alpha holds for the
+            // projected-gradient step (it follows from g = (gamma - y)/alpha and sum_k d_k = 0);
+            // every term is non-negative, so the computed value cannot lose its sign to rounding
+            // the way the plain dot product does once d is tiny.
+            C o = C(0);
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                Dd[k][c] = z[k] - G1[k][c];
+                // (tau - y_k)^+ gamma_k: the off-support terms (y_k <= tau), as one max
+                o += cmax(tau - y[k], C(0)) * G1[k][c];
+            }
+            const bool in = INT || t < T;
+            p.off += in ? o : C(0);
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const C d = in ? Dd[k][c] : C(0);
+                p.dd += d * d;
+            }
+        }
+        if (need_f) {
+#pragma unroll
+            for (int c = 0; c < CH; c++) {
+                const bool in = INT || t0 + c < T;
+#pragma unroll
+                for (int k = 0; k < K; k++)
+                    p.f += (g[k][c] + Q[k][c]) * (in ? G1[k][c] : C(0));
+            }
+        }
+        if (want_kkt) {
+#pragma unroll
+            for (int c = 0; c < CH; c++) {
+                C z[K];
+#pragma unroll
+                for (int k = 0; k < K; k++) z[k] = G1[k][c] - s_kkt * g[k][c];
+                project_simplex<K, C>(z);
+#pragma unroll
+                for (int k = 0; k < K; k++) {
+                    const C e = fabs(G1[k][c] - z[k]);
+                    if (INT || t0 + c < T) p.kkt = (e > p.kkt || e != e) ? e : p.kkt;
+                }
+            }
+        }
+    }
+    // level 3: d'A d = alpha * sum over edges (t, t+1) of 2 (d_{t+1} - d_t)^2
+    {
+        C dl[K], dr[K];
+        exch(Dd, dl, dr);
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const bool in = INT || interior || t0 + c < T - 1;
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const C dn = c < CH - 1 ? Dd[k][c + 1] : dr[k];
+                const C e = in ? dn - Dd[k][c] : C(0);
+                p.dad += e * e;
+            }
+        }
+    }
+    if (!owner) p = LevelSums<C>{};
+}
+
 // STAGED: the tile's gamma and data rows were copied into the LDS stage (interior tiles
 // only).  next: a callable run once every thread has taken the stage's rows into registers
 // (it issues the copies of the slot's next tile into the stage).
@@ -272,15 +453,7 @@ __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chu
     const bool owner = tid >= HT && tid < NT - HT;  // owned steps are stored and reduced
     const S *src = cx.src;
     S *dst = cx.dst;
-    const C alpha = cx.alpha;
-    const C alpha2 = C(2) * alpha;
-    const C bscale = cx.bscale;
-    const C s_kkt = cx.s_kkt;
-    const C a_apply = cx.a_apply;
-    const C b_apply = cx.b_apply;
-    const C a_dir = cx.a_dir;
-    const bool first = cx.first;
-    const bool need_f = cx.need_f;
+    constexpr int KS = stored_rows<K>();
 
     // data term q = -b of every step of the chunk, formed once for the two levels that use it:
     // bscale*(x - theta_k)^2 (zero when held out or outside [0,T)), or read from an explicit b
@@ -295,7 +468,7 @@ __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chu
     } else {
         C X[CH];
         if (STAGED)
-            stage_read<S, C, K, CH, NT>(stage, stored_rows<K>(), X);
+            stage_read<S, C, K, CH, NT>(stage, KS, X);
         else
             load_chunk<S, C, CH, INT>(cx.xr, t0, T, ld, X);
         bool obs[CH];
@@ -309,181 +482,70 @@ __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chu
             for (int c = 0; c < CH; c++)
                 if (obs[c]) obs[c] = cx.heldout[t0 + c] == 0;
         }
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const C th = cx.theta[k];
-#pragma unroll
-            for (int c = 0; c < CH; c++) {
-                const C dx = X[c] - th;
-                Q[k][c] = obs[c] ? bscale * dx * dx : C(0);
-            }
-        }
+        chunk_data_term<C, K, CH>(cx.theta, cx.bscale, X, obs, Q);
     }
-    // every step of the chunk is interior (both time neighbours exist): no boundary selects
-    const bool interior = INT || (t0 >= 1 && t0 + CH <= T - 1);
-    const bool want_kkt = cx.want_kkt;
-
-    // level 1: gamma_i = gamma_{i-1} + beta_{i-1} (P(gamma_{i-1} - alpha_{i-1} g_{i-1}) - gamma_{i-1})
-    constexpr int KS = stored_rows<K>();
-    C G1[K][CH];
-    {
-        C G[K][CH];
+    C G[K][CH], G1[K][CH];
+#pragma unroll
+    for (int k = 0; k < KS; k++) {
+        if (STAGED)
+            stage_read<S, C, K, CH, NT>(stage, k, G[k]);
+        else
+            load_chunk<S, C, CH, INT>(src + k * ld, t0, T, ld, G[k]);
+    }
+    if (KS < K) {
+        // gamma_0 may lie off the simplex: its last row is read (first passes are never staged)
+        if (cx.first)
+            load_chunk<S, C, CH, INT>(src + (K - 1) * ld, t0, T, ld, G[K - 1]);
+        else
+            rebuild_last_row<C, K, CH, INT>(t0, T, G);
+    }
+    LevelSums<C> p;
+    pass_levels<S, C, K, CH, INT>(
+        cx, t0, owner, Q, G,
+        [&](const C(&v)[K][CH], C(&l)[K], C(&r)[K]) {
+            exchange_edges<C, K, CH, NT>(v, lds_x, l, r);
+        },
+        [&]() {
+            // every stage read must be done before the next copies overwrite the stage: the
+            // exchange's barriers see to that, and a one-wave workgroup waits for its own reads
+            if constexpr (NT == WAVE && STAGED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            next();
+        },
+        G1, p);
+    if (owner) {
+        // store gamma_i
+        using VT = V16<S>;
+        constexpr int VW = VT::n;
 #pragma unroll
         for (int k = 0; k < KS; k++) {
-            if (STAGED)
-                stage_read<S, C, K, CH, NT>(stage, k, G[k]);
-            else
-                load_chunk<S, C, CH, INT>(src + k * ld, t0, T, ld, G[k]);
-        }
-        if (KS < K) {
-            if (first) {
-                // gamma_0 may lie off the simplex: its last row is read (first passes are
-                // never staged)
-                load_chunk<S, C, CH, INT>(src + (K - 1) * ld, t0, T, ld, G[K - 1]);
-            } else {
 #pragma unroll
-                for (int c = 0; c < CH; c++) {
-                    C r = C(1);
+            for (int q = 0; q < CH / VW; q++) {
+                const int64_t t = t0 + q * VW;
+                if (INT || t + VW <= T) {
+                    typename VT::type vec;
 #pragma unroll
-                    for (int k = 0; k < K - 1; k++) r -= G[k][c];
-                    const bool valid = INT || (t0 + c >= 0 && t0 + c < T);
-                    G[K - 1][c] = valid ? (r > C(0) ? r : C(0)) : C(0);
-                }
-            }
-        }
-        C gl[K], gr[K];
-        exchange_edges<C, K, CH, NT>(G, lds_x, gl, gr);
-        // every stage read must be done before the next copies overwrite the stage: the
-        // exchange's barriers see to that, and a one-wave workgroup waits for its own reads
-        if constexpr (NT == WAVE && STAGED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        next();
+                    for (int i = 0; i < VW; i++) VT::set(vec, i, S(G1[k][q * VW + i]));
+                    // FP64 rows: nontemporal stores (95.8 -> 87.1 us per pass at
+                    // T = 1e7, K = 3); the FP32 pass was slower with them (49.5 -> 53.8 us)
+                    if constexpr (sizeof(S) == 8)
+                        store_nt(reinterpret_cast<typename VT::type *>(dst + k * ld + t), vec);
+                    else
+                        *reinterpret_cast<typename VT::type *>(dst + k * ld + t) = vec;
+                } else {
 #pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const int64_t t = t0 + c;
-            C y[K];
-            if (first) {
-#pragma unroll
-                for (int k = 0; k < K; k++) y[k] = G[k][c];
-                project_simplex<K, C>(y);
-#pragma unroll
-                for (int k = 0; k < K; k++) G1[k][c] = y[k];
-            } else {
-#pragma unroll
-                for (int k = 0; k < K; k++) {
-                    const C vm = c > 0 ? G[k][c - 1] : gl[k];
-                    const C vp = c < CH - 1 ? G[k][c + 1] : gr[k];
-                    const C g = alpha2 * lap_half(G[k][c], vm, vp, t, T, interior) + Q[k][c];
-                    y[k] = G[k][c] - a_apply * g;
-                }
-                project_simplex<K, C>(y);
-#pragma unroll
-                for (int k = 0; k < K; k++) G1[k][c] = G[k][c] + b_apply * (y[k] - G[k][c]);
-            }
-        }
-    }
-    // level 2: g_i, d_i = P(gamma_i - alpha_i g_i) - gamma_i, and on the owned steps |d|^2, the
-    // off-support term of <g,d>, f_i and the KKT residual of gamma_i
-    C Dd[K][CH];
-    C p_dd = C(0), p_off = C(0), p_f = C(0), p_kkt = C(0);
-    {
-        C gl[K], gr[K];
-        exchange_edges<C, K, CH, NT>(G1, lds_x, gl, gr);
-#pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const int64_t t = t0 + c;
-            C g[K], y[K], z[K];
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                const C vm = c > 0 ? G1[k][c - 1] : gl[k];
-                const C vp = c < CH - 1 ? G1[k][c + 1] : gr[k];
-                g[k] = alpha2 * lap_half(G1[k][c], vm, vp, t, T, interior) + Q[k][c];
-                y[k] = G1[k][c] - a_dir * g[k];
-                z[k] = y[k];
-            }
-            const C tau = project_simplex<K, C>(z);
-            // <g, d> = -(|d|^2 + sum_{k off the support} (tau - y_k) gamma_k) / alpha holds for the
-            // projected-gradient step (it follows from g = (gamma - y)/alpha and sum_k d_k = 0);
-            // every term is non-negative, so the computed value cannot lose its sign to rounding
-            // the way the plain dot product does once d is tiny.
-            C o = C(0);
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                Dd[k][c] = z[k] - G1[k][c];
-                // (tau - y_k)^+ gamma_k: the off-support terms (y_k <= tau), as one max
-                o += cmax(tau - y[k], C(0)) * G1[k][c];
-            }
-            if (owner && (INT || t < T)) {
-                p_off += o;
-#pragma unroll
-                for (int k = 0; k < K; k++) p_dd += Dd[k][c] * Dd[k][c];
-                if (need_f) {
-#pragma unroll
-                    for (int k = 0; k < K; k++) p_f += (g[k] + Q[k][c]) * G1[k][c];
-                }
-                if (want_kkt) {
-#pragma unroll
-                    for (int k = 0; k < K; k++) z[k] = G1[k][c] - s_kkt * g[k];
-                    project_simplex<K, C>(z);
-#pragma unroll
-                    for (int k = 0; k < K; k++) {
-                        const C e = fabs(G1[k][c] - z[k]);
-                        p_kkt = (e > p_kkt || e != e) ? e : p_kkt;
-                    }
+                    for (int i = 0; i < VW; i++)
+                        if (t + i < T) dst[k * ld + t + i] = S(G1[k][q * VW + i]);
                 }
             }
         }
     }
-    // level 3: d'A d = alpha * sum over edges (t, t+1) of 2 (d_{t+1} - d_t)^2, store gamma_i
-    C p_dad = C(0);
-    {
-        C dl[K], dr[K];
-        exchange_edges<C, K, CH, NT>(Dd, lds_x, dl, dr);
-        if (owner) {
-#pragma unroll
-            for (int c = 0; c < CH; c++) {
-                const int64_t t = t0 + c;
-                if (INT || interior || t < T - 1) {
-#pragma unroll
-                    for (int k = 0; k < K; k++) {
-                        const C dn = c < CH - 1 ? Dd[k][c + 1] : dr[k];
-                        const C e = dn - Dd[k][c];
-                        p_dad += e * e;
-                    }
-                }
-            }
-            using VT = V16<S>;
-            constexpr int VW = VT::n;
-#pragma unroll
-            for (int k = 0; k < KS; k++) {
-#pragma unroll
-                for (int q = 0; q < CH / VW; q++) {
-                    const int64_t t = t0 + q * VW;
-                    if (INT || t + VW <= T) {
-                        typename VT::type vec;
-#pragma unroll
-                        for (int i = 0; i < VW; i++) VT::set(vec, i, S(G1[k][q * VW + i]));
-                        // FP64 rows: nontemporal stores (95.8 -> 87.1 us per pass at
-                        // T = 1e7, K = 3); the FP32 pass was slower with them (49.5 -> 53.8 us)
-                        if constexpr (sizeof(S) == 8)
-                            store_nt(reinterpret_cast<typename VT::type *>(dst + k * ld + t), vec);
-                        else
-                            *reinterpret_cast<typename VT::type *>(dst + k * ld + t) = vec;
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < VW; i++)
-                            if (t + i < T) dst[k * ld + t + i] = S(G1[k][q * VW + i]);
-                    }
-                }
-            }
-        }
-    }
-    const double dd = (double)p_dd;
+    const double dd = (double)p.dd;
     acc[0] += dd;
-    acc[1] += 2.0 * (double)alpha * (double)p_dad;
-    acc[2] -= (dd + (double)p_off) / (double)a_dir;
-    acc[3] += 0.5 * (double)p_f;
-    if (want_kkt) {
-        const double e = (double)p_kkt;
+    acc[1] += 2.0 * (double)cx.alpha * (double)p.dad;
+    acc[2] -= (dd + (double)p.off) / (double)cx.a_dir;
+    acc[3] += 0.5 * (double)p.f;
+    if (cx.want_kkt) {
+        const double e = (double)p.kkt;
         acc[4] = (e > acc[4] || e != e) ? e : acc[4];
     } else {
         acc[4] = -1.0;  // not evaluated on this pass

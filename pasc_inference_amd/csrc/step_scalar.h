@@ -13,8 +13,10 @@ namespace pasc {
 // reduced the instance's partial slots.
 // ---------------------------------------------------------------------------------------------
 // sample_eps: the per-sample epsilon alpha * s_kkt of the instance (FP32 hand-over floor).
-__device__ inline void step_scalar(double sample_eps, InstState &s, const double (&v)[NPART],
-                                   const StepParams &P, int32_t *dirty) {
+// St: the scalar fields of InstState; Win: its window of the last m values of f (fill, push, max).
+template <typename St, typename Win>
+__device__ __forceinline__ void step_core(double sample_eps, St &s, Win win,
+                                          const double (&v)[NPART], const StepParams &P) {
     const double dd = v[0], dAd = v[1], gd = v[2];
     // a negative residual marks a pass that did not evaluate it: keep the last value
     const bool have_kkt = v[4] >= 0.0 || v[4] != v[4];
@@ -35,13 +37,13 @@ __device__ inline void step_scalar(double sample_eps, InstState &s, const double
         stop = true;
         reason = PASC_REASON_NUMERIC;
     } else if (s.first) {
-        for (int i = 0; i < P.m; i++) s.fs[i] = f;
+        win.fill(f, P.m);
         s.fs_last = 0;
         s.it = 0;
         if ((P.stop_mask & PASC_STOP_KKT) && kkt_fresh && kkt <= P.kkt_tol) { stop = true; reason = PASC_REASON_KKT; }
     } else {
         s.fs_last = (s.fs_last + 1 >= P.m) ? 0 : s.fs_last + 1;
-        s.fs[s.fs_last] = f;
+        win.push(f, s.fs_last);
         s.it += 1;
         if ((P.stop_mask & PASC_STOP_DIFFF) && fabs(f - s.f) < P.eps) { stop = true; reason = PASC_REASON_DIFFF; }
         else if ((P.stop_mask & PASC_STOP_NORMGP) && s.dd < P.eps) { stop = true; reason = PASC_REASON_NORMGP; }
@@ -76,11 +78,9 @@ __device__ inline void step_scalar(double sample_eps, InstState &s, const double
         s.active = 0;
         s.reason = reason;
         s.first = 0;
-        *dirty = 1;  // the active-tile enumeration must be rebuilt
         return;
     }
-    double fmax = s.fs[0];
-    for (int i = 0; i < P.m; i++) fmax = s.fs[i] > fmax ? s.fs[i] : fmax;
+    const double fmax = win.max(P.m);
     double beta, alpha_next;
     if (dAd > 0.0) {
         const double xi = (fmax - f) / dAd;
@@ -101,6 +101,26 @@ __device__ inline void step_scalar(double sample_eps, InstState &s, const double
     s.alpha_apply = s.alpha_dir;
     s.alpha_dir = alpha_next;
     s.first = 0;
+}
+
+// The window kept in InstState::fs.
+struct StateWindow {
+    double *fs;
+    __device__ void fill(double f, int m) {
+        for (int i = 0; i < m; i++) fs[i] = f;
+    }
+    __device__ void push(double f, int at) { fs[at] = f; }
+    __device__ double max(int m) const {
+        double r = fs[0];
+        for (int i = 0; i < m; i++) r = fs[i] > r ? fs[i] : r;
+        return r;
+    }
+};
+
+__device__ inline void step_scalar(double sample_eps, InstState &s, const double (&v)[NPART],
+                                   const StepParams &P, int32_t *dirty) {
+    step_core(sample_eps, s, StateWindow{s.fs}, v, P);
+    if (!s.active) *dirty = 1;  // the active-tile enumeration must be rebuilt
 }
 
 // One instance's step by a workgroup of NT threads.  The state is staged in LDS word by word by
