@@ -39,6 +39,7 @@ def _units():
     units.append((os.path.join(CSRC, "engine.hip"), "engine.o", []))
     units.append((os.path.join(CSRC, "adjoint.hip"), "adjoint.o", []))
     units.append((os.path.join(CSRC, "fem.hip"), "fem.o", []))
+    units.append((os.path.join(CSRC, "transfer.hip"), "transfer.o", []))
     units.append((os.path.join(CSRC, "noalloc.hip"), "noalloc.o", []))
     units.append((os.path.join(CSRC, "capi.hip"), "capi.o", []))
     units.append((os.path.join(CSRC, "generate.cpp"), "generate.o", []))
@@ -61,7 +62,7 @@ def build(jobs: int | None = None, verbose: bool = False) -> str:
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         objs = list(ex.map(lambda u: _compile(*u), units))
     tmp = LIB + ".tmp"
-    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + objs
+    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-pthread", "-o", tmp] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr[-6000:]}")

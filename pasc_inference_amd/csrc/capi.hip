@@ -56,8 +56,6 @@ struct pasc_problem {
     bool b_set = false;  // explicit linear term instead of the data term
     bool has_data = true;  // false: created without x (only an explicit b can define the QP)
     uint8_t *d_heldout = nullptr;
-    std::vector<uint8_t> h_heldout;
-    std::vector<double> h_x;  // host copy of the data, [T][R][xdim] (for abserr etc.)
     Engine e;
     // FEM coarsening (1-D): the engine holds the coarse QP of T2 steps, the fine grid of T
     // steps lives here (data, gamma) and meets the engine through reduce / prolongate
@@ -114,7 +112,8 @@ int pasc_ctx_create(int device, pasc_ctx **out) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->c.arch = prop.gcnArchName;
     // the device address of the static scratch of pasc_theta_update_noalloc on this device
-    const int rc = noalloc_init(device);
+    int rc = noalloc_init(device);
+    if (rc == PASC_OK) rc = staging_open(device);
     if (rc) {
         (void)hipStreamDestroy(s);
         delete c;
@@ -128,13 +127,18 @@ int pasc_ctx_destroy(pasc_ctx *ctx) {
     if (!ctx) return PASC_OK;
     (void)hipSetDevice(ctx->c.device);
     if (ctx->c.own_stream && ctx->c.stream) (void)hipStreamDestroy((hipStream_t)ctx->c.stream);
+    staging_close(ctx->c.device);
     delete ctx;
     return PASC_OK;
 }
 
 int pasc_ctx_set_stream(pasc_ctx *ctx, void *stream) {
     if (!ctx) return fail(PASC_ERR_ARG, "ctx is NULL");
-    if (ctx->c.own_stream && ctx->c.stream) (void)hipStreamDestroy((hipStream_t)ctx->c.stream);
+    if (ctx->c.own_stream && ctx->c.stream) {
+        // work queued on the context's own stream is done before another stream takes over
+        HIP_TRY(hipStreamSynchronize((hipStream_t)ctx->c.stream));
+        (void)hipStreamDestroy((hipStream_t)ctx->c.stream);
+    }
     if (stream) {
         ctx->c.stream = stream;
         ctx->c.own_stream = false;
@@ -294,9 +298,7 @@ int pasc_problem_create(pasc_ctx *ctx, const pasc_problem_desc *desc, pasc_probl
     }
     const int64_t n = p->T * p->R;  // nodes
     p->has_data = desc->x != nullptr;
-    if (p->has_data) p->h_x.assign(desc->x, desc->x + n * p->xdim);
     if (desc->heldout) {
-        p->h_heldout.assign(desc->heldout, desc->heldout + n);
         hipError_t e = hipMalloc(&p->d_heldout, (size_t)n);
         if (e == hipSuccess) e = hipMemcpy(p->d_heldout, desc->heldout, (size_t)n, hipMemcpyHostToDevice);
         if (e != hipSuccess) {
@@ -313,28 +315,21 @@ int pasc_problem_create(pasc_ctx *ctx, const pasc_problem_desc *desc, pasc_probl
                       p->grid_width, descs, d.ld * p->xdim);
     if (rc == PASC_OK && p->graph)
         rc = engine_set_graph(p->e, p->T, p->R, p->grid_width, desc->nbr_ptr, desc->nbr_idx);
-    if (rc == PASC_OK && !fem) {
-        // data rows: SoA, row c holds channel c
-        std::vector<double> rows((size_t)d.ld * p->xdim, 0.0);
-        for (int c = 0; c < p->xdim; c++)
-            for (int64_t i = 0; p->has_data && i < n; i++)
-                rows[(size_t)c * d.ld + i] = desc->x[i * p->xdim + c];
-        rc = engine_upload_data(p->e, rows.data(), 0, (int64_t)rows.size());
-    }
+    // data rows: SoA, row c holds channel c (zero without data, as allocated)
+    if (rc == PASC_OK && !fem && p->has_data)
+        rc = engine_upload_data(p->e, desc->x, 0, n, d.ld, p->xdim);
     if (rc == PASC_OK && fem) {
         // the fine grid: data rows, gamma rows and a coarse scratch; the engine itself runs
         // on the explicit linear term reduced from the fine residual before every solve
         const int64_t ld1 = p->fg.ld1;
-        std::vector<double> rows((size_t)ld1 * p->xdim, 0.0);
-        for (int c = 0; c < p->xdim; c++)
-            for (int64_t i = 0; i < n; i++) rows[(size_t)c * ld1 + i] = desc->x[i * p->xdim + c];
-        hipError_t he = hipMalloc(&p->d_x1, sizeof(double) * rows.size());
-        if (he == hipSuccess)
-            he = hipMemcpy(p->d_x1, rows.data(), sizeof(double) * rows.size(), hipMemcpyHostToDevice);
+        hipError_t he = hipMalloc(&p->d_x1, sizeof(double) * (size_t)ld1 * p->xdim);
         if (he == hipSuccess) he = hipMalloc(&p->d_g1, sizeof(double) * (size_t)p->K * ld1);
-        if (he == hipSuccess) he = hipMemset(p->d_g1, 0, sizeof(double) * (size_t)p->K * ld1);
+        if (he == hipSuccess)
+            he = hipMemsetAsync(p->d_g1, 0, sizeof(double) * (size_t)p->K * ld1,
+                                (hipStream_t)ctx->c.stream);
         if (he == hipSuccess) he = hipMalloc(&p->d_tmp, sizeof(double) * (size_t)p->K * p->fg.ld2);
         if (he != hipSuccess) rc = fail(PASC_ERR_HIP, "FEM buffers: %s", hipGetErrorString(he));
+        if (rc == PASC_OK) rc = rows_from_host(&ctx->c, desc->x, true, p->d_x1, false, n, ld1, p->xdim);
         std::memset(&p->fine, 0, sizeof(p->fine));
         p->fine.T = p->T;
         p->fine.ld = ld1;
@@ -395,14 +390,10 @@ int pasc_set_gamma(pasc_problem *p, const double *gamma, int layout) {
     if (rc) return rc;
     if (p->fem_type != PASC_FEM_NONE) {
         // the fine gamma (TSData::gammavector); it is reduced to the coarse grid per solve
-        const int64_t T = p->T, ld1 = p->fg.ld1;
-        std::vector<double> rows((size_t)p->K * ld1, 0.0);
-        for (int k = 0; k < p->K; k++)
-            for (int64_t t = 0; t < T; t++)
-                rows[k * ld1 + t] = layout == PASC_LAYOUT_TMAJOR ? gamma[t * p->K + k] : gamma[k * T + t];
-        HIP_TRY(hipMemcpy(p->d_g1, rows.data(), sizeof(double) * rows.size(), hipMemcpyHostToDevice));
-        p->gamma_set = true;
-        return PASC_OK;
+        rc = rows_from_host(&p->ctx->c, gamma, layout == PASC_LAYOUT_TMAJOR, p->d_g1, false, p->T,
+                            p->fg.ld1, p->K);
+        if (rc == PASC_OK) p->gamma_set = true;
+        return rc;
     }
     rc = engine_set_gamma(p->e, 0, gamma, layout);
     if (rc == PASC_OK) p->gamma_set = true;
@@ -414,11 +405,10 @@ int pasc_set_gamma_uniform(pasc_problem *p) {
     if (!p) return fail(PASC_ERR_ARG, "set_gamma_uniform: NULL argument");
     int rc = use_device(p->ctx);
     if (rc) return rc;
-    if (p->fem_type != PASC_FEM_NONE) {
-        std::vector<double> g((size_t)p->T * p->K, 1.0 / p->K);
-        return pasc_set_gamma(p, g.data(), PASC_LAYOUT_TMAJOR);
-    }
-    rc = engine_set_uniform(p->e, 0);
+    if (p->fem_type != PASC_FEM_NONE)
+        rc = rows_fill_uniform(&p->ctx->c, p->d_g1, false, p->T, p->fg.ld1, p->K);
+    else
+        rc = engine_set_uniform(p->e, 0);
     if (rc == PASC_OK) p->gamma_set = true;
     return rc;
 }
@@ -430,19 +420,9 @@ int pasc_get_gamma(pasc_problem *p, double *gamma, int layout) {
     if (!p->gamma_set) return fail(PASC_ERR_STATE, "get_gamma: gamma was never set");
     int rc = use_device(p->ctx);
     if (rc) return rc;
-    if (p->fem_type != PASC_FEM_NONE) {
-        const int64_t T = p->T, ld1 = p->fg.ld1;
-        std::vector<double> rows((size_t)p->K * ld1);
-        HIP_TRY(hipMemcpyAsync(rows.data(), p->d_g1, sizeof(double) * rows.size(),
-                               hipMemcpyDeviceToHost, (hipStream_t)p->ctx->c.stream));
-        HIP_TRY(hipStreamSynchronize((hipStream_t)p->ctx->c.stream));
-        for (int k = 0; k < p->K; k++)
-            for (int64_t t = 0; t < T; t++) {
-                if (layout == PASC_LAYOUT_TMAJOR) gamma[t * p->K + k] = rows[k * ld1 + t];
-                else gamma[k * T + t] = rows[k * ld1 + t];
-            }
-        return PASC_OK;
-    }
+    if (p->fem_type != PASC_FEM_NONE)
+        return rows_to_host(&p->ctx->c, p->d_g1, false, p->T, p->fg.ld1, p->K, gamma,
+                            layout == PASC_LAYOUT_TMAJOR);
     return engine_get_gamma(p->e, 0, gamma, layout);
 }
 
@@ -555,19 +535,11 @@ int pasc_set_data(pasc_problem *p, const double *x) {
     int rc = use_device(p->ctx);
     if (rc) return rc;
     // the data rows as at creation: SoA, row c holds channel c (the fine grid when FEM-reduced)
-    const int64_t ld = p->fem_type != PASC_FEM_NONE ? p->fg.ld1 : p->e.h_desc[0].ld;
-    std::vector<double> rows((size_t)ld * p->xdim, 0.0);
-    for (int c = 0; c < p->xdim; c++)
-        for (int64_t i = 0; i < n; i++) rows[(size_t)c * ld + i] = x[i * p->xdim + c];
-    if (p->fem_type != PASC_FEM_NONE) {
-        const hipError_t he = hipMemcpy(p->d_x1, rows.data(), sizeof(double) * rows.size(),
-                                        hipMemcpyHostToDevice);
-        if (he != hipSuccess) return fail(PASC_ERR_HIP, "set_data: %s", hipGetErrorString(he));
-    } else {
-        rc = engine_upload_data(p->e, rows.data(), 0, (int64_t)rows.size());
-        if (rc) return rc;
-    }
-    p->h_x.assign(x, x + n * p->xdim);
+    if (p->fem_type != PASC_FEM_NONE)
+        rc = rows_from_host(&p->ctx->c, x, true, p->d_x1, false, n, p->fg.ld1, p->xdim);
+    else
+        rc = engine_upload_data(p->e, x, 0, n, p->e.h_desc[0].ld, p->xdim);
+    if (rc) return rc;
     p->solved = false;
     return PASC_OK;
 }
@@ -864,7 +836,7 @@ int pasc_batch_create(pasc_ctx *ctx, int32_t n_series, const pasc_series_desc *s
     b->n_eps = n_eps;
     rc = engine_alloc(b->e, &ctx->c, precision, STENCIL_TIME, 0, descs, xo);
     for (int s = 0; s < n_series && rc == PASC_OK; s++)
-        rc = engine_upload_data(b->e, series[s].x, xoff[s], series[s].T);
+        rc = engine_upload_data(b->e, series[s].x, xoff[s], series[s].T, series[s].T, 1);
     if (rc) {
         engine_free(b->e);
         delete b;
@@ -929,12 +901,7 @@ int pasc_batch_create_problem(pasc_ctx *ctx, const pasc_problem_desc *desc,
                       desc->grid_width, descs, ld * desc->xdim);
     if (rc == PASC_OK && graph)
         rc = engine_set_graph(b->e, desc->T, desc->R, desc->grid_width, desc->nbr_ptr, desc->nbr_idx);
-    if (rc == PASC_OK) {
-        std::vector<double> rows((size_t)ld * desc->xdim, 0.0);
-        for (int c = 0; c < desc->xdim; c++)
-            for (int64_t i = 0; i < n; i++) rows[(size_t)c * ld + i] = desc->x[i * desc->xdim + c];
-        rc = engine_upload_data(b->e, rows.data(), 0, (int64_t)rows.size());
-    }
+    if (rc == PASC_OK) rc = engine_upload_data(b->e, desc->x, 0, n, ld, desc->xdim);
     if (rc) {
         engine_free(b->e);
         if (b->d_heldout) (void)hipFree(b->d_heldout);

@@ -181,10 +181,29 @@ static int engine_retile(Engine &e, bool f64_phase) {
     HIP_TRY(hipMemcpyAsync(e.d_desc, e.h_desc.data(), sizeof(InstDesc) * e.n_inst,
                            hipMemcpyHostToDevice, S_(e)));
     HIP_TRY(hipStreamSynchronize(S_(e)));
+    e.desc_stale = false;
+    return PASC_OK;
+}
+
+// The stale descriptor and initial state of a single problem to the device, and `words` words of
+// the exchange area marked empty.
+static int prepare(Engine &e, uint64_t *ex, int64_t words) {
+    if (e.n_inst != 1 || (!e.desc_stale && !e.init_state && words == 0)) return PASC_OK;
+    static const InstState none{};
+    const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>((words + 255) / 256, 1024));
+    hipLaunchKernelGGL(prepare_single, dim3(blocks), dim3(256), 0, S_(e), e.d_desc, e.h_desc[0],
+                       e.d_state, e.init_state ? *e.init_state : none, e.init_state ? 1 : 0, ex, words);
+    HIP_TRY(hipGetLastError());
+    e.desc_stale = false;
+    e.init_state = nullptr;
     return PASC_OK;
 }
 
 int engine_update_desc(Engine &e) {
+    if (e.n_inst == 1) {
+        e.desc_stale = true;
+        return PASC_OK;
+    }
     HIP_TRY(hipMemcpyAsync(e.d_desc, e.h_desc.data(), sizeof(InstDesc) * e.n_inst,
                            hipMemcpyHostToDevice, S_(e)));
     HIP_TRY(hipStreamSynchronize(S_(e)));
@@ -237,8 +256,9 @@ int engine_alloc(Engine &e, Ctx *ctx, int precision, int stencil, int32_t grid_w
                        (uint64_t *)(e.d_done + DONE_WORDS), (int64_t)DONE_SUB * NPART, PART_EMPTY);
     HIP_TRY(hipGetLastError());
     // pinned poll area: [0] active instances, [1 + g] active tiles of K group g
-    HIP_TRY(hipHostMalloc((void **)&e.h_nactive, sizeof(int32_t) * (1 + PASC_MAX_K),
-                          hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **)&e.h_nactive, 64 + sizeof(InstState), hipHostMallocDefault));
+    static_assert(sizeof(int32_t) * (1 + PASC_MAX_K) <= 64, "the poll area fits its line");
+    e.h_state = reinterpret_cast<InstState *>((char *)e.h_nactive + 64);
     e.h_parity.assign(e.n_inst, 0);
     // K groups
     for (int K = 1; K <= PASC_MAX_K; K++) {
@@ -285,6 +305,10 @@ void engine_free(Engine &e) {
     e.d_done = nullptr;
     if (e.h_nactive) (void)hipHostFree(e.h_nactive);
     if (e.d_scratch) (void)hipFree(e.d_scratch);
+    for (auto &v : e.ev_solve) {
+        if (v) (void)hipEventDestroy((hipEvent_t)v);
+        v = nullptr;
+    }
     for (auto &g : e.groups) {
         if (g.d_ids) (void)hipFree(g.d_ids);
         if (g.d_off) (void)hipFree(g.d_off);
@@ -338,16 +362,17 @@ int engine_set_graph(Engine &e, int64_t T, int64_t R, int32_t width, const int64
     return PASC_OK;
 }
 
-int engine_upload_data(Engine &e, const double *x_host, int64_t offset, int64_t n) {
-    HIP_TRY(hipMemcpyAsync((double *)e.d_x64 + offset, x_host, 8 * (size_t)n,
-                           hipMemcpyHostToDevice, S_(e)));
+int engine_upload_data(Engine &e, const double *x_host, int64_t offset, int64_t n, int64_t ld,
+                       int xdim) {
+    int rc = rows_from_host(e.ctx, x_host, true, (double *)e.d_x64 + offset, false, n, ld, xdim);
+    if (rc) return rc;
     if (e.d_x32) {
-        const int64_t blocks = (n + 255) / 256;
+        const int64_t m = ld * (xdim - 1) + n, blocks = (m + 255) / 256;
         hipLaunchKernelGGL((convert_kernel<double, float>), dim3((unsigned)blocks), dim3(256), 0,
-                           S_(e), (const double *)e.d_x64 + offset, (float *)e.d_x32 + offset, n);
+                           S_(e), (const double *)e.d_x64 + offset, (float *)e.d_x32 + offset, m);
         HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(S_(e)));
     }
-    HIP_TRY(hipStreamSynchronize(S_(e)));
     return PASC_OK;
 }
 
@@ -393,21 +418,23 @@ static int upload_rows(Engine &e, int inst, const std::vector<double> &rows) {
     return PASC_OK;
 }
 
+// buffer 0 of an instance, which the next solve starts from
+static void *start_rows(Engine &e, int inst) {
+    e.cur64 = false;
+    e.h_parity[inst] = 0;
+    const size_t es = e.precision == PASC_FP32_BULK ? 4 : 8;
+    return (char *)e.d_gamma[0] + es * (size_t)e.h_desc[inst].goff;
+}
+
 int engine_set_uniform(Engine &e, int inst) {
     const InstDesc &d = e.h_desc[inst];
-    std::vector<double> rows((size_t)d.K * d.ld, 0.0);
-    for (int k = 0; k < d.K; k++)
-        for (int64_t t = 0; t < d.T; t++) rows[k * d.ld + t] = 1.0 / d.K;
-    return upload_rows(e, inst, rows);
+    return rows_fill_uniform(e.ctx, start_rows(e, inst), e.precision == PASC_FP32_BULK, d.T, d.ld, d.K);
 }
 
 int engine_set_gamma(Engine &e, int inst, const double *g, int layout) {
     const InstDesc &d = e.h_desc[inst];
-    std::vector<double> rows((size_t)d.K * d.ld, 0.0);
-    for (int k = 0; k < d.K; k++)
-        for (int64_t t = 0; t < d.T; t++)
-            rows[k * d.ld + t] = layout == PASC_LAYOUT_TMAJOR ? g[t * d.K + k] : g[k * d.T + t];
-    return upload_rows(e, inst, rows);
+    return rows_from_host(e.ctx, g, layout == PASC_LAYOUT_TMAJOR, start_rows(e, inst),
+                          e.precision == PASC_FP32_BULK, d.T, d.ld, d.K);
 }
 
 // Explicit linear term of one instance (the QP's b as the reference's QPData holds it): stored
@@ -423,12 +450,9 @@ int engine_set_linear_term(Engine &e, int inst, const double *b_host, int layout
     int arc = alloc_linear_term(e);
     if (arc) return arc;
     const int64_t n = (int64_t)d.K * d.ld;
-    std::vector<double> rows((size_t)n, 0.0);
-    for (int k = 0; k < d.K; k++)
-        for (int64_t t = 0; t < d.T; t++)
-            rows[k * d.ld + t] = layout == PASC_LAYOUT_TMAJOR ? b_host[t * d.K + k] : b_host[k * d.T + t];
     double *b64 = (double *)e.d_b64 + d.goff;
-    HIP_TRY(hipMemcpyAsync(b64, rows.data(), 8 * (size_t)n, hipMemcpyHostToDevice, S_(e)));
+    arc = rows_from_host(e.ctx, b_host, layout == PASC_LAYOUT_TMAJOR, b64, false, d.T, d.ld, d.K);
+    if (arc) return arc;
     float *b32 = nullptr;
     if (e.d_b32) {
         b32 = (float *)e.d_b32 + d.goff;
@@ -438,20 +462,14 @@ int engine_set_linear_term(Engine &e, int inst, const double *b_host, int layout
     }
     d.b64 = b64;
     d.b32 = b32;
-    return engine_update_desc(e);  // synchronises: rows may go out of scope
+    return engine_update_desc(e);
 }
 
 int engine_get_gamma(Engine &e, int inst, double *g, int layout) {
     const InstDesc &d = e.h_desc[inst];
-    std::vector<double> rows;
-    int rc = download_rows(e, inst, rows);
-    if (rc) return rc;
-    for (int k = 0; k < d.K; k++)
-        for (int64_t t = 0; t < d.T; t++) {
-            if (layout == PASC_LAYOUT_TMAJOR) g[t * d.K + k] = rows[k * d.ld + t];
-            else g[k * d.T + t] = rows[k * d.ld + t];
-        }
-    return PASC_OK;
+    bool f32;
+    const void *rows = engine_current_gamma(e, inst, &f32);
+    return rows_to_host(e.ctx, rows, f32, d.T, d.ld, d.K, g, layout == PASC_LAYOUT_TMAJOR);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -652,6 +670,15 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
     const LoopPlan pl = loop_plan(e, ph.f64);
     if (pl.nwg == 0) return PASC_OK;
     hipStream_t s = S_(e);
+    if (e.init_state && !e.init_state->active) {
+        // nothing to run (the polish of an FP32 phase that failed)
+        *e.h_state = *e.init_state;
+        e.init_state = nullptr;
+        HIP_TRY(hipEventRecord((hipEvent_t)e.ev_solve[1], s));
+        HIP_TRY(hipStreamSynchronize(s));
+        *ran = true;
+        return PASC_OK;
+    }
     const int64_t cap = std::max<int64_t>(1, LOOP_EXCHANGE_BYTES / (8 * pl.epoch_words));
     const int epochs = (int)std::min<int64_t>(std::min(max_passes, LOOP_EPOCHS_MAX), cap);
     void *ex;
@@ -662,9 +689,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
     while (passes < max_passes) {
         const int n = std::min(epochs, max_passes - passes);
         const int64_t words = pl.epoch_words * (n + 1);
-        hipLaunchKernelGGL(fill_u64, dim3((unsigned)std::min<int64_t>((words + 255) / 256, 1024)),
-                           dim3(256), 0, s, (uint64_t *)ex, words, PART_EMPTY);
-        HIP_TRY(hipGetLastError());
+        if ((rc = prepare(e, (uint64_t *)ex, words))) return rc;
         LoopArgs a{};
         a.p.gamma0 = g64 ? e.d_gamma64[0] : e.d_gamma[0];
         a.p.gamma1 = g64 ? e.d_gamma64[1] : e.d_gamma[1];
@@ -677,6 +702,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
         a.p.sp = ph.sp;
         a.ex = (double *)ex;
         a.flags = flags;
+        a.out = e.h_state;
         a.ntiles = pl.ntiles;
         a.tpw = pl.tpw;
         a.epochs = n;
@@ -694,6 +720,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
             (void)hipGetLastError();
             return PASC_OK;
         }
+        HIP_TRY(hipEventRecord((hipEvent_t)e.ev_solve[1], s));
         HIP_TRY(hipStreamSynchronize(s));
         if (flags[1]) return fail(PASC_ERR_HIP, "the workgroups of the persistent loop lost each other");
         passes += n;
@@ -708,8 +735,10 @@ static int run_phase(Engine &e, const PhaseCfg &ph, const pasc_spg_params &p, in
     int passes = 0;
     {
         bool ran;
-        const int rc0 = run_loop(e, ph, passes, max_passes, &ran);
+        int rc0 = run_loop(e, ph, passes, max_passes, &ran);
+        e.looped = rc0 == PASC_OK && ran;
         if (rc0 || ran) return rc0;
+        if ((rc0 = prepare(e, nullptr, 0))) return rc0;
     }
     if (e.cur_phase != (ph.f64 ? 1 : 0) || tile_len(e, ph.f64) != e.cur_tile) {
         int rc0 = engine_retile(e, ph.f64);
@@ -884,6 +913,28 @@ static int compute_normb(Engine &e, std::vector<InstState> &st) {
     return PASC_OK;
 }
 
+// The states of a phase to the device (a single problem's with its first kernel) and back.
+static int put_states(Engine &e, const std::vector<InstState> &st) {
+    if (e.n_inst == 1) {
+        e.init_state = st.data();  // alive until the phase has run
+        return PASC_OK;
+    }
+    HIP_TRY(hipMemcpyAsync(e.d_state, st.data(), sizeof(InstState) * e.n_inst,
+                           hipMemcpyHostToDevice, S_(e)));
+    return PASC_OK;
+}
+
+static int get_states(Engine &e, std::vector<InstState> &st) {
+    if (e.looped) {
+        st[0] = *e.h_state;
+        return PASC_OK;
+    }
+    HIP_TRY(hipMemcpyAsync(st.data(), e.d_state, sizeof(InstState) * e.n_inst,
+                           hipMemcpyDeviceToHost, S_(e)));
+    HIP_TRY(hipStreamSynchronize(S_(e)));
+    return PASC_OK;
+}
+
 int engine_solve(Engine &e, const pasc_spg_params &p, pasc_spg_result *res_single,
                  pasc_instance_result *res_multi, double *time_s) {
     hipStream_t s = S_(e);
@@ -910,33 +961,26 @@ int engine_solve(Engine &e, const pasc_spg_params &p, pasc_spg_result *res_singl
     }
     std::vector<char> all(e.n_inst, 1);
     init_states(e, st, p, all, false);
-    HIP_TRY(hipMemcpyAsync(e.d_state, st.data(), sizeof(InstState) * e.n_inst,
-                           hipMemcpyHostToDevice, s));
-    EventsGuard eg;
-    eg.ev.assign(2, nullptr);
-    HIP_TRY(hipEventCreate(&eg.ev[0]));
-    HIP_TRY(hipEventCreate(&eg.ev[1]));
-    hipEvent_t ev0 = eg.ev[0], ev1 = eg.ev[1];
+    int rc = put_states(e, st);
+    if (rc) return rc;
+    for (auto &v : e.ev_solve)
+        if (!v) HIP_TRY(hipEventCreate((hipEvent_t *)&v));
+    hipEvent_t ev0 = (hipEvent_t)e.ev_solve[0], ev1 = (hipEvent_t)e.ev_solve[1];
     HIP_TRY(hipEventRecord(ev0, s));
 
     const bool bulk32 = e.precision == PASC_FP32_BULK;
     std::vector<int> it32(e.n_inst, 0), it64(e.n_inst, 0);
-    int rc;
     if (!bulk32) {
         PhaseCfg ph{true, make_step(p, false), p.kkt_every};
         rc = run_phase(e, ph, p, p.maxit + 2);
         if (rc) return rc;
-        HIP_TRY(hipMemcpyAsync(st.data(), e.d_state, sizeof(InstState) * e.n_inst,
-                               hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        if ((rc = get_states(e, st))) return rc;
         for (int i = 0; i < e.n_inst; i++) { it64[i] = st[i].it; e.h_parity[i] = st[i].parity; }
     } else {
         PhaseCfg ph{false, make_step(p, true), p.kkt_every};
         rc = run_phase(e, ph, p, p.maxit + 2);
         if (rc) return rc;
-        HIP_TRY(hipMemcpyAsync(st.data(), e.d_state, sizeof(InstState) * e.n_inst,
-                               hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        if ((rc = get_states(e, st))) return rc;
         // FP64 polish: promote the FP32 iterate and certify the target in FP64
         if (!e.d_gamma64[0]) {
             for (int b = 0; b < 2; b++) {
@@ -965,24 +1009,23 @@ int engine_solve(Engine &e, const pasc_spg_params &p, pasc_spg_result *res_singl
         // polish_maxit -1: the polish gets what the FP32 phase left of maxit
         const bool shared_cap = p.polish_maxit < 0;
         for (int i = 0; i < e.n_inst; i++) st[i].it_base = shared_cap ? it32[i] : 0;
-        HIP_TRY(hipMemcpyAsync(e.d_state, st.data(), sizeof(InstState) * e.n_inst,
-                               hipMemcpyHostToDevice, s));
+        if ((rc = put_states(e, st))) return rc;
         pasc_spg_params pp = p;
         pp.maxit = p.polish_maxit > 0 ? p.polish_maxit : p.maxit;
         PhaseCfg ph2{true, make_step(pp, false), p.kkt_every};
         rc = run_phase(e, ph2, pp, pp.maxit + 2);
         if (rc) return rc;
         e.cur64 = true;
-        HIP_TRY(hipMemcpyAsync(st.data(), e.d_state, sizeof(InstState) * e.n_inst,
-                               hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        if ((rc = get_states(e, st))) return rc;
         for (int i = 0; i < e.n_inst; i++) {
             it64[i] = pol[i] ? st[i].it : 0;
             e.h_parity[i] = st[i].parity;
         }
     }
-    HIP_TRY(hipEventRecord(ev1, s));
-    HIP_TRY(hipEventSynchronize(ev1));
+    if (!e.looped) {  // (the loop recorded it before its last wait)
+        HIP_TRY(hipEventRecord(ev1, s));
+        HIP_TRY(hipEventSynchronize(ev1));
+    }
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, ev0, ev1));
     if (time_s) *time_s = ms * 1e-3;
@@ -1134,20 +1177,17 @@ int engine_theta_update(Engine &e, int inst, double *theta_out) {
 }
 
 int rows_labels(Engine &e, const void *g, bool f32, const InstDesc &d, int32_t *labels) {
-    const int blocks = (int)((d.T + 255) / 256);
-    void *buf;
-    int rc = scratch(e, sizeof(int32_t) * (size_t)d.T, &buf);
-    if (rc) return rc;
-    if (f32)
-        hipLaunchKernelGGL((labels_kernel<float>), dim3(blocks), dim3(256), 0, S_(e),
-                           (const float *)g, d, (int32_t *)buf);
-    else
-        hipLaunchKernelGGL((labels_kernel<double>), dim3(blocks), dim3(256), 0, S_(e),
-                           (const double *)g, d, (int32_t *)buf);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(labels, buf, sizeof(int32_t) * d.T, hipMemcpyDeviceToHost, S_(e)));
-    HIP_TRY(hipStreamSynchronize(S_(e)));
-    return PASC_OK;
+    return staged_transfer(
+        e.ctx, true, labels, sizeof(int32_t), d.T,
+        [=, &d](hipStream_t s, int64_t t0, int64_t n, void *p) {
+            const dim3 blocks((unsigned)((n + 255) / 256));
+            if (f32)
+                hipLaunchKernelGGL((labels_kernel<float>), blocks, dim3(256), 0, s,
+                                   (const float *)g + t0, n, d.ld, d.K, (int32_t *)p);
+            else
+                hipLaunchKernelGGL((labels_kernel<double>), blocks, dim3(256), 0, s,
+                                   (const double *)g + t0, n, d.ld, d.K, (int32_t *)p);
+        });
 }
 
 int engine_labels(Engine &e, int inst, int32_t *labels) {
@@ -1247,28 +1287,48 @@ int engine_commit_linear_term(Engine &e, int inst) {
     return engine_update_desc(e);
 }
 
+// every instance's gamma rows at 1/K (grid.y: instance, grid.x strides over the steps)
 template <typename S>
 __global__ __launch_bounds__(256) void fill_uniform_kernel(const InstDesc *desc, S *g) {
     const InstDesc &d = desc[blockIdx.y];
-    const int64_t n = (int64_t)d.K * d.ld;
     const S v = S(1.0 / d.K);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t t = i % d.ld;
-        g[d.goff + i] = t < d.T ? v : S(0);
-    }
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < d.T; t += (int64_t)gridDim.x * 256)
+        for (int k = 0; k < d.K; k++) g[d.goff + k * d.ld + t] = v;
+}
+
+template <typename S>
+__global__ __launch_bounds__(256) void fill_rows_kernel(S *g, int64_t T, int64_t ld, int K, S v) {
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < T; t += (int64_t)gridDim.x * 256)
+        for (int k = 0; k < K; k++) g[k * ld + t] = v;
+}
+
+int rows_fill_uniform(Ctx *ctx, void *rows, bool f32, int64_t T, int64_t ld, int K) {
+    hipStream_t s = (hipStream_t)ctx->stream;
+    const dim3 grid((unsigned)std::min<int64_t>((T + 255) / 256, 4096));
+    if (f32)
+        hipLaunchKernelGGL((fill_rows_kernel<float>), grid, dim3(256), 0, s, (float *)rows, T, ld, K,
+                           (float)(1.0 / K));
+    else
+        hipLaunchKernelGGL((fill_rows_kernel<double>), grid, dim3(256), 0, s, (double *)rows, T, ld,
+                           K, 1.0 / K);
+    HIP_TRY(hipGetLastError());
+    // the library's own stream orders what follows; a caller may take an external one away
+    if (!ctx->own_stream) HIP_TRY(hipStreamSynchronize(s));
+    return PASC_OK;
 }
 
 int engine_fill_uniform(Engine &e) {
     e.cur64 = false;
     for (int i = 0; i < e.n_inst; i++) e.h_parity[i] = 0;
-    const dim3 grid(64, (unsigned)e.n_inst);
+    int64_t tmax = 1;
+    for (const auto &d : e.h_desc) tmax = std::max(tmax, d.T);
+    const dim3 grid((unsigned)std::min<int64_t>((tmax + 255) / 256, e.n_inst > 8 ? 64 : 1024),
+                    (unsigned)e.n_inst);
     if (e.precision == PASC_FP32_BULK)
         hipLaunchKernelGGL((fill_uniform_kernel<float>), grid, dim3(256), 0, S_(e), e.d_desc, (float *)e.d_gamma[0]);
     else
         hipLaunchKernelGGL((fill_uniform_kernel<double>), grid, dim3(256), 0, S_(e), e.d_desc, (double *)e.d_gamma[0]);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(S_(e)));
     return PASC_OK;
 }
 

@@ -41,6 +41,7 @@ struct LoopArgs {
     PassArgs p;          // buffers, descriptor, state and step of the problem (grp, part and the
                          // counters are not used)
     double *ex;          // exchange area: `epochs` x (sums of nwg workgroups, then nwg x 2 edges)
+    InstState *out;      // pinned host copy of the final state
     int32_t *flags;      // pinned host words: [0] the instance is still active, [1] a wait ran out
     int32_t ntiles;      // one-wave tiles of the series
     int32_t tpw;         // tiles per workgroup
@@ -551,15 +552,19 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
         }
     }
     if (wg == 0 && wave == 0) {
-        InstState &g = A.p.state[0];
-        if (lane < A.p.sp.m) g.fs[lane] = window;
-        if (lane == 0) {
+        auto put = [&](InstState &g) {
+            if (lane < A.p.sp.m) g.fs[lane] = window;
+            if (lane != 0) return;
             g.f = st.f; g.f_prev = st.f_prev; g.dd_prev = st.dd_prev; g.dAd_prev = st.dAd_prev;
             g.dd = st.dd; g.dAd = st.dAd; g.gd = st.gd; g.alpha_dir = st.alpha_dir;
             g.alpha_apply = st.alpha_apply; g.beta_apply = st.beta_apply; g.kkt = st.kkt;
-            g.best_kkt = st.best_kkt; g.fs_last = st.fs_last; g.it = st.it; g.first = st.first;
-            g.active = st.active; g.reason = st.reason; g.status = st.status; g.stall = st.stall;
-            g.parity = st.parity;
+            g.best_kkt = st.best_kkt; g.normb = st.normb; g.fs_last = st.fs_last; g.it = st.it;
+            g.first = st.first; g.active = st.active; g.reason = st.reason; g.status = st.status;
+            g.stall = st.stall; g.parity = st.parity; g.it_base = st.it_base;
+        };
+        put(A.p.state[0]);
+        put(*A.out);
+        if (lane == 0) {
             A.flags[0] = st.active;
         }
     }

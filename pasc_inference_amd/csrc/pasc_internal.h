@@ -2,6 +2,7 @@
 #pragma once
 
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -154,7 +155,14 @@ struct Engine {
     int32_t *d_nactive = nullptr;        // device counter of active instances
     int32_t *d_done = nullptr;           // completed-slot counters and group partials of the
                                          // fused step (DONE_BYTES, single problems only)
-    int32_t *h_nactive = nullptr;        // pinned mirror
+    int32_t *h_nactive = nullptr;        // pinned: active instances, then active tiles per K group
+    InstState *h_state = nullptr;        // pinned: the final state of a single problem's loop
+    // single problems: h_desc (and the initial state of a solve) go to the device with the first
+    // kernel that needs them
+    bool desc_stale = false;
+    const InstState *init_state = nullptr;
+    bool looped = false;                 // the last phase ran the persistent loop (h_state holds)
+    void *ev_solve[2] = {nullptr, nullptr};  // hipEvents around a solve
     PassShape sh[2];                     // [0] FP32 phase of FP32-bulk, [1] every FP64 pass
     bool shape_pinned = false;           // the caller pinned sh: the tiled passes run it
     int grid_cap = 0;                    // persistent grid cap (0: 32 blocks per CU)
@@ -179,7 +187,11 @@ struct Ctx {
 int engine_alloc(Engine &e, Ctx *ctx, int precision, int stencil, int32_t grid_width,
                  const std::vector<InstDesc> &descs, int64_t data_elems);
 void engine_free(Engine &e);
-int engine_upload_data(Engine &e, const double *x_host, int64_t offset, int64_t n);
+// data of n nodes, interleaved [n][xdim] on the host, into rows of stride ld from element `offset`
+int engine_upload_data(Engine &e, const double *x_host, int64_t offset, int64_t n, int64_t ld,
+                       int xdim);
+// 1/K at every one of the T steps of K FP64 or FP32 rows
+int rows_fill_uniform(Ctx *ctx, void *rows, bool f32, int64_t T, int64_t ld, int K);
 // graph stencil geometry: T time steps of R nodes, grid width or CSR adjacency (host arrays)
 int engine_set_graph(Engine &e, int64_t T, int64_t R, int32_t width, const int64_t *nbr_ptr,
                      const int32_t *nbr_idx);
@@ -192,6 +204,7 @@ int engine_solve(Engine &e, const pasc_spg_params &p, pasc_spg_result *res_singl
                  pasc_instance_result *res_multi, double *time_s);
 int engine_eval(Engine &e, int inst, double *fx, double *kkt);
 int engine_eval_raw(Engine &e, int inst, double *fx, double *kkt, double *nb2);
+// after a change of h_desc: the device copy follows at once (batches) or with the next solve
 int engine_update_desc(Engine &e);
 int engine_theta_update(Engine &e, int inst, double *theta_out);
 int engine_labels(Engine &e, int inst, int32_t *labels);
@@ -218,6 +231,22 @@ int rows_theta(Engine &e, const void *g, bool f32, const InstDesc &d, const doub
 int rows_labels(Engine &e, const void *g, bool f32, const InstDesc &d, int32_t *labels);
 int rows_abserr(Engine &e, const void *g, bool f32, const InstDesc &d, const double *solution,
                 double *abserr);
+
+// transfer.hip: host <-> device transfers through pinned pieces shared by a device's contexts
+int staging_open(int device);   // once per context
+void staging_close(int device);
+// rows [K][ld] of T steps (f32 or FP64) <-> a host array of T*K doubles, interleaved (t*K + k) or
+// one row after another (k*T + t); return when the copy is done
+int rows_to_host(Ctx *ctx, const void *rows, bool f32, int64_t T, int64_t ld, int K, double *host,
+                 bool interleaved);
+int rows_from_host(Ctx *ctx, const double *host, bool interleaved, void *rows, bool f32,
+                   int64_t T, int64_t ld, int K);
+// the general form: `total` elements of esize bytes, in pieces; launch(stream, i0, n, p) enqueues
+// the kernel that writes (to_host) or reads elements [i0, i0 + n) at the pinned piece p.  It is
+// called from several threads.
+using PieceLaunch = std::function<void(struct ihipStream_t *, int64_t, int64_t, void *)>;
+int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t total,
+                    const PieceLaunch &launch);
 
 // noalloc.hip: the theta step with its partial sums in a static device array
 int noalloc_init(int device);  // once per device, with the device current

@@ -1,0 +1,257 @@
+// Host <-> device transfers of row-major state (gamma, explicit linear terms, data) in the
+// layouts of the C boundary.
+//
+// The caller's array is in the boundary's layout (interleaved or one row after another, FP64);
+// the device keeps padded rows of the problem's type.  A kernel does the change of layout and
+// type and reads or writes pinned host memory directly (48 - 55 GB/s in both directions, as fast
+// as the copy engine and without a device buffer in between); host threads move the pinned
+// pieces from and to the caller's pages.  240 MB (T = 1e7, K = 3) took 86 ms down and 73 ms up
+// when one host thread did the layout around a pageable copy; in 4 MiB pieces over 8 threads it
+// takes 5 ms, of which the link needs 4.3.  One thread would be bound by its page faults and
+// copies (23 ms), so transfers of 1 MiB and more are cut into up to 8 pieces at a time.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <condition_variable>
+#include <cstring>
+#include <functional>
+#include <mutex>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+#include "device_common.h"
+
+namespace pasc {
+
+// Element i of the boundary's array: row (k) and column (t) of the device rows.
+__device__ __forceinline__ void boundary_index(int64_t i, int64_t T, int K, int interleaved, int64_t &t,
+                                               int &k) {
+    if (interleaved) {
+        t = i / K;
+        k = (int)(i - t * K);
+    } else {
+        k = (int)(i / T);
+        t = i - (int64_t)k * T;
+    }
+}
+
+template <typename S>
+__global__ __launch_bounds__(256) void rows_pack(const S *rows, int64_t T, int64_t ld, int K,
+                                                 int interleaved, int64_t i0, int64_t n,
+                                                 double *out) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        int64_t t;
+        int k;
+        boundary_index(i0 + i, T, K, interleaved, t, k);
+        out[i] = (double)rows[k * ld + t];
+    }
+}
+
+template <typename S>
+__global__ __launch_bounds__(256) void rows_unpack(const double *in, int64_t T, int64_t ld, int K,
+                                                   int interleaved, int64_t i0, int64_t n,
+                                                   S *rows) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        int64_t t;
+        int k;
+        boundary_index(i0 + i, T, K, interleaved, t, k);
+        rows[k * ld + t] = S(in[i]);
+    }
+}
+
+// Pinned pieces of one device, shared by its contexts: at most SLOTS of SLOT_BYTES, allocated
+// when first needed and freed with the device's last context.  A transfer holds the slots it
+// works on and waits for none but its first, so transfers of several threads share them.
+struct Slot {
+    double *p = nullptr;
+    hipEvent_t ev = nullptr;
+};
+constexpr int SLOTS = 8;
+constexpr size_t SLOT_BYTES = (size_t)4 << 20;
+constexpr int POOL_DEVICES = 64;
+constexpr size_t STAGING_SINGLE = (size_t)1 << 20;      // up to here one thread is as fast
+constexpr size_t STAGING_PIECE_MIN = (size_t)256 << 10;  // pieces are multiples of this
+
+struct SlotPool {
+    std::mutex mu;
+    std::condition_variable cv;
+    std::vector<Slot> idle;
+    int allocated = 0;
+    int users = 0;
+
+    // a slot, or none when all are taken and wait is false
+    hipError_t take(bool wait, Slot &s) {
+        std::unique_lock<std::mutex> lk(mu);
+        for (;;) {
+            if (!idle.empty()) {
+                s = idle.back();
+                idle.pop_back();
+                return hipSuccess;
+            }
+            if (allocated < SLOTS) {
+                Slot n;
+                hipError_t e = hipHostMalloc((void **)&n.p, SLOT_BYTES, hipHostMallocDefault);
+                if (e != hipSuccess) return e;
+                e = hipEventCreateWithFlags(&n.ev, hipEventDisableTiming);
+                if (e != hipSuccess) {
+                    (void)hipHostFree(n.p);
+                    return e;
+                }
+                allocated++;
+                s = n;
+                return hipSuccess;
+            }
+            if (!wait) return hipErrorNotReady;
+            cv.wait(lk);
+        }
+    }
+    void give(const Slot &s) {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            idle.push_back(s);
+        }
+        cv.notify_one();
+    }
+};
+
+static SlotPool g_pool[POOL_DEVICES];
+
+int staging_open(int device) {
+    if (device < 0 || device >= POOL_DEVICES)
+        return fail(PASC_ERR_ARG, "staging: device %d beyond %d", device, POOL_DEVICES);
+    SlotPool &p = g_pool[device];
+    std::lock_guard<std::mutex> lk(p.mu);
+    p.idle.reserve(SLOTS);
+    p.users++;
+    return PASC_OK;
+}
+
+void staging_close(int device) {
+    if (device < 0 || device >= POOL_DEVICES) return;
+    SlotPool &p = g_pool[device];
+    std::lock_guard<std::mutex> lk(p.mu);
+    if (--p.users > 0) return;
+    for (auto &s : p.idle) {
+        (void)hipEventDestroy(s.ev);
+        (void)hipHostFree(s.p);
+    }
+    p.allocated -= (int)p.idle.size();
+    p.idle.clear();
+}
+
+// One transfer: pieces of `piece` elements, taken in turn by the calling thread and its helpers.
+struct Transfer {
+    int device;
+    hipStream_t stream;
+    bool to_host;
+    char *host;
+    size_t esize;
+    int64_t total, piece;
+    const PieceLaunch *launch;
+    std::atomic<int64_t> next{0};
+    std::atomic<int> error{(int)hipSuccess};
+
+    hipError_t one(const Slot &s, int64_t i0, int64_t n) {
+        if (!to_host) std::memcpy(s.p, host + (size_t)i0 * esize, (size_t)n * esize);
+        (*launch)(stream, i0, n, s.p);
+        hipError_t e;
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = hipEventRecord(s.ev, stream)) != hipSuccess) return e;
+        if ((e = hipEventSynchronize(s.ev)) != hipSuccess) return e;
+        if (to_host) std::memcpy(host + (size_t)i0 * esize, s.p, (size_t)n * esize);
+        return hipSuccess;
+    }
+
+    // first: the calling thread, which waits for a slot; helpers leave when there is none
+    void work(bool first) {
+        hipError_t e = first ? hipSuccess : hipSetDevice(device);
+        Slot s;
+        if (e == hipSuccess) {
+            e = g_pool[device].take(first, s);
+            if (!first && e != hipSuccess) return;  // the others do the work
+        }
+        if (e == hipSuccess) {
+            for (int64_t i = next.fetch_add(piece); i < total && error.load() == (int)hipSuccess;
+                 i = next.fetch_add(piece)) {
+                e = one(s, i, std::min(piece, total - i));
+                if (e != hipSuccess) break;
+            }
+            g_pool[device].give(s);
+        }
+        if (e != hipSuccess) {
+            int none = (int)hipSuccess;
+            error.compare_exchange_strong(none, (int)e);
+        }
+    }
+};
+
+int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t total,
+                    const PieceLaunch &launch) {
+    if (total <= 0) return PASC_OK;
+    Transfer t;
+    t.device = ctx->device;
+    t.stream = (hipStream_t)ctx->stream;
+    t.to_host = to_host;
+    t.host = (char *)host;
+    t.esize = esize;
+    t.total = total;
+    t.launch = &launch;
+    const int64_t slot = (int64_t)(SLOT_BYTES / esize), page = (int64_t)(STAGING_PIECE_MIN / esize);
+    const int most = std::min(SLOTS, std::max(1, (int)std::thread::hardware_concurrency() / 2));
+    t.piece = slot;
+    int helpers = 0;
+    if ((size_t)total * esize > STAGING_SINGLE) {
+        const int64_t share = (total + most - 1) / most;
+        t.piece = std::min(slot, (share + page - 1) / page * page);
+        helpers = (int)std::min<int64_t>(most, (total + t.piece - 1) / t.piece) - 1;
+    }
+    std::vector<std::thread> th;
+    try {
+        th.reserve(helpers);
+        for (int i = 0; i < helpers; i++) th.emplace_back([&t]() { t.work(false); });
+    } catch (const std::exception &) {
+        // fewer helpers: the threads that run, this one included, do the rest
+    }
+    t.work(true);
+    for (auto &x : th) x.join();
+    const hipError_t e = (hipError_t)t.error.load();
+    if (e != hipSuccess)
+        return fail(PASC_ERR_HIP, "%s transfer: %s", to_host ? "device to host" : "host to device",
+                    hipGetErrorString(e));
+    return PASC_OK;
+}
+
+static unsigned piece_blocks(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 1024); }
+
+int rows_to_host(Ctx *ctx, const void *rows, bool f32, int64_t T, int64_t ld, int K, double *host,
+                 bool interleaved) {
+    const int il = interleaved ? 1 : 0;
+    return staged_transfer(
+        ctx, true, host, sizeof(double), T * K, [=](hipStream_t s, int64_t i0, int64_t n, void *p) {
+            if (f32)
+                hipLaunchKernelGGL(rows_pack<float>, dim3(piece_blocks(n)), dim3(256), 0, s,
+                                   (const float *)rows, T, ld, K, il, i0, n, (double *)p);
+            else
+                hipLaunchKernelGGL(rows_pack<double>, dim3(piece_blocks(n)), dim3(256), 0, s,
+                                   (const double *)rows, T, ld, K, il, i0, n, (double *)p);
+        });
+}
+
+int rows_from_host(Ctx *ctx, const double *host, bool interleaved, void *rows, bool f32,
+                   int64_t T, int64_t ld, int K) {
+    const int il = interleaved ? 1 : 0;
+    return staged_transfer(
+        ctx, false, const_cast<double *>(host), sizeof(double), T * K,
+        [=](hipStream_t s, int64_t i0, int64_t n, void *p) {
+            if (f32)
+                hipLaunchKernelGGL(rows_unpack<float>, dim3(piece_blocks(n)), dim3(256), 0, s,
+                                   (const double *)p, T, ld, K, il, i0, n, (float *)rows);
+            else
+                hipLaunchKernelGGL(rows_unpack<double>, dim3(piece_blocks(n)), dim3(256), 0, s,
+                                   (const double *)p, T, ld, K, il, i0, n, (double *)rows);
+        });
+}
+
+}  // namespace pasc

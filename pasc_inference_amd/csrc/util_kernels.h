@@ -211,13 +211,14 @@ __global__ __launch_bounds__(256) void theta_partials(const S *gam, const double
 
 // ---- labels (argmax over k, lowest k on ties) and |sum_k theta_k gamma_k - sol| partials -----
 template <typename S>
-__global__ __launch_bounds__(256) void labels_kernel(const S *gam, InstDesc D, int32_t *lab) {
+__global__ __launch_bounds__(256) void labels_kernel(const S *gam, int64_t n, int64_t ld, int K,
+                                                     int32_t *lab) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= D.T) return;
+    if (t >= n) return;
     int best = 0;
     double bv = (double)gam[t];
-    for (int k = 1; k < D.K; k++) {
-        const double v = (double)gam[k * D.ld + t];
+    for (int k = 1; k < K; k++) {
+        const double v = (double)gam[k * ld + t];
         if (v > bv) { bv = v; best = k; }
     }
     lab[t] = best;
@@ -251,6 +252,19 @@ __global__ __launch_bounds__(256) void convert_kernel(const A *src, B *dst, int6
 static __global__ __launch_bounds__(256) void fill_u64(uint64_t *p, int64_t n, uint64_t v) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
         p[i] = v;
+}
+
+// ---- a single problem's descriptor and, with put_state, its initial state, handed over in kernel
+// arguments; the persistent loop's exchange area (n words) is marked empty by the same launch ----
+static __global__ __launch_bounds__(256) void prepare_single(InstDesc *desc, InstDesc d,
+                                                             InstState *state, InstState st,
+                                                             int put_state, uint64_t *ex, int64_t n) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *desc = d;
+        if (put_state) *state = st;
+    }
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        ex[i] = PART_EMPTY;
 }
 
 // ---- last gamma row ----------------------------------------------------------------------------
