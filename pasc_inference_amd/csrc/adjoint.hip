@@ -13,10 +13,12 @@
 // iteration needs no host round trip; the host reads the stop flag every CG_POLL iterations.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
 #include "device_common.h"
+#include "util_kernels.h"
 
 namespace pasc {
 
@@ -29,6 +31,12 @@ namespace pasc {
 
 constexpr int ANT = 256;
 constexpr double FREE_EPS = 1e-12;  // gamma entries at or below this are on the bound
+
+}  // namespace pasc
+
+#include "adjoint_loop.h"
+
+namespace pasc {
 
 struct AdjArgs {
     const double *gam;      // gamma* (k-major, stride ld)
@@ -55,23 +63,6 @@ struct CgState {
 constexpr int CG_POLL = 16;  // CG iterations launched between host reads of the stop flag
 constexpr int RNT = 1024;    // threads of the one-workgroup partial reductions
 
-// (A0 v)_n of one row
-__device__ inline double adj_lap(const AdjArgs &a, const double *row, int64_t n) {
-    const double c = row[n];
-    double l = 0.0;
-    for_neighbours(a.G, n, [&](int64_t n2, double w) { l += w * (c - row[n2]); });
-    return l;
-}
-
-// (A0 v)_n of one row of v = rv + b pv, formed at n and at its neighbours
-__device__ inline double adj_lap_upd(const AdjArgs &a, const double *rv, const double *pv,
-                                     double b, int64_t n) {
-    const double c = rv[n] + b * pv[n];
-    double l = 0.0;
-    for_neighbours(a.G, n, [&](int64_t n2, double w) { l += w * (c - (rv[n2] + b * pv[n2])); });
-    return l;
-}
-
 template <int NV>
 __device__ inline void block_sum(double (&v)[NV], double *lds, double *out) {
     const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
@@ -92,48 +83,61 @@ __device__ inline void block_sum(double (&v)[NV], double *lds, double *out) {
 }
 
 // P applied to the K values of one time step (in place); free flags per k.
-__device__ inline void project_face(double *v, const bool *fr, int K) {
+template <int K>
+__device__ __forceinline__ void project_face(double (&v)[K], const bool (&fr)[K]) {
     int nf = 0;
     double s = 0.0;
+#pragma unroll
     for (int k = 0; k < K; k++)
         if (fr[k]) { nf++; s += v[k]; }
     const double m = nf > 0 ? s / nf : 0.0;
+#pragma unroll
     for (int k = 0; k < K; k++) v[k] = (fr[k] && nf > 1) ? v[k] - m : 0.0;
 }
 
-// r = P dJ/dgamma; partials: [0] J, [1] r'r, [2 + k*xdim + c] direct dJ/dtheta_kc
+// r = P dJ/dgamma; partials: [0] J, [1] r'r, [2 + 3 k + c] direct dJ/dtheta_kc.  (K is a template
+// argument here and below so that the values of a step stay in registers.)
+template <int K>
 __global__ __launch_bounds__(ANT) void adj_init(AdjArgs a, double *r, double *part) {
-    __shared__ double lds[(2 + NTH) * (ANT / WAVE)];
+    constexpr int NV = 2 + 3 * K;
+    __shared__ double lds[NV * (ANT / WAVE)];
     const int64_t t = (int64_t)blockIdx.x * ANT + threadIdx.x;
-    double v[2 + NTH];
-    for (int i = 0; i < 2 + NTH; i++) v[i] = 0.0;
+    double v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) v[i] = 0.0;
     if (t < a.T) {
-        double g[PASC_MAX_K], dj[PASC_MAX_K];
-        bool fr[PASC_MAX_K];
-        for (int k = 0; k < a.K; k++) {
+        double g[K], dj[K];
+        bool fr[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
             g[k] = a.gam[k * a.ld + t];
             fr[k] = g[k] > FREE_EPS;
             a.freeset[k * a.ld + t] = fr[k] ? 1 : 0;
             dj[k] = 0.0;
         }
         const bool held = a.mask[t] != 0;
-        for (int c = 0; c < a.xdim; c++) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            if (c >= a.xdim) break;
             double rec = 0.0;
-            for (int k = 0; k < a.K; k++) rec += a.theta[k * a.xdim + c] * g[k];
+#pragma unroll
+            for (int k = 0; k < K; k++) rec += a.theta[k * a.xdim + c] * g[k];
             const double res = held ? a.x[c * a.ld + t] - rec : 0.0;
             v[0] += res * res;
-            for (int k = 0; k < a.K; k++) {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
                 dj[k] += -2.0 * res * a.theta[k * a.xdim + c];
-                v[2 + k * a.xdim + c] = -2.0 * res * g[k];
+                v[2 + 3 * k + c] = -2.0 * res * g[k];
             }
         }
-        project_face(dj, fr, a.K);
-        for (int k = 0; k < a.K; k++) {
+        project_face<K>(dj, fr);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
             r[k * a.ld + t] = dj[k];
             v[1] += dj[k] * dj[k];
         }
     }
-    block_sum<2 + NTH>(v, lds, part);
+    block_sum<NV>(v, lds, part);
 }
 
 // Sum of part[0 .. blocks) in a fixed order (thread i adds blocks i, i + RNT, ..., then the
@@ -179,6 +183,7 @@ __global__ __launch_bounds__(RNT) void adj_cg_rr(const double *part, int blocks,
 // The search direction p = r + b pold of this step (b = 0 on the first, where pold = r), written
 // to pnew, and q = P A P p (p in range(P)); partial p'q.  pnew and pold are two buffers, since
 // the neighbours' pold are read while other workgroups write.
+template <int K>
 __global__ __launch_bounds__(ANT) void adj_matvec(AdjArgs a, const double *r, const double *pold,
                                                   double *pnew, double *q, double *part,
                                                   const CgState *cs) {
@@ -188,16 +193,25 @@ __global__ __launch_bounds__(ANT) void adj_matvec(AdjArgs a, const double *r, co
     const int64_t t = (int64_t)blockIdx.x * ANT + threadIdx.x;
     double v[1] = {0.0};
     if (t < a.T) {
-        double w[PASC_MAX_K], pn[PASC_MAX_K];
-        bool fr[PASC_MAX_K];
-        for (int k = 0; k < a.K; k++) {
-            const double *rv = r + k * a.ld, *pv = pold + k * a.ld;
-            pn[k] = rv[t] + b * pv[t];
-            w[k] = a.alpha * adj_lap_upd(a, rv, pv, b, t);
+        double w[K], pn[K];
+        bool fr[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            pn[k] = r[k * a.ld + t] + b * pold[k * a.ld + t];
             fr[k] = a.freeset[k * a.ld + t] != 0;
+            w[k] = 0.0;
         }
-        project_face(w, fr, a.K);
-        for (int k = 0; k < a.K; k++) {
+        // (A0 p) at the node, p formed at the neighbours too
+        for_neighbours(a.G, t, [&](int64_t n2, double wt) {
+#pragma unroll
+            for (int k = 0; k < K; k++)
+                w[k] += wt * (pn[k] - (r[k * a.ld + n2] + b * pold[k * a.ld + n2]));
+        });
+#pragma unroll
+        for (int k = 0; k < K; k++) w[k] *= a.alpha;
+        project_face<K>(w, fr);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
             pnew[k * a.ld + t] = pn[k];
             q[k * a.ld + t] = w[k];
             v[0] += pn[k] * w[k];
@@ -207,6 +221,7 @@ __global__ __launch_bounds__(ANT) void adj_matvec(AdjArgs a, const double *r, co
 }
 
 // lam += s p; r -= s q with s the step; partial r'r
+template <int K>
 __global__ __launch_bounds__(ANT) void adj_axpy(AdjArgs a, const CgState *cs, const double *p,
                                                 const double *q, double *lam, double *r,
                                                 double *part) {
@@ -216,34 +231,54 @@ __global__ __launch_bounds__(ANT) void adj_axpy(AdjArgs a, const CgState *cs, co
     const int64_t t = (int64_t)blockIdx.x * ANT + threadIdx.x;
     double v[1] = {0.0};
     if (t < a.T) {
-        for (int k = 0; k < a.K; k++) {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
             const int64_t i = k * a.ld + t;
             lam[i] += s * p[i];
-            r[i] -= s * q[i];
-            v[0] += r[i] * r[i];
+            const double rn = r[i] - s * q[i];
+            r[i] = rn;
+            v[0] += rn * rn;
         }
     }
     block_sum<1>(v, lds, part);
 }
 
-// partials: [0] lambda' A gamma, [1 + k*xdim + c] sum_{n with data} lambda_kn 2 (x_nc - theta_kc) bscale
+// partials: [0] lambda' A gamma, [1 + 3 k + c] sum_{n with data} lambda_kn 2 (x_nc - theta_kc) bscale
+template <int K>
 __global__ __launch_bounds__(ANT) void adj_final(AdjArgs a, const double *lam, double *part) {
-    __shared__ double lds[(1 + NTH) * (ANT / WAVE)];
+    constexpr int NV = 1 + 3 * K;
+    __shared__ double lds[NV * (ANT / WAVE)];
     const int64_t t = (int64_t)blockIdx.x * ANT + threadIdx.x;
-    double v[1 + NTH];
-    for (int i = 0; i < 1 + NTH; i++) v[i] = 0.0;
+    double v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) v[i] = 0.0;
     if (t < a.T) {
         const bool nodata = a.qmask && a.qmask[t] != 0;  // b_kn does not depend on theta there
-        for (int k = 0; k < a.K; k++) {
-            const double lk = lam[k * a.ld + t];
-            v[0] += lk * a.alpha * adj_lap(a, a.gam + k * a.ld, t);
-            if (!nodata)
-                for (int c = 0; c < a.xdim; c++)
-                    v[1 + k * a.xdim + c] =
-                        lk * 2.0 * (a.x[c * a.ld + t] - a.theta[k * a.xdim + c]) * a.bscale;
+        double g[K], l[K], lk[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            g[k] = a.gam[k * a.ld + t];
+            lk[k] = lam[k * a.ld + t];
+            l[k] = 0.0;
+        }
+        for_neighbours(a.G, t, [&](int64_t n2, double w) {
+#pragma unroll
+            for (int k = 0; k < K; k++) l[k] += w * (g[k] - a.gam[k * a.ld + n2]);
+        });
+#pragma unroll
+        for (int k = 0; k < K; k++) v[0] += lk[k] * a.alpha * l[k];
+        if (!nodata) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                if (c >= a.xdim) break;
+                const double xc = a.x[c * a.ld + t];
+#pragma unroll
+                for (int k = 0; k < K; k++)
+                    v[1 + 3 * k + c] = lk[k] * 2.0 * (xc - a.theta[k * a.xdim + c]) * a.bscale;
+            }
         }
     }
-    block_sum<1 + NTH>(v, lds, part);
+    block_sum<NV>(v, lds, part);
 }
 
 static int sum_partials(hipStream_t s, const double *d_part, int blocks, int nv,
@@ -263,47 +298,143 @@ __global__ __launch_bounds__(256) void adj_convert(const A *src, B *dst, int64_t
     if (i < n) dst[i] = B(src[i]);
 }
 
-int engine_adjoint(Engine &e, int inst, const uint8_t *mask_host, double cg_tol, int cg_maxit,
-                   double *loss, double *dlogeps, double *dtheta, int *cg_it) {
-    const InstDesc &D = e.h_desc[inst];
-    if (D.b64) return fail(PASC_ERR_ARG, "adjoint: needs the data term");
+__global__ __launch_bounds__(256) void copy_bytes(const uint8_t *src, uint8_t *dst, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        dst[i] = src[i];
+}
+
+// the caller's mask to the device
+static int upload_mask(Engine &e, const uint8_t *mask, uint8_t *dst, int64_t n) {
+    return staged_transfer(e.ctx, false, const_cast<uint8_t *>(mask), 1, n,
+                           [=](hipStream_t s, int64_t i0, int64_t m, void *p) {
+                               const unsigned b = (unsigned)std::min<int64_t>((m + 255) / 256, 1024);
+                               hipLaunchKernelGGL(copy_bytes, dim3(b), dim3(256), 0, s,
+                                                  (const uint8_t *)p, dst + i0, m);
+                           });
+}
+
+struct AdjResult {
+    double loss, lag;  // J and lambda' A gamma
+    double dtheta[PASC_MAX_K * 3];
+    int it;
+};
+
+// One problem on the 1-D graph whose CG vectors fit on chip: the persistent launch (adjoint_loop.h).
+// *ran = false when it does not qualify or the launch is refused.
+template <int K, int CH, int NW>
+static bool launch_adj_loop(const AdjLoopArgs &a, int nwg, hipStream_t s) {
+    const void *fn = reinterpret_cast<const void *>(adj_loop<K, CH, NW>);
+    const size_t lds = (size_t)K * NW * WAVE * CH * sizeof(double);
+    AdjLoopArgs args = a;
+    void *params[] = {&args};
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
+        hipLaunchCooperativeKernel(fn, dim3(nwg), dim3(NW * WAVE), params, (unsigned)lds, s) == hipSuccess)
+        return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+template <int K>
+static int run_adj_loop(Engine &e, const InstDesc &D, const double *gam, const uint8_t *mask_host,
+                        double cg_tol, int cg_maxit, AdjResult &res, bool *ran) {
+    *ran = false;
+    constexpr int CH = adj_chunk(K);
+    const int64_t n_cu = std::max(e.ctx->n_cu, 1);
+    auto groups = [&](int steps) { return (D.T + steps - 1) / steps; };
+    // 4 waves of half chunks, 8 of half chunks, 8 of whole chunks: the first whose workgroups fit
+    const int steps = groups(4 * WAVE * CH / 2) <= n_cu ? 4 * WAVE * CH / 2
+                      : groups(8 * WAVE * CH / 2) <= n_cu ? 8 * WAVE * CH / 2 : 8 * WAVE * CH;
+    if (groups(steps) > n_cu) return PASC_OK;
     hipStream_t s = (hipStream_t)e.ctx->stream;
-    const int64_t T = D.T, ld = D.ld, n = (int64_t)D.K * ld;
-    const int blocks = (int)((T + ANT - 1) / ANT);
-    const int par = e.h_parity[inst];
-    double *buf = nullptr;
-    uint8_t *fr = nullptr, *mk = nullptr;
-    double *part = nullptr;
-    CgState *d_cs = nullptr;
-    // gamma (FP64 copy when the state is FP32), lambda, r, q and two buffers of p
-    HIP_TRY(hipMalloc(&buf, sizeof(double) * 6 * (size_t)n));
-    HIP_TRY(hipMalloc(&fr, (size_t)n));
-    HIP_TRY(hipMalloc(&mk, (size_t)T));
-    HIP_TRY(hipMalloc(&part, sizeof(double) * (size_t)blocks * (2 + NTH)));
-    HIP_TRY(hipMalloc(&d_cs, sizeof(CgState)));
-    double *gam = buf, *lam = buf + n, *r = buf + 2 * n, *q = buf + 3 * n;
-    double *pb[2] = {buf + 4 * n, buf + 5 * n};
-    int rc = PASC_OK;
-    auto cleanup = [&]() {
-        (void)hipFree(buf);
-        (void)hipFree(fr);
-        (void)hipFree(mk);
-        (void)hipFree(part);
-        (void)hipFree(d_cs);
-    };
-    const unsigned cb = (unsigned)((n + 255) / 256);
-    if (e.cur64) {
-        hipLaunchKernelGGL((adj_convert<double, double>), dim3(cb), dim3(256), 0, s,
-                           (const double *)e.d_gamma64[par] + D.goff, gam, n);
-    } else if (e.precision == PASC_FP32_BULK) {
-        hipLaunchKernelGGL((adj_convert<float, double>), dim3(cb), dim3(256), 0, s,
-                           (const float *)e.d_gamma[par] + D.goff, gam, n);
-    } else {
-        hipLaunchKernelGGL((adj_convert<double, double>), dim3(cb), dim3(256), 0, s,
-                           (const double *)e.d_gamma[par] + D.goff, gam, n);
+    const int nwg = (int)groups(steps);
+    const int64_t ew = adj_epoch_words<K>(nwg), ow = adj_open_words<K>(nwg);
+    const int64_t cap = std::max<int64_t>(1, LOOP_EXCHANGE_BYTES / (8 * ew));
+    const int epochs = (int)std::min<int64_t>(std::max(cg_maxit, 1), std::min<int64_t>(cap, 512));
+    // exchange area, r'r, (with more steps than a launch holds) r, p and lambda, the mask
+    const int64_t save = cg_maxit > epochs ? 3 * (int64_t)K * D.ld : 0;
+    const size_t bytes = sizeof(double) * (size_t)(ow + ew * epochs + 2 + save) + (size_t)D.T;
+    void *buf;
+    int rc = engine_scratch(e, bytes, &buf);
+    if (rc) return rc;
+    double *ex = (double *)buf;
+    uint8_t *mk = (uint8_t *)(ex + ow + ew * epochs + 2 + save);
+    rc = upload_mask(e, mask_host, mk, D.T);
+    if (rc) return rc;
+    AdjLoopArgs a{};
+    a.gam = gam;
+    a.x = (const double *)e.d_x64 + D.xoff;
+    a.mask = mk;
+    a.qmask = D.heldout;
+    a.T = D.T;
+    a.ld = D.ld;
+    a.alpha = D.alpha;
+    a.bscale = D.bscale;
+    a.tol2 = cg_tol * cg_tol;
+    for (int k = 0; k < K; k++) a.theta[k] = D.theta[k];
+    a.save_rr = ex + ow + ew * epochs;
+    a.save = a.save_rr + 2;
+    a.out = (double *)e.h_state;  // pinned; no solve is under way
+    a.flags = e.h_nactive;
+    a.ex = ex;
+    a.epochs = epochs;
+    a.maxit = cg_maxit;
+    for (a.resume = 0;; a.resume = 1) {
+        const int64_t words = ow + ew * epochs;
+        hipLaunchKernelGGL(fill_u64, dim3((unsigned)std::min<int64_t>((words + 255) / 256, 1024)),
+                           dim3(256), 0, s, (uint64_t *)ex, words, PART_EMPTY);
+        HIP_TRY(hipGetLastError());
+        a.flags[0] = 0;
+        a.flags[1] = 0;
+        const bool ok = steps == 4 * WAVE * CH / 2   ? launch_adj_loop<K, CH / 2, 4>(a, nwg, s)
+                        : steps == 8 * WAVE * CH / 2 ? launch_adj_loop<K, CH / 2, 8>(a, nwg, s)
+                                                     : launch_adj_loop<K, CH, 8>(a, nwg, s);
+        if (!ok) return PASC_OK;
+        HIP_TRY(hipStreamSynchronize(s));
+        if (a.flags[1]) return fail(PASC_ERR_HIP, "adjoint: the workgroups lost each other");
+        if (!a.flags[0]) break;
     }
-    HIP_TRY(hipMemcpyAsync(mk, mask_host, (size_t)T, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemsetAsync(buf + n, 0, sizeof(double) * 5 * (size_t)n, s));
+    res.loss = a.out[0];
+    res.lag = a.out[1];
+    for (int k = 0; k < K; k++) res.dtheta[k] = a.out[2 + k];
+    res.it = a.flags[2];
+    *ran = true;
+    return PASC_OK;
+}
+
+// Any graph, size and number of channels: CG as kernels over vectors in device memory.
+template <int K>
+static int run_adj_kernels(Engine &e, const InstDesc &D, const uint8_t *mask_host, double cg_tol,
+                           int cg_maxit, AdjResult &res) {
+    hipStream_t s = (hipStream_t)e.ctx->stream;
+    const int64_t T = D.T, ld = D.ld, n = (int64_t)K * ld;
+    const int blocks = (int)((T + ANT - 1) / ANT);
+    const int par = e.h_parity[0];
+    constexpr int NV = 2 + 3 * K;
+    // gamma when the state is FP32, lambda, r, q and two buffers of p, the partials, the CG
+    // state, the free set and the mask
+    const bool f32 = !e.cur64 && e.precision == PASC_FP32_BULK;
+    void *mem;
+    int rc = engine_scratch(e, sizeof(double) * (size_t)(6 * n + (int64_t)blocks * NV) + 128 +
+                                   (size_t)n + (size_t)T, &mem);
+    if (rc) return rc;
+    double *buf = (double *)mem;
+    double *lam = buf + n, *r = buf + 2 * n, *q = buf + 3 * n;
+    double *pb[2] = {buf + 4 * n, buf + 5 * n};
+    double *part = buf + 6 * n;
+    CgState *d_cs = (CgState *)(part + (int64_t)blocks * NV);
+    uint8_t *fr = (uint8_t *)d_cs + 128, *mk = fr + n;
+    static_assert(sizeof(CgState) <= 128, "the CG state fits its place");
+    const double *gam = e.cur64 ? (const double *)e.d_gamma64[par] + D.goff
+                                : (const double *)e.d_gamma[par] + D.goff;
+    if (f32) {
+        gam = buf;
+        hipLaunchKernelGGL((convert_kernel<float, double>), dim3((unsigned)((n + 255) / 256)), dim3(256),
+                           0, s, (const float *)e.d_gamma[par] + D.goff, buf, n);
+        HIP_TRY(hipGetLastError());
+    }
+    rc = upload_mask(e, mask_host, mk, T);
+    if (rc) return rc;
+    HIP_TRY(hipMemsetAsync(lam, 0, sizeof(double) * (size_t)n, s));
     AdjArgs a;
     a.gam = gam;
     a.x = (const double *)e.d_x64 + D.xoff;
@@ -312,19 +443,20 @@ int engine_adjoint(Engine &e, int inst, const uint8_t *mask_host, double cg_tol,
     a.freeset = fr;
     a.T = T;
     a.ld = ld;
-    a.K = D.K;
+    a.K = K;
     a.xdim = D.xdim;
     a.alpha = D.alpha;
     a.bscale = D.bscale;
-    for (int i = 0; i < NTH; i++) a.theta[i] = i < D.K * D.xdim ? D.theta[i] : 0.0;
+    for (int i = 0; i < NTH; i++) a.theta[i] = i < K * D.xdim ? D.theta[i] : 0.0;
     a.G = e.stencil == STENCIL_TIME ? GraphGeo{T, 1, 0, nullptr, nullptr} : e.geo;
 
     std::vector<double> v;
-    hipLaunchKernelGGL(adj_init, dim3(blocks), dim3(ANT), 0, s, a, r, part);
+    hipLaunchKernelGGL(adj_init<K>, dim3(blocks), dim3(ANT), 0, s, a, r, part);
     HIP_TRY(hipGetLastError());
-    if ((rc = sum_partials(s, part, blocks, 2 + NTH, v))) { cleanup(); return rc; }
-    *loss = v[0];
-    std::vector<double> direct(v.begin() + 2, v.begin() + 2 + D.K * D.xdim);
+    if ((rc = sum_partials(s, part, blocks, NV, v))) return rc;
+    res.loss = v[0];
+    for (int k = 0; k < K; k++)
+        for (int c = 0; c < D.xdim; c++) res.dtheta[k * D.xdim + c] = v[2 + 3 * k + c];
     HIP_TRY(hipMemcpyAsync(pb[0], r, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, s));
     // conjugate gradients on P A P (symmetric positive semi-definite on range(P)), the scalars
     // on the device; the host reads the stop flag every CG_POLL iterations
@@ -340,10 +472,10 @@ int engine_adjoint(Engine &e, int inst, const uint8_t *mask_host, double cg_tol,
             // step launched + i reads p from pb[(launched + i) & 1] and writes the other
             const double *pold = pb[i & 1];
             double *pnew = pb[(i + 1) & 1];
-            hipLaunchKernelGGL(adj_matvec, dim3(blocks), dim3(ANT), 0, s, a, r, pold, pnew, q,
+            hipLaunchKernelGGL(adj_matvec<K>, dim3(blocks), dim3(ANT), 0, s, a, r, pold, pnew, q,
                                part, d_cs);
             hipLaunchKernelGGL(adj_cg_step, dim3(1), dim3(RNT), 0, s, part, blocks, d_cs);
-            hipLaunchKernelGGL(adj_axpy, dim3(blocks), dim3(ANT), 0, s, a, d_cs, pnew, q, lam, r,
+            hipLaunchKernelGGL(adj_axpy<K>, dim3(blocks), dim3(ANT), 0, s, a, d_cs, pnew, q, lam, r,
                                part);
             hipLaunchKernelGGL(adj_cg_rr, dim3(1), dim3(RNT), 0, s, part, blocks, d_cs);
         }
@@ -351,14 +483,52 @@ int engine_adjoint(Engine &e, int inst, const uint8_t *mask_host, double cg_tol,
         HIP_TRY(hipMemcpyAsync(&h, d_cs, sizeof(CgState), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
     }
-    const int it = h.it;
+    res.it = h.it;
+    hipLaunchKernelGGL(adj_final<K>, dim3(blocks), dim3(ANT), 0, s, a, lam, part);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(adj_final, dim3(blocks), dim3(ANT), 0, s, a, lam, part);
-    if ((rc = sum_partials(s, part, blocks, 1 + NTH, v))) { cleanup(); return rc; }
-    *dlogeps = -v[0];
-    for (int i = 0; i < D.K * D.xdim; i++) dtheta[i] = direct[i] + v[1 + i];
-    if (cg_it) *cg_it = it;
-    cleanup();
+    if ((rc = sum_partials(s, part, blocks, 1 + 3 * K, v))) return rc;
+    res.lag = v[0];
+    for (int k = 0; k < K; k++)
+        for (int c = 0; c < D.xdim; c++) res.dtheta[k * D.xdim + c] += v[1 + 3 * k + c];
+    return PASC_OK;
+}
+
+template <int K>
+static int run_adj(Engine &e, const InstDesc &D, const uint8_t *mask, double cg_tol, int cg_maxit,
+                   AdjResult &res) {
+    const bool f32 = !e.cur64 && e.precision == PASC_FP32_BULK;
+    if (e.stencil == STENCIL_TIME && D.xdim == 1 && !f32 && !e.profile) {
+        const int par = e.h_parity[0];
+        const double *gam = (const double *)(e.cur64 ? e.d_gamma64[par] : e.d_gamma[par]) + D.goff;
+        bool ran;
+        const int rc = run_adj_loop<K>(e, D, gam, mask, cg_tol, cg_maxit, res, &ran);
+        if (rc || ran) return rc;
+    }
+    return run_adj_kernels<K>(e, D, mask, cg_tol, cg_maxit, res);
+}
+
+int engine_adjoint(Engine &e, int inst, const uint8_t *mask_host, double cg_tol, int cg_maxit,
+                   double *loss, double *dlogeps, double *dtheta, int *cg_it) {
+    const InstDesc &D = e.h_desc[inst];
+    if (D.b64) return fail(PASC_ERR_ARG, "adjoint: needs the data term");
+    AdjResult r{};
+    int rc;
+    switch (D.K) {
+        case 1: rc = run_adj<1>(e, D, mask_host, cg_tol, cg_maxit, r); break;
+        case 2: rc = run_adj<2>(e, D, mask_host, cg_tol, cg_maxit, r); break;
+        case 3: rc = run_adj<3>(e, D, mask_host, cg_tol, cg_maxit, r); break;
+        case 4: rc = run_adj<4>(e, D, mask_host, cg_tol, cg_maxit, r); break;
+        case 5: rc = run_adj<5>(e, D, mask_host, cg_tol, cg_maxit, r); break;
+        case 6: rc = run_adj<6>(e, D, mask_host, cg_tol, cg_maxit, r); break;
+        case 7: rc = run_adj<7>(e, D, mask_host, cg_tol, cg_maxit, r); break;
+        case 8: rc = run_adj<8>(e, D, mask_host, cg_tol, cg_maxit, r); break;
+        default: rc = fail(PASC_ERR_ARG, "unsupported K");
+    }
+    if (rc) return rc;
+    *loss = r.loss;
+    *dlogeps = -r.lag;
+    for (int i = 0; i < D.K * D.xdim; i++) dtheta[i] = r.dtheta[i];
+    if (cg_it) *cg_it = r.it;
     if (!std::isfinite(*dlogeps)) return fail(PASC_ERR_NUMERIC, "adjoint: non-finite gradient");
     return PASC_OK;
 }

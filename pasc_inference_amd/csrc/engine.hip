@@ -324,7 +324,7 @@ void engine_free(Engine &e) {
     e.d_scratch = nullptr;
 }
 
-static int scratch(Engine &e, size_t bytes, void **p) {
+int engine_scratch(Engine &e, size_t bytes, void **p) {
     if (bytes > e.scratch_bytes) {
         if (e.d_scratch) (void)hipFree(e.d_scratch);
         e.d_scratch = nullptr;
@@ -682,7 +682,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
     const int64_t cap = std::max<int64_t>(1, LOOP_EXCHANGE_BYTES / (8 * pl.epoch_words));
     const int epochs = (int)std::min<int64_t>(std::min(max_passes, LOOP_EPOCHS_MAX), cap);
     void *ex;
-    int rc = scratch(e, sizeof(double) * (size_t)pl.epoch_words * (epochs + 1), &ex);
+    int rc = engine_scratch(e, sizeof(double) * (size_t)pl.epoch_words * (epochs + 1), &ex);
     if (rc) return rc;
     const bool g64 = ph.f64 && e.precision == PASC_FP32_BULK;
     int32_t *flags = e.h_nactive;
@@ -1098,7 +1098,7 @@ int engine_eval_raw(Engine &e, int inst, double *fx, double *kkt, double *nb2) {
     const void *g = cur_gamma(e, inst, f32);
     const int blocks = (int)((d.T + 255) / 256);
     void *part;
-    int rc = scratch(e, sizeof(double) * 3 * (size_t)blocks, &part);
+    int rc = engine_scratch(e, sizeof(double) * 3 * (size_t)blocks, &part);
     if (rc) return rc;
     switch (d.K) {
         case 1: launch_eval<1>(e, d, g, f32, (double *)part, blocks); break;
@@ -1137,7 +1137,7 @@ int rows_theta(Engine &e, const void *g, bool f32, const InstDesc &d, const doub
     const int blocks = (int)((d.T + 255) / 256);
     const int nv = d.K * (1 + d.xdim);
     void *part;
-    int rc = scratch(e, sizeof(double) * (size_t)nv * blocks, &part);
+    int rc = engine_scratch(e, sizeof(double) * (size_t)nv * blocks, &part);
     if (rc) return rc;
     if (f32)
         hipLaunchKernelGGL((theta_partials<float>), dim3(blocks), dim3(256), 0, S_(e),
@@ -1202,7 +1202,7 @@ int rows_abserr(Engine &e, const void *g, bool f32, const InstDesc &d, const dou
     const int blocks = (int)((d.T + 255) / 256);
     void *buf;
     const size_t need = sizeof(double) * ((size_t)d.T + blocks);
-    int rc = scratch(e, need, &buf);
+    int rc = engine_scratch(e, need, &buf);
     if (rc) return rc;
     double *sol = (double *)buf;
     double *part = sol + d.T;

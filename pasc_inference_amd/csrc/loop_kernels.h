@@ -25,17 +25,15 @@
 // only if they all fit.  Waits are bounded; a value that does not come makes the solve fail.
 #pragma once
 
+#include "exchange.h"
 #include "spg_kernels.h"
 
 namespace pasc {
 
-constexpr int LOOP_SPIN_LIMIT = 1 << 22;  // re-reads (~1 us each) before a value counts as lost
 
 constexpr int LOOP_WAVES_MIN = 4;         // waves per workgroup: one per SIMD of the CU,
 constexpr int LOOP_WAVES_MAX = 8;         // or two when a workgroup has more than 4 tiles
-constexpr size_t LOOP_LDS_BYTES = 159 * 1024;        // dynamic LDS (160 KiB less the static part)
 constexpr int LOOP_EPOCHS_MAX = 512;                 // iterations per launch at most
-constexpr int64_t LOOP_EXCHANGE_BYTES = 16 << 20;    // exchange area at most
 
 struct LoopArgs {
     PassArgs p;          // buffers, descriptor, state and step of the problem (grp, part and the
@@ -58,10 +56,6 @@ constexpr bool loop_has_chunk(bool f64, int K, int ch) {
     return f64 ? ch == 2 || (ch == 4 && K <= 4) : ch == 4;
 }
 
-// The exchange area holds each of the five sums as one row over the workgroups (a wave reads 64
-// workgroups' values as 512 contiguous bytes).
-__host__ __device__ constexpr int slot_stride(int nwg) { return (nwg + 15) / 16 * 16; }
-
 // Layout of a workgroup's dynamic LDS and of the exchange area, used on both sides.
 template <typename S, int K, int CH>
 struct LoopShape {
@@ -80,64 +74,6 @@ struct LoopShape {
         return (int64_t)slot_stride(nwg) * NPART + (int64_t)nwg * 2 * EDGE;
     }
 };
-
-// ---- wave-wide sums by lane swaps and DPP (VALU moves; no LDS round trips) -------------------
-template <int CTRL>
-__device__ __forceinline__ double dpp_from(double v) {
-    const long long u = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)(unsigned)hi << 32) | (long long)(unsigned)lo);
-}
-__device__ __forceinline__ double from_lane(double v, int lane) {
-    const long long u = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)u, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
-    return __longlong_as_double(((long long)(unsigned)hi << 32) | (long long)(unsigned)lo);
-}
-__device__ __forceinline__ double join_words(unsigned lo, unsigned hi) {
-    return __longlong_as_double(((long long)hi << 32) | (long long)lo);
-}
-// a's upper 32 lanes <-> b's lower 32 lanes (v_permlane32_swap), and a's odd rows of 16 lanes <->
-// b's even rows (v_permlane16_swap): after either, a + b holds a's pairwise sums in one half of
-// the lanes and b's in the other, so two values are folded by two swaps and one add
-__device__ __forceinline__ double fold32(double a, double b) {
-    const long long u = __double_as_longlong(a), w = __double_as_longlong(b);
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)w, false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(w >> 32), false, false);
-    return join_words(lo[0], hi[0]) + join_words(lo[1], hi[1]);
-}
-__device__ __forceinline__ double fold16(double a, double b) {
-    const long long u = __double_as_longlong(a), w = __double_as_longlong(b);
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)w, false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(w >> 32), false, false);
-    return join_words(lo[0], hi[0]) + join_words(lo[1], hi[1]);
-}
-constexpr int DPP_ROR = 0x120;          // + n: rotate within a row of 16 lanes
-constexpr int DPP_XOR1 = 0xB1;          // quad_perm 1,0,3,2
-constexpr int DPP_XOR2 = 0x4E;          // quad_perm 2,3,0,1
-constexpr int DPP_HALF_MIRROR = 0x141;  // lane i <- lane 7 - i of its half row
-// sums of four values over the wave: every lane of row 0 / 1 / 2 / 3 (16 lanes each) ends with
-// the sum of a / c / b / d
-__device__ __forceinline__ double wave_sum4(double a, double b, double c, double d) {
-    double v = fold16(fold32(a, b), fold32(c, d));
-    v += dpp_from<DPP_ROR + 8>(v);
-    v += dpp_from<DPP_ROR + 4>(v);
-    v += dpp_from<DPP_ROR + 2>(v);
-    v += dpp_from<DPP_ROR + 1>(v);
-    return v;
-}
-constexpr int ROW_A = 0, ROW_B = 32, ROW_C = 16, ROW_D = 48;  // a lane of each sum
-__device__ __forceinline__ double nan_max(double a, double b) { return (b > a || b != b) ? b : a; }
-// maximum over the wave (a NaN wins), in every lane
-__device__ __forceinline__ double wave_max_all(double v) {
-    v = nan_max(v, dpp_from<DPP_ROR + 8>(v));
-    v = nan_max(v, dpp_from<DPP_ROR + 4>(v));
-    v = nan_max(v, dpp_from<DPP_ROR + 2>(v));
-    v = nan_max(v, dpp_from<DPP_ROR + 1>(v));
-    return nan_max(nan_max(from_lane(v, 0), from_lane(v, 16)),
-                   nan_max(from_lane(v, 32), from_lane(v, 48)));
-}
 
 // The scalar fields of InstState, in registers of wave 0 (the same in every lane).
 struct LoopState {
@@ -169,10 +105,6 @@ struct LoopBroadcast {
     double a_apply, b_apply, a_dir;
     int32_t it, active, parity;
 };
-
-__device__ __forceinline__ bool published(double v) {
-    return __builtin_bit_cast(uint64_t, v) != PART_EMPTY;
-}
 
 // max |gamma - P(gamma - s g)| over a thread's owned steps (the natural KKT residual)
 template <typename S, typename C, int K, int CH, typename Exch>
@@ -466,10 +398,8 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
                 const int nb = side == 0 ? wg - 1 : wg + 1;
                 if (nb < 0 || nb >= nwg) continue;
                 const double *src = ex_edges + ((int64_t)nb * 2 + (side ^ 1)) * EDGE + r;
-                double v = load_coherent(src);
-                for (int n = 0; !published(v) && n < LOOP_SPIN_LIMIT; n++) v = load_coherent(src);
-                if (!published(v)) A.flags[1] = 1;
-                edge(par ^ 1, side == 0 ? -1 : ntl, side ^ 1)[r] = S(v);
+                edge(par ^ 1, side == 0 ? -1 : ntl, side ^ 1)[r] =
+                    S(await_value(src, A.flags + 1));
             }
         }
         lds_barrier();
@@ -503,12 +433,8 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
             for (int w = 0; w < NW; w++) kkt = nan_max(kkt, red[4][w]);
             if (lane == 0) store_coherent(ex + wg, kkt);
             if (wg == 0) {
-                for (int j = lane; j < nwg; j += WAVE) {
-                    double v = load_coherent(ex + j);
-                    for (int n = 0; !published(v) && n < LOOP_SPIN_LIMIT; n++) v = load_coherent(ex + j);
-                    if (!published(v)) A.flags[1] = 1;
-                    kkt = nan_max(kkt, v);
-                }
+                for (int j = lane; j < nwg; j += WAVE)
+                    kkt = nan_max(kkt, await_value(ex + j, A.flags + 1));
                 st.kkt = wave_max_all(kkt);
             }
         }

@@ -207,6 +207,8 @@ int engine_eval_raw(Engine &e, int inst, double *fx, double *kkt, double *nb2);
 // after a change of h_desc: the device copy follows at once (batches) or with the next solve
 int engine_update_desc(Engine &e);
 int engine_theta_update(Engine &e, int inst, double *theta_out);
+// the engine's scratch buffer, grown to `bytes` (any earlier content may be lost)
+int engine_scratch(Engine &e, size_t bytes, void **p);
 int engine_labels(Engine &e, int inst, int32_t *labels);
 int engine_abserr(Engine &e, int inst, const double *solution, double *abserr);
 int engine_adjoint(Engine &e, int inst, const uint8_t *mask, double cg_tol, int cg_maxit,
