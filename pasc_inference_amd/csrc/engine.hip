@@ -1078,87 +1078,8 @@ static const void *cur_gamma(Engine &e, int inst, bool &f32) {
     return e.d_gamma[par];
 }
 
-template <int K>
-static void launch_eval(Engine &e, const InstDesc &d, const void *g, bool f32, double *part,
-                        int blocks) {
-    hipStream_t s = S_(e);
-    // the 1-D time graph of this instance, or the engine's graph
-    const GraphGeo G = e.stencil == STENCIL_TIME ? GraphGeo{d.T, 1, 0, nullptr, nullptr} : e.geo;
-    if (f32)
-        hipLaunchKernelGGL((eval_kernel<float, K>), dim3(blocks), dim3(256), 0, s,
-                           (const float *)g + d.goff, (const double *)e.d_x64, d, G, part);
-    else
-        hipLaunchKernelGGL((eval_kernel<double, K>), dim3(blocks), dim3(256), 0, s,
-                           (const double *)g + d.goff, (const double *)e.d_x64, d, G, part);
-}
-
-int engine_eval_raw(Engine &e, int inst, double *fx, double *kkt, double *nb2) {
-    const InstDesc &d = e.h_desc[inst];
-    bool f32;
-    const void *g = cur_gamma(e, inst, f32);
-    const int blocks = (int)((d.T + 255) / 256);
-    void *part;
-    int rc = engine_scratch(e, sizeof(double) * 3 * (size_t)blocks, &part);
-    if (rc) return rc;
-    switch (d.K) {
-        case 1: launch_eval<1>(e, d, g, f32, (double *)part, blocks); break;
-        case 2: launch_eval<2>(e, d, g, f32, (double *)part, blocks); break;
-        case 3: launch_eval<3>(e, d, g, f32, (double *)part, blocks); break;
-        case 4: launch_eval<4>(e, d, g, f32, (double *)part, blocks); break;
-        case 5: launch_eval<5>(e, d, g, f32, (double *)part, blocks); break;
-        case 6: launch_eval<6>(e, d, g, f32, (double *)part, blocks); break;
-        case 7: launch_eval<7>(e, d, g, f32, (double *)part, blocks); break;
-        case 8: launch_eval<8>(e, d, g, f32, (double *)part, blocks); break;
-        default: return fail(PASC_ERR_ARG, "unsupported K");
-    }
-    HIP_TRY(hipGetLastError());
-    std::vector<double> h(3 * (size_t)blocks);
-    HIP_TRY(hipMemcpyAsync(h.data(), part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, S_(e)));
-    HIP_TRY(hipStreamSynchronize(S_(e)));
-    double f = 0, n2 = 0, k = 0;
-    for (int b = 0; b < blocks; b++) {
-        f += h[3 * b];
-        n2 += h[3 * b + 1];
-        const double m = h[3 * b + 2];
-        if (m > k || m != m) k = m;
-    }
-    if (fx) *fx = f;
-    if (kkt) *kkt = k;
-    if (nb2) *nb2 = n2;
-    return PASC_OK;
-}
-
 int engine_eval(Engine &e, int inst, double *fx, double *kkt) {
     return engine_eval_raw(e, inst, fx, kkt, nullptr);
-}
-
-int rows_theta(Engine &e, const void *g, bool f32, const InstDesc &d, const double *x,
-               double *theta_out) {
-    const int blocks = (int)((d.T + 255) / 256);
-    const int nv = d.K * (1 + d.xdim);
-    void *part;
-    int rc = engine_scratch(e, sizeof(double) * (size_t)nv * blocks, &part);
-    if (rc) return rc;
-    if (f32)
-        hipLaunchKernelGGL((theta_partials<float>), dim3(blocks), dim3(256), 0, S_(e),
-                           (const float *)g, x, d, (double *)part);
-    else
-        hipLaunchKernelGGL((theta_partials<double>), dim3(blocks), dim3(256), 0, S_(e),
-                           (const double *)g, x, d, (double *)part);
-    HIP_TRY(hipGetLastError());
-    std::vector<double> h((size_t)nv * blocks);
-    HIP_TRY(hipMemcpyAsync(h.data(), part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, S_(e)));
-    HIP_TRY(hipStreamSynchronize(S_(e)));
-    std::vector<double> tot(nv, 0.0);
-    for (int b = 0; b < blocks; b++)
-        for (int v = 0; v < nv; v++) tot[v] += h[(size_t)b * nv + v];
-    // graphh1fem.cpp:374-379: theta_k = <x, gamma_k> / sum(gamma_k), 0 if the sum is 0
-    for (int k = 0; k < d.K; k++)
-        for (int c = 0; c < d.xdim; c++) {
-            const double gs = tot[k];
-            theta_out[k * d.xdim + c] = gs != 0 ? tot[d.K + k * d.xdim + c] / gs : 0.0;
-        }
-    return PASC_OK;
 }
 
 int engine_theta_update(Engine &e, int inst, double *theta_out) {
@@ -1195,32 +1116,6 @@ int engine_labels(Engine &e, int inst, int32_t *labels) {
     bool f32;
     const void *g = cur_gamma(e, inst, f32);
     return rows_labels(e, (const char *)g + (f32 ? 4 : 8) * d.goff, f32, d, labels);
-}
-
-int rows_abserr(Engine &e, const void *g, bool f32, const InstDesc &d, const double *solution,
-                double *abserr) {
-    const int blocks = (int)((d.T + 255) / 256);
-    void *buf;
-    const size_t need = sizeof(double) * ((size_t)d.T + blocks);
-    int rc = engine_scratch(e, need, &buf);
-    if (rc) return rc;
-    double *sol = (double *)buf;
-    double *part = sol + d.T;
-    HIP_TRY(hipMemcpyAsync(sol, solution, sizeof(double) * d.T, hipMemcpyHostToDevice, S_(e)));
-    if (f32)
-        hipLaunchKernelGGL((abserr_kernel<float>), dim3(blocks), dim3(256), 0, S_(e),
-                           (const float *)g, d, (const double *)sol, part);
-    else
-        hipLaunchKernelGGL((abserr_kernel<double>), dim3(blocks), dim3(256), 0, S_(e),
-                           (const double *)g, d, (const double *)sol, part);
-    HIP_TRY(hipGetLastError());
-    std::vector<double> h(blocks);
-    HIP_TRY(hipMemcpyAsync(h.data(), part, sizeof(double) * blocks, hipMemcpyDeviceToHost, S_(e)));
-    HIP_TRY(hipStreamSynchronize(S_(e)));
-    double a = 0;
-    for (double v : h) a += v;
-    *abserr = a;
-    return PASC_OK;
 }
 
 int engine_abserr(Engine &e, int inst, const double *solution, double *abserr) {

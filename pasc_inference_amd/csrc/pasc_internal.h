@@ -250,6 +250,14 @@ using PieceLaunch = std::function<void(struct ihipStream_t *, int64_t, int64_t, 
 int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t total,
                     const PieceLaunch &launch);
 
+// elements of one piece of such a transfer (the last one may be shorter)
+int64_t staged_piece(size_t esize, int64_t total);
+
+// readout.hip: the theta step with its partials at `part` (READ_BLOCKS * K (1 + xdim) doubles)
+constexpr int READ_BLOCKS = 1024;
+int theta_from_rows(Engine &e, const void *g, bool f32, const InstDesc &d, const double *x,
+                    double *part, double *theta_out);
+
 // noalloc.hip: the theta step with its partial sums in a static device array
 int noalloc_init(int device);  // once per device, with the device current
 int64_t noalloc_theta_max_T(int K, int xdim);

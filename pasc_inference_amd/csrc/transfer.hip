@@ -187,6 +187,17 @@ struct Transfer {
     }
 };
 
+static int staging_threads() {
+    return std::min(SLOTS, std::max(1, (int)std::thread::hardware_concurrency() / 2));
+}
+
+int64_t staged_piece(size_t esize, int64_t total) {
+    const int64_t slot = (int64_t)(SLOT_BYTES / esize), page = (int64_t)(STAGING_PIECE_MIN / esize);
+    if ((size_t)total * esize <= STAGING_SINGLE) return slot;
+    const int64_t share = (total + staging_threads() - 1) / staging_threads();
+    return std::min(slot, (share + page - 1) / page * page);
+}
+
 int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t total,
                     const PieceLaunch &launch) {
     if (total <= 0) return PASC_OK;
@@ -198,15 +209,10 @@ int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t to
     t.esize = esize;
     t.total = total;
     t.launch = &launch;
-    const int64_t slot = (int64_t)(SLOT_BYTES / esize), page = (int64_t)(STAGING_PIECE_MIN / esize);
-    const int most = std::min(SLOTS, std::max(1, (int)std::thread::hardware_concurrency() / 2));
-    t.piece = slot;
+    t.piece = staged_piece(esize, total);
     int helpers = 0;
-    if ((size_t)total * esize > STAGING_SINGLE) {
-        const int64_t share = (total + most - 1) / most;
-        t.piece = std::min(slot, (share + page - 1) / page * page);
-        helpers = (int)std::min<int64_t>(most, (total + t.piece - 1) / t.piece) - 1;
-    }
+    if ((size_t)total * esize > STAGING_SINGLE)
+        helpers = (int)std::min<int64_t>(staging_threads(), (total + t.piece - 1) / t.piece) - 1;
     std::vector<std::thread> th;
     try {
         th.reserve(helpers);

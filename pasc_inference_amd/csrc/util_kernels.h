@@ -1,5 +1,5 @@
 // Auxiliary kernels: stand-alone projection and matvec (the kernel-level C-ABI entry points),
-// explicit FP64 objective/KKT evaluation, the theta update, labels, abserr and conversions.
+// labels, fills and conversions.
 #pragma once
 
 #include "device_common.h"
@@ -105,111 +105,7 @@ __global__ __launch_bounds__(256) void matvec_graph(const S *x, S *y, GraphGeo G
     y[k * ld + n] = S(alpha * a);
 }
 
-// ---- explicit FP64 evaluation of f = 1/2 g'Ag - b'g, the KKT residual and ||b||^2 -----------
-// Partials per block: [0] f, [1] ||b||^2, [2] kkt (max).
-template <typename S, int K>
-__global__ __launch_bounds__(256) void eval_kernel(const S *gam, const double *x,
-                                                   InstDesc D, GraphGeo G, double *part) {
-    __shared__ double lds[3 * 4];
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t T = D.T;
-    double f = 0.0, nb2 = 0.0, kkt = 0.0;
-    if (t < T) {
-        double g0[K], lap[K], q[K];
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            g0[k] = (double)gam[k * D.ld + t];
-            lap[k] = 0.0;
-            q[k] = 0.0;
-        }
-        for_neighbours(G, t, [&](int64_t n2, double w) {
-#pragma unroll
-            for (int k = 0; k < K; k++) lap[k] += w * (g0[k] - (double)gam[k * D.ld + n2]);
-        });
-        if (D.b64) {
-#pragma unroll
-            for (int k = 0; k < K; k++) q[k] = -D.b64[k * D.ld + t];
-        } else if (!(D.heldout && D.heldout[t])) {
-            for (int c = 0; c < D.xdim; c++) {
-                const double xc = x[D.xoff + c * D.ld + t];
-#pragma unroll
-                for (int k = 0; k < K; k++) {
-                    const double dx = xc - D.theta[k * D.xdim + c];
-                    q[k] += dx * dx;
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < K; k++) q[k] *= D.bscale;
-        }
-        double z[K];
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const double g = D.alpha * lap[k] + q[k];
-            f += 0.5 * D.alpha * lap[k] * g0[k] + q[k] * g0[k];
-            nb2 += q[k] * q[k];
-            z[k] = g0[k] - D.s_kkt * g;
-        }
-        project_simplex<K, double>(z);
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const double e = fabs(g0[k] - z[k]);
-            kkt = (e > kkt || e != e) ? e : kkt;
-        }
-    }
-    f = wave_sum(f);
-    nb2 = wave_sum(nb2);
-    kkt = wave_max(kkt);
-    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-    if (lane == 0) {
-        lds[w * 3 + 0] = f;
-        lds[w * 3 + 1] = nb2;
-        lds[w * 3 + 2] = kkt;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q2 = 1; q2 < 4; q2++) {
-            f += lds[q2 * 3 + 0];
-            nb2 += lds[q2 * 3 + 1];
-            const double m = lds[q2 * 3 + 2];
-            kkt = (m > kkt || m != m) ? m : kkt;
-        }
-        part[blockIdx.x * 3 + 0] = f;
-        part[blockIdx.x * 3 + 1] = nb2;
-        part[blockIdx.x * 3 + 2] = kkt;
-    }
-}
-
-// ---- theta update partials: per block sum_t gamma_k and sum_t x_c gamma_k (FP64) -------------
-// part layout per block: [k] sums for k < K, then [K + k*xdim + c].
-template <typename S>
-__global__ __launch_bounds__(256) void theta_partials(const S *gam, const double *x, InstDesc D,
-                                                      double *part) {
-    const int K = D.K, xd = D.xdim;
-    const int nv = K * (1 + xd);
-    __shared__ double lds[PASC_MAX_K * 4 * 4];
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-    for (int v = 0; v < nv; v++) {
-        double a = 0.0;
-        if (t < D.T && !(D.heldout && D.heldout[t])) {
-            if (v < K) {
-                a = (double)gam[v * D.ld + t];
-            } else {
-                const int k = (v - K) / xd, c = (v - K) % xd;
-                a = x[D.xoff + c * D.ld + t] * (double)gam[k * D.ld + t];
-            }
-        }
-        a = wave_sum(a);
-        if (lane == 0) lds[v * 4 + w] = a;
-    }
-    __syncthreads();
-    if (threadIdx.x < nv) {
-        const int v = threadIdx.x;
-        part[(int64_t)blockIdx.x * nv + v] = lds[v * 4 + 0] + lds[v * 4 + 1] + lds[v * 4 + 2] + lds[v * 4 + 3];
-    }
-}
-
-// ---- labels (argmax over k, lowest k on ties) and |sum_k theta_k gamma_k - sol| partials -----
+// ---- labels (argmax over k, lowest k on ties) -------------------------------------------------
 template <typename S>
 __global__ __launch_bounds__(256) void labels_kernel(const S *gam, int64_t n, int64_t ld, int K,
                                                      int32_t *lab) {
@@ -222,23 +118,6 @@ __global__ __launch_bounds__(256) void labels_kernel(const S *gam, int64_t n, in
         if (v > bv) { bv = v; best = k; }
     }
     lab[t] = best;
-}
-
-template <typename S>
-__global__ __launch_bounds__(256) void abserr_kernel(const S *gam, InstDesc D, const double *sol,
-                                                     double *part) {
-    __shared__ double lds[4];
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    double a = 0.0;
-    if (t < D.T) {
-        double rec = -sol[t];
-        for (int k = 0; k < D.K; k++) rec += D.theta[k] * (double)gam[k * D.ld + t];
-        a = fabs(rec);
-    }
-    a = wave_sum(a);
-    if ((threadIdx.x & (WAVE - 1)) == 0) lds[threadIdx.x / WAVE] = a;
-    __syncthreads();
-    if (threadIdx.x == 0) part[blockIdx.x] = lds[0] + lds[1] + lds[2] + lds[3];
 }
 
 // ---- element-wise conversion (FP32 state -> FP64 polish state) ------------------------------
