@@ -240,8 +240,7 @@ int pasc_get_labels(pasc_problem *p, int32_t *labels);
 /* ---- kernel-level entry points on caller-owned device memory ----
  * SimplexFeasibleSet_Local<PetscVector>::project (simplex_local.cpp:37-65, kernel_project
  * simplex_local.cu:70-139): project every K-block (t-major: K consecutive values; k-major:
- * stride ld between the K values) of x in place.  K <= 32 uses one thread per block; larger K
- * uses one wavefront per block. */
+ * stride ld between the K values) of x in place. */
 int pasc_project_simplex(pasc_ctx *ctx, void *x_dev, int64_t nblocks, int32_t K, int dtype,
                          int layout, int64_t ld);
 /* BlockGraphSparseMatrix<PetscVector>::matmult (blockgraphsparse.cpp:151-194): y = alpha*A0*x

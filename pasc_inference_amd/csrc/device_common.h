@@ -55,6 +55,31 @@ __device__ __forceinline__ void store_nt(double2 *p, const double2 &v) {
     __builtin_nontemporal_store(n, reinterpret_cast<nt_double2 *>(p));
 }
 
+// Whole-wave lane shifts by one lane (DPP wave_shr:1 / wave_shl:1, VALU moves): lane i gets
+// lane i-1 (from_left) or lane i+1 (from_right); the lane without a source gets 0 (the
+// bound-control bit: no register has to be set to 0 before each move).
+template <int CTRL>
+__device__ __forceinline__ float dpp_shift(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift(double v) {
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(u & 0xffffffffll), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)(unsigned)hi << 32) | (long long)(unsigned)lo);
+}
+constexpr int DPP_WAVE_SHR1 = 0x138;  // lane i <- lane i-1
+constexpr int DPP_WAVE_SHL1 = 0x130;  // lane i <- lane i+1
+
+// the value a lane holds, in every lane
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)u, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
+    return __longlong_as_double(((long long)(unsigned)hi << 32) | (long long)(unsigned)lo);
+}
+
 // max via the hardware min/max instructions (one VALU op instead of a compare and a select)
 __device__ inline float cmax(float a, float b) { return __builtin_fmaxf(a, b); }
 __device__ inline double cmax(double a, double b) { return __builtin_fmax(a, b); }

@@ -13,6 +13,7 @@
 
 #include "img_kernels.h"
 #include "loop_kernels.h"
+#include "project_kernels.h"
 #include "spg_kernels.h"
 #include "step_kernels.h"
 #include "util_kernels.h"
@@ -1475,8 +1476,7 @@ static int project_dispatch(Ctx *ctx, S *x, int64_t nb, int K, int layout, int64
 #undef PCASE
         }
     } else {
-        const unsigned blocks = (unsigned)((nb + 3) / 4);
-        hipLaunchKernelGGL((project_wave<S>), dim3(blocks), dim3(256), 0, s, x, nb, K, layout, ld);
+        launch_project_many<S>(x, nb, K, layout == PASC_LAYOUT_TMAJOR, ld, s);
     }
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
@@ -1495,8 +1495,19 @@ int kernel_matvec(Ctx *ctx, const void *x, void *y, int64_t T, int64_t R, int K,
     hipStream_t s = (hipStream_t)ctx->stream;
     const int64_t n = T * R;
     if (n == 0) return PASC_OK;
-    const dim3 grid((unsigned)((n + 255) / 256), (unsigned)K);
-    if (R == 1 && grid_width == 0 && !nbr_ptr_dev) {
+    dim3 grid((unsigned)((n + 255) / 256), (unsigned)K);
+    // the image kernel's columns are 64 lanes wide: narrower images run the general walk
+    const bool image = T == 1 && grid_width >= 48 && !nbr_ptr_dev && R / grid_width < (int64_t)65535 * 4 * MV_ROWS;
+    if (image && K <= 65535) {
+        const int32_t H = (int32_t)(R / grid_width);
+        grid = dim3((unsigned)((grid_width + 63) / 64), (unsigned)((H + 4 * MV_ROWS - 1) / (4 * MV_ROWS)),
+                    (unsigned)K);
+        if (dtype == PASC_DTYPE_F32)
+            hipLaunchKernelGGL((matvec_image<float>), grid, dim3(256), 0, s, (const float *)x, (float *)y, grid_width, H, ld, alpha);
+        else
+            hipLaunchKernelGGL((matvec_image<double>), grid, dim3(256), 0, s, (const double *)x, (double *)y, grid_width, H, ld, alpha);
+    } else if (R == 1 && grid_width == 0 && !nbr_ptr_dev) {
+        grid.x = (unsigned)((n + 256 * MV_SEG - 1) / (256 * MV_SEG));
         if (dtype == PASC_DTYPE_F32)
             hipLaunchKernelGGL((matvec_time<float>), grid, dim3(256), 0, s, (const float *)x, (float *)y, T, K, ld, alpha);
         else

@@ -22,12 +22,6 @@ __device__ __forceinline__ double dpp_from(double v) {
     const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, true);
     return __longlong_as_double(((long long)(unsigned)hi << 32) | (long long)(unsigned)lo);
 }
-__device__ __forceinline__ double from_lane(double v, int lane) {
-    const long long u = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)u, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
-    return __longlong_as_double(((long long)(unsigned)hi << 32) | (long long)(unsigned)lo);
-}
 __device__ __forceinline__ double join_words(unsigned lo, unsigned hi) {
     return __longlong_as_double(((long long)hi << 32) | (long long)lo);
 }
@@ -68,8 +62,8 @@ __device__ __forceinline__ double wave_max_all(double v) {
     v = nan_max(v, dpp_from<DPP_ROR + 4>(v));
     v = nan_max(v, dpp_from<DPP_ROR + 2>(v));
     v = nan_max(v, dpp_from<DPP_ROR + 1>(v));
-    return nan_max(nan_max(from_lane(v, 0), from_lane(v, 16)),
-                   nan_max(from_lane(v, 32), from_lane(v, 48)));
+    return nan_max(nan_max(lane_value(v, 0), lane_value(v, 16)),
+                   nan_max(lane_value(v, 32), lane_value(v, 48)));
 }
 
 // sum over the wave, in every lane
@@ -78,7 +72,7 @@ __device__ __forceinline__ double wave_sum_all(double v) {
     v += dpp_from<DPP_ROR + 4>(v);
     v += dpp_from<DPP_ROR + 2>(v);
     v += dpp_from<DPP_ROR + 1>(v);
-    return (from_lane(v, 0) + from_lane(v, 16)) + (from_lane(v, 32) + from_lane(v, 48));
+    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
 __device__ __forceinline__ bool published(double v) {

@@ -376,10 +376,10 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
                 }
             }
             const double tot = wave_sum4(v[0], v[1], v[2], v[3]);
-            v[0] = from_lane(tot, ROW_A);
-            v[1] = 2.0 * (double)cx.alpha * from_lane(tot, ROW_B);
-            v[2] = -from_lane(tot, ROW_C) / (double)cx.a_dir;
-            v[3] = 0.5 * from_lane(tot, ROW_D);
+            v[0] = lane_value(tot, ROW_A);
+            v[1] = 2.0 * (double)cx.alpha * lane_value(tot, ROW_B);
+            v[2] = -lane_value(tot, ROW_C) / (double)cx.a_dir;
+            v[3] = 0.5 * lane_value(tot, ROW_D);
             v[4] = cx.want_kkt ? wave_max_all(v[4]) : -1.0;  // -1: not evaluated on this pass
             step_core(sample_eps, st, win, v, A.p.sp);
             if (lane == 0) {

@@ -24,72 +24,72 @@ __global__ __launch_bounds__(256) void project_thread(S *x, int64_t nblocks, int
     }
 }
 
-// ---- stand-alone projection, large K: one wavefront per block ------------------------------
-// Lanes hold the entries k = lane + 64*i.  The threshold is bracketed in [max-1, max) and
-// bisected (wave-wide sums), then finished exactly by the support fixed point.
-template <typename S>
-__global__ __launch_bounds__(256) void project_wave(S *x, int64_t nblocks, int K, int layout,
-                                                    int64_t ld) {
-    const int64_t b = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int lane = threadIdx.x & (WAVE - 1);
-    if (b >= nblocks) return;
-    auto at = [&](int k) -> int64_t { return layout == 0 ? b * K + k : (int64_t)k * ld + b; };
-    double s = 0.0, mx = -1e308;
-    int neg = 0;
-    for (int k = lane; k < K; k += WAVE) {
-        const double v = (double)x[at(k)];
-        s += v;
-        neg |= v < 0.0;
-        mx = v > mx ? v : mx;
-    }
-    s = wave_sum(s);
-    neg = wave_sum_i(neg);
-    mx = wave_max(mx);
-    if (neg == 0 && s == 1.0) return;
-    double lo = mx - 1.0, hi = mx;
-    for (int it = 0; it < 24; it++) {
-        const double mid = 0.5 * (lo + hi);
-        double phi = 0.0;
-        for (int k = lane; k < K; k += WAVE) {
-            const double v = (double)x[at(k)] - mid;
-            phi += v > 0.0 ? v : 0.0;
-        }
-        phi = wave_sum(phi) - 1.0;
-        if (phi >= 0.0) lo = mid; else hi = mid;
-    }
-    double tau = lo;
-    int cnt_prev = -1;
-    for (int it = 0; it < K; it++) {
-        double sum = 0.0;
-        int cnt = 0;
-        for (int k = lane; k < K; k += WAVE) {
-            const double v = (double)x[at(k)];
-            if (v > tau) { sum += v; cnt++; }
-        }
-        sum = wave_sum(sum);
-        cnt = wave_sum_i(cnt);
-        if (cnt == cnt_prev || cnt == 0) break;
-        cnt_prev = cnt;
-        tau = (sum - 1.0) / (double)cnt;
-    }
-    for (int k = lane; k < K; k += WAVE) {
-        const double v = (double)x[at(k)] - tau;
-        x[at(k)] = S(v > 0.0 ? v : 0.0);
-    }
-}
-
 // ---- stand-alone matvec y = alpha*A0*x (k-major rows of stride ld) --------------------------
+// Time graph: a wave covers MV_SEG segments of 64 consecutive steps, all loaded before any is used;
+// the neighbours come from the adjacent lanes and segments, so a step is loaded once per wave
+// (rows of any stride and alignment: 8- or 4-byte loads).  One step a thread with three loads
+// each took 23.8 us for 2 million steps of 3 rows in FP64 (96 MB).
+constexpr int MV_SEG = 4;
 template <typename S>
 __global__ __launch_bounds__(256) void matvec_time(const S *x, S *y, int64_t T, int K,
                                                    int64_t ld, double alpha) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int64_t t0 = (((int64_t)blockIdx.x * 256 + threadIdx.x) / WAVE) * (WAVE * MV_SEG);
     const int k = blockIdx.y;
-    if (t >= T || k >= K) return;
+    if (t0 >= T) return;
     const S *r = x + k * ld;
-    double a = 0.0;
-    if (t > 0) a += 2.0 * ((double)r[t] - (double)r[t - 1]);
-    if (t < T - 1) a += 2.0 * ((double)r[t] - (double)r[t + 1]);
-    y[k * ld + t] = S(alpha * a);
+    double v[MV_SEG], before = 0.0, after = 0.0;
+#pragma unroll
+    for (int j = 0; j < MV_SEG; j++) {
+        const int64_t t = t0 + j * WAVE + lane;
+        v[j] = t < T ? (double)r[t] : 0.0;
+    }
+    if (lane == 0 && t0 > 0) before = (double)r[t0 - 1];
+    if (lane == WAVE - 1 && t0 + WAVE * MV_SEG < T) after = (double)r[t0 + WAVE * MV_SEG];
+#pragma unroll
+    for (int j = 0; j < MV_SEG; j++) {
+        const int64_t t = t0 + j * WAVE + lane;
+        // the lane before and after, at the segment's ends the neighbouring segment's end
+        double left = dpp_shift<DPP_WAVE_SHR1>(v[j]), right = dpp_shift<DPP_WAVE_SHL1>(v[j]);
+        const double lastl = j > 0 ? lane_value(v[j > 0 ? j - 1 : 0], WAVE - 1) : before;
+        const double firstr = j < MV_SEG - 1 ? lane_value(v[j < MV_SEG - 1 ? j + 1 : j], 0) : after;
+        left = lane == 0 ? lastl : left;
+        right = lane == WAVE - 1 ? firstr : right;
+        double a = 0.0;
+        if (t > 0) a += 2.0 * (v[j] - left);
+        if (t < T - 1) a += 2.0 * (v[j] - right);
+        if (t < T) y[k * ld + t] = S(alpha * a);
+    }
+}
+
+// Image (T = 1 on the 4-neighbour grid): a thread walks MV_ROWS rows of its column with the rows
+// above and below in registers; the sum's order (up, left, right, down) is the general walk's.
+constexpr int MV_ROWS = 8;
+template <typename S>
+__global__ __launch_bounds__(256) void matvec_image(const S *x, S *y, int32_t W, int32_t H,
+                                                    int64_t ld, double alpha) {
+    const int col = blockIdx.x * 64 + (threadIdx.x & 63);
+    const int r0 = (blockIdx.y * 4 + threadIdx.x / 64) * MV_ROWS;
+    if (col >= W || r0 >= H) return;
+    const S *v = x + blockIdx.z * ld;
+    S *o = y + blockIdx.z * ld;
+    const int64_t n0 = (int64_t)r0 * W + col;
+    double up = r0 > 0 ? (double)v[n0 - W] : 0.0, c = (double)v[n0];
+#pragma unroll
+    for (int j = 0; j < MV_ROWS; j++) {
+        const int r = r0 + j;
+        if (r >= H) break;
+        const int64_t n = n0 + (int64_t)j * W;
+        const double dn = r + 1 < H ? (double)v[n + W] : 0.0;
+        double a = 0.0;
+        if (r > 0) a += c - up;
+        if (col > 0) a += c - (double)v[n - 1];
+        if (col < W - 1) a += c - (double)v[n + 1];
+        if (r + 1 < H) a += c - dn;
+        o[n] = S(alpha * a);
+        up = c;
+        c = dn;
+    }
 }
 
 template <typename S>
