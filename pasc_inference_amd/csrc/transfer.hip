@@ -8,16 +8,18 @@
 // pieces from and to the caller's pages.  240 MB (T = 1e7, K = 3) took 86 ms down and 73 ms up
 // when one host thread did the layout around a pageable copy; in 4 MiB pieces over 8 threads it
 // takes 5 ms, of which the link needs 4.3.  One thread would be bound by its page faults and
-// copies (23 ms), so transfers of 1 MiB and more are cut into up to 8 pieces at a time.
+// copies (23 ms).  Up to one piece, a single kernel moves the whole transfer and the threads share
+// the host copy (1.4 MB into fresh pages: 150 us by one thread, 75 by several).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <deque>
+#include <memory>
 #include <functional>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -71,8 +73,7 @@ struct Slot {
 constexpr int SLOTS = 8;
 constexpr size_t SLOT_BYTES = (size_t)4 << 20;
 constexpr int POOL_DEVICES = 64;
-constexpr size_t STAGING_SINGLE = (size_t)1 << 20;      // up to here one thread is as fast
-constexpr size_t STAGING_PIECE_MIN = (size_t)256 << 10;  // pieces are multiples of this
+constexpr size_t COPY_PIECE = (size_t)128 << 10;  // share of a host copy worth another thread
 
 struct SlotPool {
     std::mutex mu;
@@ -116,12 +117,97 @@ struct SlotPool {
     }
 };
 
-static SlotPool g_pool[POOL_DEVICES];
+static SlotPool *const g_pool = new SlotPool[POOL_DEVICES];
+
+// Helper threads of the host copies, parked between transfers; started when first needed, ended
+// with the process's last context.
+class Team {
+    struct Job {
+        const std::function<void()> *fn = nullptr;
+        int running = 0;
+        bool closed = false;
+    };
+    std::mutex mu;
+    std::condition_variable wake, done;
+    std::deque<std::shared_ptr<Job>> queue;
+    std::vector<std::thread> threads;
+    int users = 0;
+    bool stop = false;
+
+    void loop() {
+        std::unique_lock<std::mutex> lk(mu);
+        for (;;) {
+            wake.wait(lk, [&] { return stop || !queue.empty(); });
+            if (stop) return;
+            std::shared_ptr<Job> j = queue.front();
+            queue.pop_front();
+            if (j->closed) continue;
+            j->running++;
+            lk.unlock();
+            (*j->fn)();
+            lk.lock();
+            if (--j->running == 0) done.notify_all();
+        }
+    }
+
+  public:
+    static constexpr int MOST = SLOTS - 1;
+
+    static int helpers() {
+        return std::min(MOST, std::max(1, (int)std::thread::hardware_concurrency() / 2) - 1);
+    }
+    void open() {
+        std::lock_guard<std::mutex> lk(mu);
+        users++;
+    }
+    void close() {
+        std::vector<std::thread> gone;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            if (--users > 0) return;
+            stop = true;
+            gone.swap(threads);
+        }
+        wake.notify_all();
+        for (auto &t : gone) t.join();
+        std::lock_guard<std::mutex> lk(mu);
+        stop = false;
+    }
+    // fn on this thread and on up to n helpers; back when every helper that started has ended.
+    // fn must not throw.
+    void run(int n, const std::function<void()> &fn) {
+        std::shared_ptr<Job> job;
+        if (n > 0) {
+            try {
+                job = std::make_shared<Job>();
+                job->fn = &fn;
+                std::lock_guard<std::mutex> lk(mu);
+                while ((int)threads.size() < std::min(n, helpers()) && !stop)
+                    threads.emplace_back([this] { loop(); });
+                for (int i = 0; i < n; i++) queue.push_back(job);
+            } catch (const std::exception &) {
+                // fewer helpers: this thread does the rest
+            }
+            if (n == 1) wake.notify_one();
+            else wake.notify_all();
+        }
+        fn();
+        if (job) {
+            std::unique_lock<std::mutex> lk(mu);
+            job->closed = true;
+            done.wait(lk, [&] { return job->running == 0; });
+        }
+    }
+};
+
+// never destroyed: parked threads end with the process when a context is still open then
+static Team &g_team = *new Team;
 
 int staging_open(int device) {
     if (device < 0 || device >= POOL_DEVICES)
         return fail(PASC_ERR_ARG, "staging: device %d beyond %d", device, POOL_DEVICES);
     SlotPool &p = g_pool[device];
+    g_team.open();
     std::lock_guard<std::mutex> lk(p.mu);
     p.idle.reserve(SLOTS);
     p.users++;
@@ -130,6 +216,7 @@ int staging_open(int device) {
 
 void staging_close(int device) {
     if (device < 0 || device >= POOL_DEVICES) return;
+    g_team.close();
     SlotPool &p = g_pool[device];
     std::lock_guard<std::mutex> lk(p.mu);
     if (--p.users > 0) return;
@@ -141,32 +228,54 @@ void staging_close(int device) {
     p.idle.clear();
 }
 
+// memcpy by several threads
+static void team_copy(void *dst, const void *src, size_t bytes) {
+    const int n = (int)std::min<size_t>((size_t)Team::helpers(), bytes / COPY_PIECE);
+    if (n < 1) {
+        std::memcpy(dst, src, bytes);
+        return;
+    }
+    const size_t share = (bytes / (n + 1) + 4095) / 4096 * 4096;
+    std::atomic<size_t> next{0};
+    g_team.run(n, [&]() {
+        for (size_t i = next.fetch_add(share); i < bytes; i = next.fetch_add(share))
+            std::memcpy((char *)dst + i, (const char *)src + i, std::min(share, bytes - i));
+    });
+}
+
 // One transfer: pieces of `piece` elements, taken in turn by the calling thread and its helpers.
 struct Transfer {
     int device;
     hipStream_t stream;
-    bool to_host;
+    bool to_host, single;
     char *host;
     size_t esize;
     int64_t total, piece;
     const PieceLaunch *launch;
     std::atomic<int64_t> next{0};
     std::atomic<int> error{(int)hipSuccess};
+    std::atomic<bool> caller{true};
+
+    void copy(void *dst, const void *src, size_t bytes) {
+        if (single) team_copy(dst, src, bytes);
+        else std::memcpy(dst, src, bytes);
+    }
 
     hipError_t one(const Slot &s, int64_t i0, int64_t n) {
-        if (!to_host) std::memcpy(s.p, host + (size_t)i0 * esize, (size_t)n * esize);
+        if (!to_host) copy(s.p, host + (size_t)i0 * esize, (size_t)n * esize);
         (*launch)(stream, i0, n, s.p);
         hipError_t e;
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if ((e = hipEventRecord(s.ev, stream)) != hipSuccess) return e;
         if ((e = hipEventSynchronize(s.ev)) != hipSuccess) return e;
-        if (to_host) std::memcpy(host + (size_t)i0 * esize, s.p, (size_t)n * esize);
+        if (to_host) copy(host + (size_t)i0 * esize, s.p, (size_t)n * esize);
         return hipSuccess;
     }
 
-    // first: the calling thread, which waits for a slot; helpers leave when there is none
-    void work(bool first) {
-        hipError_t e = first ? hipSuccess : hipSetDevice(device);
+    // The first to come waits for a slot; the others leave when there is none.
+    void work() {
+        const bool first = caller.exchange(false);
+        hipError_t e = hipSetDevice(device);
         Slot s;
         if (e == hipSuccess) {
             e = g_pool[device].take(first, s);
@@ -187,15 +296,12 @@ struct Transfer {
     }
 };
 
-static int staging_threads() {
-    return std::min(SLOTS, std::max(1, (int)std::thread::hardware_concurrency() / 2));
-}
-
+// Whole slots, or an eighth of a transfer that would fill only a few.
 int64_t staged_piece(size_t esize, int64_t total) {
-    const int64_t slot = (int64_t)(SLOT_BYTES / esize), page = (int64_t)(STAGING_PIECE_MIN / esize);
-    if ((size_t)total * esize <= STAGING_SINGLE) return slot;
-    const int64_t share = (total + staging_threads() - 1) / staging_threads();
-    return std::min(slot, (share + page - 1) / page * page);
+    const int64_t slot = (int64_t)(SLOT_BYTES / esize);
+    if (total <= slot) return slot;
+    const int64_t unit = (int64_t)(COPY_PIECE / esize), share = (total + SLOTS - 1) / SLOTS;
+    return std::min(slot, std::max(8 * unit, (share + unit - 1) / unit * unit));
 }
 
 int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t total,
@@ -210,18 +316,9 @@ int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t to
     t.total = total;
     t.launch = &launch;
     t.piece = staged_piece(esize, total);
-    int helpers = 0;
-    if ((size_t)total * esize > STAGING_SINGLE)
-        helpers = (int)std::min<int64_t>(staging_threads(), (total + t.piece - 1) / t.piece) - 1;
-    std::vector<std::thread> th;
-    try {
-        th.reserve(helpers);
-        for (int i = 0; i < helpers; i++) th.emplace_back([&t]() { t.work(false); });
-    } catch (const std::exception &) {
-        // fewer helpers: the threads that run, this one included, do the rest
-    }
-    t.work(true);
-    for (auto &x : th) x.join();
+    t.single = total <= t.piece;
+    const int64_t pieces = (total + t.piece - 1) / t.piece;
+    g_team.run((int)std::min<int64_t>(Team::helpers(), pieces - 1), [&t]() { t.work(); });
     const hipError_t e = (hipError_t)t.error.load();
     if (e != hipSuccess)
         return fail(PASC_ERR_HIP, "%s transfer: %s", to_host ? "device to host" : "host to device",
