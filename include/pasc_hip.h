@@ -106,8 +106,9 @@ typedef struct {
     double alphainit;     /* default 2 */
     uint32_t stop_mask;   /* default PASC_STOP_DIFFF */
     double kkt_tol;       /* default 1e-6 */
-    int32_t check_every;  /* iterations between host convergence polls (default 1) */
-    int32_t use_graph;    /* capture check_every iterations in a hipGraph (default 0) */
+    int32_t check_every;  /* batches with use_graph: iterations per graph (default 1).  Otherwise not
+                             used: the host enqueues a few iterations ahead and never waits for one */
+    int32_t use_graph;    /* batches: replay graphs of check_every iterations (default 0) */
     double fp32_switch;   /* FP32-bulk: hand over to FP64 once the FP32 KKT <= this
                              (default 0 = 100 * kkt_tol; never below the level
                              1e-5 * epsilon where FP32 storage stalls SPG) */

@@ -374,7 +374,7 @@ static int run_adj_loop(Engine &e, const InstDesc &D, const double *gam, const u
     a.save_rr = ex + ow + ew * epochs;
     a.save = a.save_rr + 2;
     a.out = (double *)e.h_state;  // pinned; no solve is under way
-    a.flags = e.h_nactive;
+    a.flags = e.h_poll;
     a.ex = ex;
     a.epochs = epochs;
     a.maxit = cg_maxit;

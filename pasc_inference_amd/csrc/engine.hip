@@ -152,17 +152,21 @@ static int engine_retile(Engine &e, bool f64_phase) {
         d.ntiles = (int32_t)((raw + d.msub - 1) / d.msub);
         slots += d.ntiles;
     }
-    if (slots != e.total_slots || !e.d_part) {
+    e.total_slots = slots;
+    if (slots > e.part_slots || !e.d_part) {
         if (e.d_part) (void)hipFree(e.d_part);
         e.d_part = nullptr;
-        e.total_slots = slots;
+        e.part_slots = 0;
         HIP_TRY(hipMalloc(&e.d_part, sizeof(double) * (size_t)std::max(slots, 1) * NPART));
-        // every partial starts unpublished (the fused step's hand-over, take_published)
+        e.part_slots = std::max(slots, 1);
+        // every partial starts unpublished (the fused step's hand-over, settle_published); the
+        // fused passes leave them so, and the other paths overwrite what they read
         const int64_t nw = (int64_t)std::max(slots, 1) * NPART;
         hipLaunchKernelGGL(fill_u64, dim3((unsigned)std::min<int64_t>((nw + 255) / 256, 1024)),
                            dim3(256), 0, S_(e), (uint64_t *)e.d_part, nw, PART_EMPTY);
         HIP_TRY(hipGetLastError());
     }
+    e.tiled_scan = false;
     for (auto &g : e.groups) {
         std::vector<int32_t> ids;
         int64_t tiles = 0;
@@ -222,6 +226,16 @@ int engine_alloc(Engine &e, Ctx *ctx, int precision, int stencil, int32_t grid_w
     e.data_elems = data_elems;
     e.sh[0] = PassShape{256, 4, 0, 2048, 1};
     e.sh[1] = PassShape{256, 2, 0, 2048, 1};
+    if (e.n_inst == 1 && stencil == STENCIL_TIME) {
+        // One series beyond what the persistent loop holds: one-wave workgroups, the next tile
+        // staged.  us per pass at T = 1e7 against the shapes above: FP64 K = 2 / 3 / 4 58 / 93 /
+        // 136 (71 / 112 / 151), K = 8 (shorter chunk) 395 (443), FP32 41 / 53 / 76 / 244 (44 / 59
+        // / 82 / 273); at T = 2e6 24 / 32 / 41 / 100 (30 / 36 / 44 / 109).  The FP32 chunk stays 4:
+        // a thread's FP32 sums cover its chunk, so it fixes their rounding.
+        const bool wide = descs[0].K > 4;
+        e.sh[0] = PassShape{64, 4, 1, 4096, 1};
+        e.sh[1] = PassShape{64, wide ? 2 : 4, 1, wide ? 8192 : 4096, 1};
+    }
     if (stencil != STENCIL_TIME) {
         // graph problems (fixed shape): at most 512 partial slots per instance, i.e. each
         // workgroup walks 8 consecutive 256-node tiles of a 1024^2 image (two image rows).
@@ -249,7 +263,7 @@ int engine_alloc(Engine &e, Ctx *ctx, int precision, int stencil, int32_t grid_w
     }
     HIP_TRY(hipMalloc(&e.d_desc, sizeof(InstDesc) * std::max(e.n_inst, 1)));
     HIP_TRY(hipMalloc(&e.d_state, sizeof(InstState) * std::max(e.n_inst, 1)));
-    HIP_TRY(hipMalloc(&e.d_nactive, 2 * sizeof(int32_t)));  // [0] active count, [1] dirty flag
+    HIP_TRY(hipMalloc(&e.d_dirty, sizeof(int32_t)));
     HIP_TRY(hipMalloc(&e.d_done, DONE_BYTES));
     HIP_TRY(hipMemsetAsync(e.d_done, 0, DONE_BYTES, S_(e)));
     // the group partials after the counters start unpublished
@@ -257,9 +271,9 @@ int engine_alloc(Engine &e, Ctx *ctx, int precision, int stencil, int32_t grid_w
                        (uint64_t *)(e.d_done + DONE_WORDS), (int64_t)DONE_SUB * NPART, PART_EMPTY);
     HIP_TRY(hipGetLastError());
     // pinned poll area: [0] active instances, [1 + g] active tiles of K group g
-    HIP_TRY(hipHostMalloc((void **)&e.h_nactive, 64 + sizeof(InstState), hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **)&e.h_poll, 64 + sizeof(InstState), hipHostMallocDefault));
     static_assert(sizeof(int32_t) * (1 + PASC_MAX_K) <= 64, "the poll area fits its line");
-    e.h_state = reinterpret_cast<InstState *>((char *)e.h_nactive + 64);
+    e.h_state = reinterpret_cast<InstState *>((char *)e.h_poll + 64);
     e.h_parity.assign(e.n_inst, 0);
     // K groups
     for (int K = 1; K <= PASC_MAX_K; K++) {
@@ -301,15 +315,16 @@ void engine_free(Engine &e) {
     if (e.d_desc) (void)hipFree(e.d_desc);
     if (e.d_state) (void)hipFree(e.d_state);
     if (e.d_part) (void)hipFree(e.d_part);
-    if (e.d_nactive) (void)hipFree(e.d_nactive);
+    if (e.d_dirty) (void)hipFree(e.d_dirty);
     if (e.d_done) (void)hipFree(e.d_done);
     e.d_done = nullptr;
-    if (e.h_nactive) (void)hipHostFree(e.h_nactive);
+    if (e.h_poll) (void)hipHostFree(e.h_poll);
     if (e.d_scratch) (void)hipFree(e.d_scratch);
-    for (auto &v : e.ev_solve) {
-        if (v) (void)hipEventDestroy((hipEvent_t)v);
-        v = nullptr;
-    }
+    for (auto *evs : {e.ev_solve, e.ev_batch})
+        for (int i = 0; i < 2; i++) {
+            if (evs[i]) (void)hipEventDestroy((hipEvent_t)evs[i]);
+            evs[i] = nullptr;
+        }
     for (auto &g : e.groups) {
         if (g.d_ids) (void)hipFree(g.d_ids);
         if (g.d_off) (void)hipFree(g.d_off);
@@ -320,8 +335,8 @@ void engine_free(Engine &e) {
     e.d_desc = nullptr;
     e.d_state = nullptr;
     e.d_part = nullptr;
-    e.d_nactive = nullptr;
-    e.h_nactive = nullptr;
+    e.d_dirty = nullptr;
+    e.h_poll = nullptr;
     e.d_scratch = nullptr;
 }
 
@@ -508,7 +523,7 @@ static int enqueue_iteration(Engine &e, const PhaseCfg &ph, const std::vector<in
             const void *bb = ph.f64 ? e.d_b64 : e.d_b32;
             PassArgs a{g0, g1, x, e.d_desc, e.d_state, e.d_part, gv, ph.kkt_every,
                        ph.sp.fx_identity ? 0 : 1, bb, ph.sp, fused ? e.d_done : nullptr,
-                       e.d_nactive, e.d_nactive + 1};
+                       e.h_poll, e.d_dirty};
             const PassShape &sh = e.sh[ph.f64 ? 1 : 0];
             rc = launch_pass_1d(ph.f64, g.K, a, grids[gi], sh.block, sh.chunk, sh.prefetch, s);
         } else if (img) {
@@ -518,8 +533,8 @@ static int enqueue_iteration(Engine &e, const PhaseCfg &ph, const std::vector<in
             const int rows = sh.chunk;
             ImgArgs a{g0, g1, d0, d1, e.d_q[ph.f64 ? 1 : 0], e.d_desc, e.d_state, e.d_part, gv,
                       e.geo.width, (int32_t)(e.geo.R / e.geo.width), rows, img_ncol(e),
-                      ph.kkt_every, ph.sp, fused ? e.d_done : nullptr, e.d_nactive,
-                      e.d_nactive + 1};
+                      ph.kkt_every, ph.sp, fused ? e.d_done : nullptr, e.h_poll,
+                      e.d_dirty};
             rc = ph.f64 ? launch_pass_img_double(g.K, a, grids[gi], sh.prefetch, s)
                         : launch_pass_img_float(g.K, a, grids[gi], sh.prefetch, s);
         } else {
@@ -548,8 +563,8 @@ static int enqueue_iteration(Engine &e, const PhaseCfg &ph, const std::vector<in
     // graph kernels skip the tiles of a stopped instance, so no scan is launched.
     const bool single = e.n_inst == 1;
     hipLaunchKernelGGL(spg_step, dim3(std::min(e.n_inst, std::max(e.ctx->n_cu, 1) * 4)), dim3(256),
-                       0, s, e.d_desc, e.d_state, e.d_part, e.n_inst, ph.sp, e.d_nactive + 1,
-                       single ? e.d_nactive : nullptr);
+                       0, s, e.d_desc, e.d_state, e.d_part, e.n_inst, ph.sp, e.d_dirty,
+                       single ? e.h_poll : nullptr);
     if (single) {
         HIP_TRY(hipGetLastError());
         return PASC_OK;
@@ -560,8 +575,8 @@ static int enqueue_iteration(Engine &e, const PhaseCfg &ph, const std::vector<in
         sa.g[gi] = ScanGroup{e.groups[gi].d_ids, e.groups[gi].d_off, e.groups[gi].d_hint, e.groups[gi].n};
     sa.desc = e.d_desc;
     sa.state = e.d_state;
-    sa.nactive = e.d_nactive;
-    sa.dirty = e.d_nactive + 1;
+    sa.poll = e.h_poll;
+    sa.dirty = e.d_dirty;
     hipLaunchKernelGGL(spg_scan, dim3(1), dim3(1024), 0, s, sa);
     HIP_TRY(hipGetLastError());
     return PASC_OK;
@@ -686,7 +701,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
     int rc = engine_scratch(e, sizeof(double) * (size_t)pl.epoch_words * (epochs + 1), &ex);
     if (rc) return rc;
     const bool g64 = ph.f64 && e.precision == PASC_FP32_BULK;
-    int32_t *flags = e.h_nactive;
+    int32_t *flags = e.h_poll;
     while (passes < max_passes) {
         const int n = std::min(epochs, max_passes - passes);
         const int64_t words = pl.epoch_words * (n + 1);
@@ -739,9 +754,16 @@ static int run_phase(Engine &e, const PhaseCfg &ph, const pasc_spg_params &p, in
         int rc0 = run_loop(e, ph, passes, max_passes, &ran);
         e.looped = rc0 == PASC_OK && ran;
         if (rc0 || ran) return rc0;
-        if ((rc0 = prepare(e, nullptr, 0))) return rc0;
     }
-    if (e.cur_phase != (ph.f64 ? 1 : 0) || tile_len(e, ph.f64) != e.cur_tile) {
+    const bool runs = !e.init_state || e.init_state->active;
+    {
+        const int rc0 = prepare(e, nullptr, 0);
+        if (rc0) return rc0;
+    }
+    // the tiles of an image, and of other graphs, do not depend on the type: one tiling serves
+    // both phases
+    const bool phase_tiles = e.stencil == STENCIL_TIME && e.cur_phase != (ph.f64 ? 1 : 0);
+    if (phase_tiles || e.cur_phase < 0 || tile_len(e, ph.f64) != e.cur_tile) {
         int rc0 = engine_retile(e, ph.f64);
         if (rc0) return rc0;
     }
@@ -753,36 +775,65 @@ static int run_phase(Engine &e, const PhaseCfg &ph, const pasc_spg_params &p, in
                                : img_data_terms<float>(e, x, (float *)e.d_q[0]);
         if (rc0) return rc0;
     }
-    // initial scan (active tiles of every group)
-    {
+    // the active tiles of every group (a single problem's stay as they are until the next tiling)
+    e.h_poll[0] = e.n_inst;
+    for (size_t gi = 0; gi < e.groups.size(); gi++) e.h_poll[1 + gi] = (int32_t)e.groups[gi].max_tiles;
+    if (!e.tiled_scan) {
         ScanArgs sa{};
         sa.n_groups = (int)e.groups.size();
         for (size_t gi = 0; gi < e.groups.size(); gi++)
             sa.g[gi] = ScanGroup{e.groups[gi].d_ids, e.groups[gi].d_off, e.groups[gi].d_hint, e.groups[gi].n};
         sa.desc = e.d_desc;
         sa.state = e.d_state;
-        sa.nactive = e.d_nactive;
-        sa.dirty = e.d_nactive + 1;
+        sa.poll = e.h_poll;
+        sa.dirty = e.d_dirty;
         // force the initial rebuild (any non-zero dirty flag)
-        HIP_TRY(hipMemsetAsync(e.d_nactive + 1, 1, sizeof(int32_t), s));
+        HIP_TRY(hipMemsetAsync(e.d_dirty, 1, sizeof(int32_t), s));
         hipLaunchKernelGGL(spg_scan, dim3(1), dim3(1024), 0, s, sa);
         HIP_TRY(hipGetLastError());
+        e.tiled_scan = e.n_inst == 1 && runs;
     }
     std::vector<int> grids;
     for (auto &g : e.groups) {
         int64_t cap = e.grid_cap > 0 ? e.grid_cap : (int64_t)std::max(e.ctx->n_cu, 1) * 64;
         grids.push_back((int)std::max<int64_t>(1, std::min<int64_t>(g.max_tiles, cap)));
     }
-    const int every = std::max(1, p.check_every);
-    std::vector<int32_t *> d_totals;
-    for (auto &g : e.groups) d_totals.push_back(g.d_off + g.n);
     GraphGuard gg;
     EventsGuard eg;
     std::vector<hipEvent_t> &evs = eg.ev;
     int rc = PASC_OK;
-    while (passes < max_passes) {
-        const int n = std::min(every, max_passes - passes);
-        if (p.use_graph && n == every && !e.profile) {
+    // The passes are enqueued in batches, two of them in flight: the device tells through pinned
+    // words what has stopped, so the host never waits for a batch whose successor is not queued.
+    // (Passes past the stop find no active instance; a poll after every iteration cost 10 - 15 us
+    // of each.)  Batches of problems replay a graph of check_every iterations when asked to: their
+    // iterations are several launches of a few microseconds.
+    const bool graph = p.use_graph && e.n_inst > 1 && !e.profile;
+    const int batch = graph ? std::max(1, p.check_every) : 4;
+    for (auto &v : e.ev_batch)
+        if (!v) HIP_TRY(hipEventCreateWithFlags((hipEvent_t *)&v, hipEventDisableTiming));
+    const volatile int32_t *poll = e.h_poll;
+    for (int b = 0; passes < max_passes; b++) {
+        hipEvent_t ev = (hipEvent_t)e.ev_batch[b & 1];
+        if (b >= 2) {
+            HIP_TRY(hipEventSynchronize(ev));
+            if (poll[0] == 0) break;
+            // shrink the persistent grids once most tiles have converged (idle workgroups still
+            // cost a dispatch each); the graph is re-captured with the new launch shapes
+            bool shrink = false;
+            for (size_t gi = 0; gi < grids.size(); gi++) {
+                const int need = std::max(1, (int)poll[1 + gi]);
+                if (grids[gi] > 2 * need && grids[gi] > 64) {
+                    grids[gi] = std::max(need, 64);
+                    shrink = true;
+                }
+            }
+            if (shrink && gg.exec) {
+                HIP_TRY(hipStreamSynchronize(s));  // the old graph may still be in flight
+                gg.reset();
+            }
+        }
+        const int n = std::min(batch, max_passes - passes);
+        if (graph && n == batch) {
             if (!gg.exec) {
                 HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
                 for (int i = 0; i < n && rc == PASC_OK; i++) rc = enqueue_iteration(e, ph, grids);
@@ -800,24 +851,9 @@ static int run_phase(Engine &e, const PhaseCfg &ph, const pasc_spg_params &p, in
             }
         }
         passes += n;
-        HIP_TRY(hipMemcpyAsync(e.h_nactive, e.d_nactive, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        for (size_t gi = 0; gi < d_totals.size(); gi++)
-            HIP_TRY(hipMemcpyAsync(e.h_nactive + 1 + gi, d_totals[gi], sizeof(int32_t),
-                                   hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        if (*e.h_nactive == 0) break;
-        // shrink the persistent grids once most tiles have converged (idle workgroups still cost
-        // a dispatch each); the graph is re-captured with the new launch shapes
-        bool shrink = false;
-        for (size_t gi = 0; gi < grids.size(); gi++) {
-            const int need = std::max(1, (int)e.h_nactive[1 + gi]);
-            if (grids[gi] > 2 * need && grids[gi] > 64) {
-                grids[gi] = std::max(need, 64);
-                shrink = true;
-            }
-        }
-        if (shrink) gg.reset();
+        HIP_TRY(hipEventRecord(ev, s));
     }
+    if (gg.exec) HIP_TRY(hipStreamSynchronize(s));
     gg.reset();
     {
         // the passes stored K - 1 rows: write the last one of every current iterate
@@ -973,13 +1009,13 @@ int engine_solve(Engine &e, const pasc_spg_params &p, pasc_spg_result *res_singl
     std::vector<int> it32(e.n_inst, 0), it64(e.n_inst, 0);
     if (!bulk32) {
         PhaseCfg ph{true, make_step(p, false), p.kkt_every};
-        rc = run_phase(e, ph, p, p.maxit + 2);
+        rc = run_phase(e, ph, p, p.maxit + 1);
         if (rc) return rc;
         if ((rc = get_states(e, st))) return rc;
         for (int i = 0; i < e.n_inst; i++) { it64[i] = st[i].it; e.h_parity[i] = st[i].parity; }
     } else {
         PhaseCfg ph{false, make_step(p, true), p.kkt_every};
-        rc = run_phase(e, ph, p, p.maxit + 2);
+        rc = run_phase(e, ph, p, p.maxit + 1);
         if (rc) return rc;
         if ((rc = get_states(e, st))) return rc;
         // FP64 polish: promote the FP32 iterate and certify the target in FP64
@@ -1014,7 +1050,7 @@ int engine_solve(Engine &e, const pasc_spg_params &p, pasc_spg_result *res_singl
         pasc_spg_params pp = p;
         pp.maxit = p.polish_maxit > 0 ? p.polish_maxit : p.maxit;
         PhaseCfg ph2{true, make_step(pp, false), p.kkt_every};
-        rc = run_phase(e, ph2, pp, pp.maxit + 2);
+        rc = run_phase(e, ph2, pp, pp.maxit + 1);
         if (rc) return rc;
         e.cur64 = true;
         if ((rc = get_states(e, st))) return rc;

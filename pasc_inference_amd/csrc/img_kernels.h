@@ -52,7 +52,7 @@ struct ImgArgs {
     int32_t kkt_every;      // evaluate the KKT residual on passes with it % kkt_every == 0
     StepParams sp;
     int32_t *done;          // fused step (single problems, as PassArgs::done) or null
-    int32_t *nactive;
+    int32_t *running;       // as PassArgs::running
     int32_t *dirty;
 };
 
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(WAVE) void spg_pass_img(ImgArgs A) {
             }
             __syncthreads();
             if (step_due)
-                fused_step<WAVE>(A.desc, A.state, A.done, A.sp, A.dirty, A.nactive, 0, &lds_state,
+                fused_step<WAVE>(A.desc, A.state, A.done, A.sp, A.dirty, A.running, 0, &lds_state,
                                  lds_red);
         }
     }

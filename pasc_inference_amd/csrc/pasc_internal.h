@@ -152,10 +152,11 @@ struct Engine {
         int hint_len = 0;
     };
     std::vector<Group> groups;
-    int32_t *d_nactive = nullptr;        // device counter of active instances
+    int32_t *d_dirty = nullptr;          // set when an instance stopped (the tile scan rebuilds)
     int32_t *d_done = nullptr;           // completed-slot counters and group partials of the
                                          // fused step (DONE_BYTES, single problems only)
-    int32_t *h_nactive = nullptr;        // pinned: active instances, then active tiles per K group
+    int32_t *h_poll = nullptr;           // pinned, written by the device: active instances, then
+                                         // active tiles per K group
     InstState *h_state = nullptr;        // pinned: the final state of a single problem's loop
     // single problems: h_desc (and the initial state of a solve) go to the device with the first
     // kernel that needs them
@@ -163,6 +164,9 @@ struct Engine {
     const InstState *init_state = nullptr;
     bool looped = false;                 // the last phase ran the persistent loop (h_state holds)
     void *ev_solve[2] = {nullptr, nullptr};  // hipEvents around a solve
+    void *ev_batch[2] = {nullptr, nullptr};  // and after the last two batches of passes
+    int64_t part_slots = 0;              // slots d_part holds (all empty between solves)
+    bool tiled_scan = false;             // a single problem's tile enumeration is on the device
     PassShape sh[2];                     // [0] FP32 phase of FP32-bulk, [1] every FP64 pass
     bool shape_pinned = false;           // the caller pinned sh: the tiled passes run it
     int grid_cap = 0;                    // persistent grid cap (0: 32 blocks per CU)

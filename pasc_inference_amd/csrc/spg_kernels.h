@@ -41,7 +41,7 @@ struct PassArgs {
     int32_t *done;      // DONE_WORDS counters of completed slots in this pass (back to 0
                         // after), then DONE_SUB group partials; null: the step kernel runs
                         // the step
-    int32_t *nactive;   // active instances (decremented when one stops)
+    int32_t *running;   // pinned host word: 0 once a single problem has stopped
     int32_t *dirty;     // set when an instance stops (the batch's tile scan rebuilds)
 };
 
@@ -544,7 +544,7 @@ __device__ __forceinline__ double *group_partials(int32_t *done) {
 // partials are reduced in a fixed order and step_scalar advances the instance.
 template <int NT>
 __device__ __forceinline__ void fused_step(const InstDesc *desc, InstState *state, int32_t *done,
-                                           const StepParams &sp, int32_t *dirty, int32_t *nactive,
+                                           const StepParams &sp, int32_t *dirty, int32_t *running,
                                            int inst, InstState *lds_state, double *lds_red) {
     const InstDesc &D = desc[inst];
     const int ns = uni(D.ntiles);
@@ -558,7 +558,7 @@ __device__ __forceinline__ void fused_step(const InstDesc *desc, InstState *stat
     // the group partials are taken: empty again for the next pass
     const int ng = ns < DONE_SUB ? ns : DONE_SUB;
     for (int i = threadIdx.x; i < ng * NPART; i += NT) reset_published(gp + i);
-    if (threadIdx.x == 0 && !lds_state->active) atomicSub(nactive, 1);
+    if (threadIdx.x == 0 && !lds_state->active) *running = 0;
 }
 
 // Counts one completed partial slot of a single problem (its values already written with
@@ -713,7 +713,7 @@ __global__ __launch_bounds__(NT) void spg_pass_1d(PassArgs A) {
             }
             __syncthreads();
             if (step_due)
-                fused_step<NT>(A.desc, A.state, A.done, A.sp, A.dirty, A.nactive, 0, &lds_state,
+                fused_step<NT>(A.desc, A.state, A.done, A.sp, A.dirty, A.running, 0, &lds_state,
                                lds_red);
         }
     }

@@ -8,11 +8,11 @@ namespace pasc {
 
 // Step kernel: workgroups stride over the instances; each reduces one active instance's partial
 // slots in a fixed order (deterministic) and runs step_scalar.
-// nactive: decremented when an instance stops (single problems, which launch no scan); null
-// when the active-tile scan recounts the active instances.
+// running: a pinned host word, 0 once the instance has stopped (single problems, which launch no
+// scan); null when the active-tile scan counts the active instances.
 __global__ __launch_bounds__(256) void spg_step(const InstDesc *desc, InstState *state,
                                                  const double *part, int n_inst, StepParams P,
-                                                 int32_t *dirty, int32_t *nactive) {
+                                                 int32_t *dirty, int32_t *running) {
     // one workgroup per instance: a single instance of T = 1e7 owns ~1e4 partial slots
     __shared__ double lds[NPART * 4];
     __shared__ InstState lds_state;
@@ -23,7 +23,7 @@ __global__ __launch_bounds__(256) void spg_step(const InstDesc *desc, InstState 
         step_instance<256>(state + w, uni(D.ntiles), D.alpha * D.s_kkt, P, dirty, &lds_state, lds,
                            [&](int i, int q) { return pw[(int64_t)i * NPART + q]; },
                            [](int, int, double v) { return v; });
-        if (nactive && threadIdx.x == 0 && !lds_state.active) atomicSub(nactive, 1);
+        if (running && threadIdx.x == 0 && !lds_state.active) *running = 0;
         __syncthreads();  // lds_state is reused by the next instance
     }
 }
@@ -47,7 +47,7 @@ struct ScanArgs {
     int32_t n_groups;
     const InstDesc *desc;
     const InstState *state;
-    int32_t *nactive;
+    int32_t *poll;   // pinned host words: [0] active instances, [1 + g] active tiles of K group g
     int32_t *dirty;  // set by the step kernel when an instance stopped; cleared here
 };
 
@@ -106,7 +106,8 @@ __global__ __launch_bounds__(1024) void spg_scan(ScanArgs A) {
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        *A.nactive = red[0];
+        for (int gi = 0; gi < A.n_groups; gi++) A.poll[1 + gi] = A.g[gi].off[A.g[gi].n];
+        A.poll[0] = red[0];
         *A.dirty = 0;
     }
 }
