@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "img_kernels.h"
+#include "img_loop.h"
 #include "loop_kernels.h"
 #include "project_kernels.h"
 #include "spg_kernels.h"
@@ -49,6 +50,11 @@ int launch_pass_grid_double(int K, const GridArgs &a, int grid, hipStream_t s);
 int launch_pass_img_float(int K, const ImgArgs &a, int grid, int pd, hipStream_t s);
 int launch_pass_img_double(int K, const ImgArgs &a, int grid, int pd, hipStream_t s);
 
+#define PASC_IMG_LOOP(S, R) \
+    int launch_img_loop_##S##_##R##_(int K, const ImgLoopArgs &a, int nwg, int nw, hipStream_t s);
+PASC_IMG_LOOP(float, 1) PASC_IMG_LOOP(float, 2) PASC_IMG_LOOP(float, 4) PASC_IMG_LOOP(float, 8)
+PASC_IMG_LOOP(double, 1) PASC_IMG_LOOP(double, 2) PASC_IMG_LOOP(double, 4) PASC_IMG_LOOP(double, 8)
+#undef PASC_IMG_LOOP
 int launch_loop_1d_float_4_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
 int launch_loop_1d_float_8_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
 int launch_loop_1d_double_4_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
@@ -624,11 +630,12 @@ static int img_data_terms(Engine &e, const void *x, S *q) {
     return PASC_OK;
 }
 
-// The persistent loop of a phase (loop_kernels.h): how many workgroups of how many waves with how
-// many steps per lane, or nwg = 0 when the problem does not run it.
+// The persistent loop of a phase (loop_kernels.h, img_loop.h): how many workgroups of how many
+// waves with how many steps per lane or rows per wave, or nwg = 0 when the problem does not run it.
 struct LoopPlan {
     int nwg = 0, nw = 0, chunk = 0, tpw = 0, ntiles = 0;
-    int64_t epoch_words = 0;
+    int rows = 0, nct = 0;  // images: rows per wave, tiles across
+    int64_t epoch_words = 0, edge_words = 0;
 };
 
 template <typename S, int K, int CH>
@@ -662,11 +669,35 @@ static void loop_shapes(int64_t T, int n_cu, LoopPlan &pl) {
     if constexpr (loop_has_chunk(f64, K, 4)) loop_shape<S, K, 4>(T, n_cu, pl);
 }
 
+// The smallest tiles that give every workgroup a compute unit (the iteration is as long as a
+// wave's rows).
+static void img_loop_plan(const Engine &e, bool f64, int n_cu, LoopPlan &pl) {
+    const int K = e.h_desc[0].K;
+    const int64_t w = e.geo.width, h = e.geo.R / e.geo.width, nct = (w + WAVE - 1) / WAVE;
+    const int most = f64 ? img_loop_rows<double>(K) : img_loop_rows<float>(K);
+    static const int shapes[][2] = {{4, 1}, {8, 1}, {8, 2}, {8, 4}, {8, 8}};  // waves, rows per wave
+    for (const auto &s : shapes) {
+        const int th = s[0] * s[1];
+        const int64_t nwg = nct * ((h + th - 1) / th);
+        if (s[1] > most) break;
+        if (nwg > n_cu) continue;
+        pl.nwg = (int)nwg;
+        pl.nw = s[0];
+        pl.rows = s[1];
+        pl.nct = (int)nct;
+        pl.epoch_words = (int64_t)NPART * slot_stride(pl.nwg);
+        pl.edge_words = (int64_t)IMG_SETS * nwg * K * (2 * WAVE + 2 * th);
+        return;
+    }
+}
+
 static LoopPlan loop_plan(const Engine &e, bool f64) {
     LoopPlan pl;
-    if (e.n_inst != 1 || e.stencil != STENCIL_TIME || e.profile || e.shape_pinned) return pl;
+    if (e.n_inst != 1 || e.profile || e.shape_pinned) return pl;
     const InstDesc &d = e.h_desc[0];
     const int n_cu = std::max(e.ctx->n_cu, 1);
+    if (engine_is_image(e)) img_loop_plan(e, f64, n_cu, pl);
+    if (e.stencil != STENCIL_TIME) return pl;
     switch (d.K) {
 #define PASC_LK(KK)                                        \
     case KK:                                               \
@@ -698,40 +729,76 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
     const int64_t cap = std::max<int64_t>(1, LOOP_EXCHANGE_BYTES / (8 * pl.epoch_words));
     const int epochs = (int)std::min<int64_t>(std::min(max_passes, LOOP_EPOCHS_MAX), cap);
     void *ex;
-    int rc = engine_scratch(e, sizeof(double) * (size_t)pl.epoch_words * (epochs + 1), &ex);
+    int rc = engine_scratch(
+        e, sizeof(double) * (size_t)(pl.epoch_words * (epochs + 1) + pl.edge_words), &ex);
     if (rc) return rc;
+    const bool img = pl.rows > 0;
+    const int b = ph.f64 ? 1 : 0;
     const bool g64 = ph.f64 && e.precision == PASC_FP32_BULK;
+    void *g0 = g64 ? e.d_gamma64[0] : e.d_gamma[0], *g1 = g64 ? e.d_gamma64[1] : e.d_gamma[1];
+    const void *x = ph.f64 ? (const void *)e.d_x64 : (const void *)e.d_x32;
     int32_t *flags = e.h_poll;
-    while (passes < max_passes) {
+    const int K = e.h_desc[0].K;
+    const int need_f = ph.sp.fx_identity ? 0 : 1;
+    // a residual that no stop test reads is only reported: it is formed for the last iterate
+    const int kkt_last = !ph.sp.fp32_phase && ph.kkt_every <= 1 && !(ph.sp.stop_mask & PASC_STOP_KKT);
+    if (img && !e.d_q[b]) HIP_TRY(hipMalloc(&e.d_q[b], (ph.f64 ? 8 : 4) * (size_t)e.state_elems));
+    for (bool fresh = true; passes < max_passes; fresh = false) {
         const int n = std::min(epochs, max_passes - passes);
-        const int64_t words = pl.epoch_words * (n + 1);
-        if ((rc = prepare(e, (uint64_t *)ex, words))) return rc;
-        LoopArgs a{};
-        a.p.gamma0 = g64 ? e.d_gamma64[0] : e.d_gamma[0];
-        a.p.gamma1 = g64 ? e.d_gamma64[1] : e.d_gamma[1];
-        a.p.x = ph.f64 ? e.d_x64 : e.d_x32;
-        a.p.b = ph.f64 ? e.d_b64 : e.d_b32;
-        a.p.desc = e.d_desc;
-        a.p.state = e.d_state;
-        a.p.kkt_every = ph.kkt_every;
-        a.p.need_f = ph.sp.fx_identity ? 0 : 1;
-        a.p.sp = ph.sp;
-        a.ex = (double *)ex;
-        a.flags = flags;
-        a.out = e.h_state;
-        a.ntiles = pl.ntiles;
-        a.tpw = pl.tpw;
-        a.epochs = n;
-        // a residual that no stop test reads is only reported: it is formed for the last iterate
-        a.kkt_last = !ph.sp.fp32_phase && ph.kkt_every <= 1 && !(ph.sp.stop_mask & PASC_STOP_KKT);
+        const int64_t sums = pl.epoch_words * (n + 1);
+        if ((rc = prepare(e, (uint64_t *)ex, sums + pl.edge_words))) return rc;
         flags[0] = 1;
         flags[1] = 0;
-        const int K = e.h_desc[0].K;
-        const bool small = pl.nw == LOOP_WAVES_MIN;
-        if (ph.f64)
-            rc = small ? launch_loop_1d_double_4_(K, a, pl.nwg, pl.chunk, s) : launch_loop_1d_double_8_(K, a, pl.nwg, pl.chunk, s);
-        else
-            rc = small ? launch_loop_1d_float_4_(K, a, pl.nwg, pl.chunk, s) : launch_loop_1d_float_8_(K, a, pl.nwg, pl.chunk, s);
+        if (img) {
+            if (fresh) rc = ph.f64 ? img_data_terms<double>(e, x, (double *)e.d_q[1])
+                                   : img_data_terms<float>(e, x, (float *)e.d_q[0]);
+            if (rc) return rc;
+            ImgLoopArgs a{};
+            a.p = ImgArgs{g0, g1, g64 ? e.d_dir64[0] : e.d_dir[0], g64 ? e.d_dir64[1] : e.d_dir[1],
+                          e.d_q[b], e.d_desc, e.d_state, nullptr, GroupView{}, e.geo.width,
+                          (int32_t)(e.geo.R / e.geo.width), 0, 0, ph.kkt_every, ph.sp, nullptr,
+                          nullptr, nullptr};
+            a.ex = (double *)ex;
+            a.edges = (double *)ex + sums;
+            a.out = e.h_state;
+            a.flags = flags;
+            a.nct = pl.nct;
+            a.epochs = n;
+            a.kkt_last = kkt_last;
+            a.need_f = need_f;
+#define PASC_IL(R)                                                                  \
+    case R:                                                                         \
+        rc = ph.f64 ? launch_img_loop_double_##R##_(K, a, pl.nwg, pl.nw, s)         \
+                    : launch_img_loop_float_##R##_(K, a, pl.nwg, pl.nw, s);         \
+        break;
+            switch (pl.rows) { PASC_IL(1) PASC_IL(2) PASC_IL(4) PASC_IL(8) }
+#undef PASC_IL
+        } else {
+            LoopArgs a{};
+            a.p.gamma0 = g0;
+            a.p.gamma1 = g1;
+            a.p.x = x;
+            a.p.b = ph.f64 ? e.d_b64 : e.d_b32;
+            a.p.desc = e.d_desc;
+            a.p.state = e.d_state;
+            a.p.kkt_every = ph.kkt_every;
+            a.p.need_f = need_f;
+            a.p.sp = ph.sp;
+            a.ex = (double *)ex;
+            a.flags = flags;
+            a.out = e.h_state;
+            a.ntiles = pl.ntiles;
+            a.tpw = pl.tpw;
+            a.epochs = n;
+            a.kkt_last = kkt_last;
+            const bool small = pl.nw == LOOP_WAVES_MIN;
+            if (ph.f64)
+                rc = small ? launch_loop_1d_double_4_(K, a, pl.nwg, pl.chunk, s)
+                           : launch_loop_1d_double_8_(K, a, pl.nwg, pl.chunk, s);
+            else
+                rc = small ? launch_loop_1d_float_4_(K, a, pl.nwg, pl.chunk, s)
+                           : launch_loop_1d_float_8_(K, a, pl.nwg, pl.chunk, s);
+        }
         if (rc) {
             (void)hipGetLastError();
             return PASC_OK;

@@ -100,11 +100,119 @@ struct LaneWindow {
     __device__ double max(int) const { return top; }
 };
 
-// What the waves need of the step, published in LDS by wave 0.
-struct LoopBroadcast {
+__device__ __forceinline__ void loop_load_state(const InstState &g, int m, int lane, LoopState &st,
+                                                double &window) {
+    st.f = g.f; st.f_prev = g.f_prev; st.dd_prev = g.dd_prev; st.dAd_prev = g.dAd_prev;
+    st.dd = g.dd; st.dAd = g.dAd; st.gd = g.gd; st.alpha_dir = g.alpha_dir;
+    st.alpha_apply = g.alpha_apply; st.beta_apply = g.beta_apply; st.kkt = g.kkt;
+    st.best_kkt = g.best_kkt; st.normb = g.normb; st.fs_last = g.fs_last; st.it = g.it;
+    st.first = g.first; st.active = g.active; st.reason = g.reason; st.status = g.status;
+    st.stall = g.stall; st.parity = g.parity; st.it_base = g.it_base;
+    window = lane < m ? g.fs[lane] : -__builtin_huge_val();
+}
+
+__device__ __forceinline__ void loop_put_state(InstState &g, int m, int lane, const LoopState &st,
+                                               double window) {
+    if (lane < m) g.fs[lane] = window;
+    if (lane != 0) return;
+    g.f = st.f; g.f_prev = st.f_prev; g.dd_prev = st.dd_prev; g.dAd_prev = st.dAd_prev;
+    g.dd = st.dd; g.dAd = st.dAd; g.gd = st.gd; g.alpha_dir = st.alpha_dir;
+    g.alpha_apply = st.alpha_apply; g.beta_apply = st.beta_apply; g.kkt = st.kkt;
+    g.best_kkt = st.best_kkt; g.normb = st.normb; g.fs_last = st.fs_last; g.it = st.it;
+    g.first = st.first; g.active = st.active; g.reason = st.reason; g.status = st.status;
+    g.stall = st.stall; g.parity = st.parity; g.it_base = st.it_base;
+}
+
+// LDS of the exchange: the waves' sums, and what the waves need of the step (written by wave 0).
+struct LoopShared {
+    double red[NPART][8];  // [sum][wave]; waves from NW on stay 0
     double a_apply, b_apply, a_dir;
     int32_t it, active, parity;
 };
+
+// A wave's share of the iteration's sums dd, (sum of the edge terms), dd + off, f, residual: four
+// by lane folds, the residual (a maximum) where it is wanted.
+template <int NW>
+__device__ __forceinline__ void loop_sums(LoopShared &sh, double (&acc)[NPART], bool want_kkt,
+                                          int lane, int wave) {
+    const double sums = wave_sum4(acc[0], acc[1], acc[2], acc[3]);
+    if (want_kkt) acc[4] = wave_max_all(acc[4]);
+    if ((lane & 15) == 0)
+        sh.red[lane == ROW_A ? 0 : lane == ROW_B ? 1 : lane == ROW_C ? 2 : 3][wave] = sums;
+    if (lane == 1) sh.red[4][wave] = acc[4];
+}
+
+// Wave 0, after a barrier: the workgroup's sums to its place in the exchange area's rows, every
+// workgroup's sums added up, and the SPG step on them (the same bits in every workgroup).
+// edge_scale: d'Ad = edge_scale * (sum of the edge terms).
+__device__ __forceinline__ void loop_step(LoopShared &sh, bool want_kkt, double edge_scale,
+                                          double a_dir, double sample_eps, double *ex, int slot_ld,
+                                          int nwg, int wg, int lane, LoopState &st, double &window,
+                                          const StepParams &sp, int32_t *flags) {
+    // lane 8 q + w holds wave w's value q; three exchanges sum over w
+    double v0 = lane < 8 * NPART ? sh.red[lane >> 3][lane & 7] : 0.0, v1 = v0;
+    v0 += dpp_from<DPP_XOR1>(v0);
+    v0 += dpp_from<DPP_XOR2>(v0);
+    v0 += dpp_from<DPP_HALF_MIRROR>(v0);
+    if (want_kkt) {
+        v1 = nan_max(v1, dpp_from<DPP_XOR1>(v1));
+        v1 = nan_max(v1, dpp_from<DPP_XOR2>(v1));
+        v1 = nan_max(v1, dpp_from<DPP_HALF_MIRROR>(v1));
+    }
+    if (lane < 8 * NPART && (lane & 7) == 0)
+        store_coherent(ex + (int64_t)(lane >> 3) * slot_ld + wg, lane == 32 ? v1 : v0);
+    // the window's maximum without the entry this step replaces
+    const int at = st.fs_last + 1 >= sp.m ? 0 : st.fs_last + 1;
+    const LaneWindow win{window, wave_max_all(lane == at ? -__builtin_huge_val() : window),
+                         lane, 0.0};
+    // every workgroup's sums, in slot order per lane; all values of a lane's slots are
+    // re-read together until the last one is there
+    double v[NPART] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int j0 = lane; j0 < nwg; j0 += 4 * WAVE) {
+        double w[4][NPART];
+        bool all;
+        int n = 0;
+        do {
+            all = true;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const int j = j0 + b * WAVE;
+#pragma unroll
+                for (int q = 0; q < NPART; q++)
+                    w[b][q] = j < nwg ? load_coherent(ex + (int64_t)q * slot_ld + j) : 0.0;
+            }
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+#pragma unroll
+                for (int q = 0; q < NPART; q++) all = all && published(w[b][q]);
+        } while (!all && ++n < LOOP_SPIN_LIMIT);
+        if (!all) {
+            flags[1] = 1;
+            w[0][0] = __builtin_nan("");
+        }
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+#pragma unroll
+            for (int q = 0; q < NPART - 1; q++) v[q] += w[b][q];
+            v[NPART - 1] = nan_max(v[NPART - 1], w[b][NPART - 1]);
+        }
+    }
+    const double tot = wave_sum4(v[0], v[1], v[2], v[3]);
+    v[0] = lane_value(tot, ROW_A);
+    v[1] = edge_scale * lane_value(tot, ROW_B);
+    v[2] = -lane_value(tot, ROW_C) / a_dir;
+    v[3] = 0.5 * lane_value(tot, ROW_D);
+    v[4] = want_kkt ? wave_max_all(v[4]) : -1.0;  // -1: not evaluated on this pass
+    step_core(sample_eps, st, win, v, sp);
+    if (lane == 0) {
+        sh.a_apply = st.alpha_apply;
+        sh.b_apply = st.beta_apply;
+        sh.a_dir = st.alpha_dir;
+        sh.it = st.it;
+        sh.active = st.active;
+        sh.parity = st.parity;
+    }
+}
 
 // max |gamma - P(gamma - s g)| over a thread's owned steps (the natural KKT residual)
 template <typename S, typename C, int K, int CH, typename Exch>
@@ -137,8 +245,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
     using VT = V16<S>;
     constexpr int VW = VT::n;
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    __shared__ double red[NPART][8];  // [sum][wave]; waves from NW on stay 0
-    __shared__ LoopBroadcast bc;
+    __shared__ LoopShared sh;
 
     const int nwg = gridDim.x, wg = blockIdx.x;
     const int lane = threadIdx.x & (WAVE - 1), wave = uni((int32_t)(threadIdx.x / WAVE));
@@ -162,18 +269,9 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
 
     LoopState st{};
     double window = 0.0;
-    if (wave == 0) {
-        const InstState &g = A.p.state[0];
-        st.f = g.f; st.f_prev = g.f_prev; st.dd_prev = g.dd_prev; st.dAd_prev = g.dAd_prev;
-        st.dd = g.dd; st.dAd = g.dAd; st.gd = g.gd; st.alpha_dir = g.alpha_dir;
-        st.alpha_apply = g.alpha_apply; st.beta_apply = g.beta_apply; st.kkt = g.kkt;
-        st.best_kkt = g.best_kkt; st.normb = g.normb; st.fs_last = g.fs_last; st.it = g.it;
-        st.first = g.first; st.active = g.active; st.reason = g.reason; st.status = g.status;
-        st.stall = g.stall; st.parity = g.parity; st.it_base = g.it_base;
-        window = lane < A.p.sp.m ? g.fs[lane] : -__builtin_huge_val();
-    }
+    if (wave == 0) loop_load_state(A.p.state[0], A.p.sp.m, lane, st, window);
     const int slot_ld = slot_stride(nwg);
-    if (threadIdx.x < 8 * NPART) red[threadIdx.x >> 3][threadIdx.x & 7] = 0.0;
+    if (threadIdx.x < 8 * NPART) sh.red[threadIdx.x >> 3][threadIdx.x & 7] = 0.0;
     // the series ends where no neighbouring workgroup is: zero halos there
     for (int i = threadIdx.x; i < 2 * 2 * EDGE; i += NW * WAVE) {
         const int par = i / (2 * EDGE), r = i - par * 2 * EDGE;
@@ -320,77 +418,11 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
             else
                 levels(std::false_type{});
         }
-        // the workgroup's sums: four of the wave's by lane folds, then over the waves in LDS
-        const double sums = wave_sum4(acc[0], acc[1], acc[2], acc[3]);
-        if (cx.want_kkt) acc[4] = wave_max_all(acc[4]);
-        if ((lane & 15) == 0) red[lane == ROW_A ? 0 : lane == ROW_B ? 1 : lane == ROW_C ? 2 : 3][wave] = sums;
-        if (lane == 1) red[4][wave] = acc[4];
+        loop_sums<NW>(sh, acc, cx.want_kkt, lane, wave);
         lds_barrier();
-        if (wave == 0) {
-            // lane 8 q + w holds wave w's value q; three exchanges sum over w
-            double v0 = lane < 8 * NPART ? red[lane >> 3][lane & 7] : 0.0, v1 = v0;
-            v0 += dpp_from<DPP_XOR1>(v0);
-            v0 += dpp_from<DPP_XOR2>(v0);
-            v0 += dpp_from<DPP_HALF_MIRROR>(v0);
-            if (cx.want_kkt) {
-                v1 = nan_max(v1, dpp_from<DPP_XOR1>(v1));
-                v1 = nan_max(v1, dpp_from<DPP_XOR2>(v1));
-                v1 = nan_max(v1, dpp_from<DPP_HALF_MIRROR>(v1));
-            }
-            if (lane < 8 * NPART && (lane & 7) == 0)
-                store_coherent(ex + (int64_t)(lane >> 3) * slot_ld + wg, lane == 32 ? v1 : v0);
-            // the window's maximum without the entry this step replaces
-            const int at = st.fs_last + 1 >= A.p.sp.m ? 0 : st.fs_last + 1;
-            const LaneWindow win{window, wave_max_all(lane == at ? -__builtin_huge_val() : window),
-                                 lane, 0.0};
-            // every workgroup's sums, in slot order per lane; all values of a lane's slots are
-            // re-read together until the last one is there
-            double v[NPART] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            for (int j0 = lane; j0 < nwg; j0 += 4 * WAVE) {
-                double w[4][NPART];
-                bool all;
-                int n = 0;
-                do {
-                    all = true;
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        const int j = j0 + b * WAVE;
-#pragma unroll
-                        for (int q = 0; q < NPART; q++)
-                            w[b][q] = j < nwg ? load_coherent(ex + (int64_t)q * slot_ld + j) : 0.0;
-                    }
-#pragma unroll
-                    for (int b = 0; b < 4; b++)
-#pragma unroll
-                        for (int q = 0; q < NPART; q++) all = all && published(w[b][q]);
-                } while (!all && ++n < LOOP_SPIN_LIMIT);
-                if (!all) {
-                    A.flags[1] = 1;
-                    w[0][0] = __builtin_nan("");
-                }
-#pragma unroll
-                for (int b = 0; b < 4; b++) {
-#pragma unroll
-                    for (int q = 0; q < NPART - 1; q++) v[q] += w[b][q];
-                    v[NPART - 1] = nan_max(v[NPART - 1], w[b][NPART - 1]);
-                }
-            }
-            const double tot = wave_sum4(v[0], v[1], v[2], v[3]);
-            v[0] = lane_value(tot, ROW_A);
-            v[1] = 2.0 * (double)cx.alpha * lane_value(tot, ROW_B);
-            v[2] = -lane_value(tot, ROW_C) / (double)cx.a_dir;
-            v[3] = 0.5 * lane_value(tot, ROW_D);
-            v[4] = cx.want_kkt ? wave_max_all(v[4]) : -1.0;  // -1: not evaluated on this pass
-            step_core(sample_eps, st, win, v, A.p.sp);
-            if (lane == 0) {
-                bc.a_apply = st.alpha_apply;
-                bc.b_apply = st.beta_apply;
-                bc.a_dir = st.alpha_dir;
-                bc.it = st.it;
-                bc.active = st.active;
-                bc.parity = st.parity;
-            }
-        }
+        if (wave == 0)
+            loop_step(sh, cx.want_kkt, 2.0 * (double)cx.alpha, (double)cx.a_dir, sample_eps, ex, slot_ld,
+                      nwg, wg, lane, st, window, A.p.sp, A.flags);
         if (wave == NW - 1) {
             // the neighbouring workgroups' edges of this iteration
             for (int i = lane; i < 2 * EDGE; i += WAVE) {
@@ -403,16 +435,16 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
             }
         }
         lds_barrier();
-        cx.a_apply = uni(C(bc.a_apply));
-        cx.b_apply = uni(C(bc.b_apply));
-        cx.a_dir = uni(C(bc.a_dir));
+        cx.a_apply = uni(C(sh.a_apply));
+        cx.b_apply = uni(C(sh.b_apply));
+        cx.a_dir = uni(C(sh.a_dir));
         cx.first = false;
         cx.need_f = A.p.need_f;
-        cx.want_kkt = !A.kkt_last && uni(bc.it) % kkt_every == 0;
-        if (uni(bc.active) == 0) break;
+        cx.want_kkt = !A.kkt_last && uni(sh.it) % kkt_every == 0;
+        if (uni(sh.active) == 0) break;
     }
     // the residual of the iterate that stopped, where no iteration asked for it
-    if (A.kkt_last && uni(bc.active) == 0) {
+    if (A.kkt_last && uni(sh.active) == 0) {
         double kkt = 0.0;
         for (int lt = wave; lt < ntl; lt += NW) {
             const int64_t t0 = (int64_t)(tile0 + lt) * TILE - (int64_t)HT * CH + (int64_t)lane * CH;
@@ -424,13 +456,13 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
             kkt = nan_max(kkt, (double)p);
         }
         kkt = wave_max_all(kkt);
-        if (lane == 0) red[4][wave] = kkt;
+        if (lane == 0) sh.red[4][wave] = kkt;
         __syncthreads();
         double *ex = A.ex + L::epoch_words(nwg) * (e + 1);
         if (wave == 0) {
             kkt = 0.0;
 #pragma unroll
-            for (int w = 0; w < NW; w++) kkt = nan_max(kkt, red[4][w]);
+            for (int w = 0; w < NW; w++) kkt = nan_max(kkt, sh.red[4][w]);
             if (lane == 0) store_coherent(ex + wg, kkt);
             if (wg == 0) {
                 for (int j = lane; j < nwg; j += WAVE)
@@ -440,7 +472,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
         }
     }
     // the iterate to the buffer its parity names: K rows, the last rebuilt as complete_last_row
-    S *dst = reinterpret_cast<S *>(uni(bc.parity) ? A.p.gamma1 : A.p.gamma0) + uni(A.p.desc[0].goff);
+    S *dst = reinterpret_cast<S *>(uni(sh.parity) ? A.p.gamma1 : A.p.gamma0) + uni(A.p.desc[0].goff);
     for (int lt = wave; lt < ntl; lt += NW) {
         const int64_t t0 = (int64_t)(tile0 + lt) * TILE - (int64_t)HT * CH + (int64_t)lane * CH;
         const S *trow = rows + (size_t)lt * (KS + 1) * ROW + lane * CH;
@@ -478,18 +510,8 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
         }
     }
     if (wg == 0 && wave == 0) {
-        auto put = [&](InstState &g) {
-            if (lane < A.p.sp.m) g.fs[lane] = window;
-            if (lane != 0) return;
-            g.f = st.f; g.f_prev = st.f_prev; g.dd_prev = st.dd_prev; g.dAd_prev = st.dAd_prev;
-            g.dd = st.dd; g.dAd = st.dAd; g.gd = st.gd; g.alpha_dir = st.alpha_dir;
-            g.alpha_apply = st.alpha_apply; g.beta_apply = st.beta_apply; g.kkt = st.kkt;
-            g.best_kkt = st.best_kkt; g.normb = st.normb; g.fs_last = st.fs_last; g.it = st.it;
-            g.first = st.first; g.active = st.active; g.reason = st.reason; g.status = st.status;
-            g.stall = st.stall; g.parity = st.parity; g.it_base = st.it_base;
-        };
-        put(A.p.state[0]);
-        put(*A.out);
+        loop_put_state(A.p.state[0], A.p.sp.m, lane, st, window);
+        loop_put_state(*A.out, A.p.sp.m, lane, st, window);
         if (lane == 0) {
             A.flags[0] = st.active;
         }
