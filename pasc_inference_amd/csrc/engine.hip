@@ -685,7 +685,7 @@ static void img_loop_plan(const Engine &e, bool f64, int n_cu, LoopPlan &pl) {
         pl.nw = s[0];
         pl.rows = s[1];
         pl.nct = (int)nct;
-        pl.epoch_words = (int64_t)NPART * slot_stride(pl.nwg);
+        pl.epoch_words = sum_words(pl.nwg);
         pl.edge_words = (int64_t)IMG_SETS * nwg * K * (2 * WAVE + 2 * th);
         return;
     }

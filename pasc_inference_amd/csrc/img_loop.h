@@ -6,9 +6,9 @@
 // rows; lane = column, each wave holds RPW rows of gamma_i and p_i in registers (their last
 // components in LDS), and q too or prefetches it a row ahead.  Left and right neighbours come from
 // the adjacent lanes, rows above and below from registers or, between waves, LDS; no node is
-// computed twice.  us per iteration, image pass / here (FP64): 250 x 150, K = 2 13.4 / 6.4;
-// 512 x 512, K = 3 16.4 / 8.8; 1024 x 1024, K = 2 / 3 / 4 19.7 / 23.7 / 29.5 against 10.9 / 13.1 /
-// 17.6 (FP32, K = 4: 25 / 9.8); 300 x 200, K = 8 36 / 9.9.  Issue bounds the large ones (270 - 370
+// computed twice.  us per iteration, image pass / here (FP64): 250 x 150, K = 2 13.4 / 5.3;
+// 512 x 512, K = 3 16.4 / 7.9; 1024 x 1024, K = 2 / 3 / 4 19.7 / 23.7 / 29.5 against 9.7 / 12.1 /
+// 15.5 (FP32, K = 4: 25 / 9.2); 300 x 200, K = 8 36 / 8.8.  Issue bounds the large ones (270 - 370
 // instructions a row, two waves per SIMD), the two exchanges (~2 us each) the small ones.
 // What the layout costs when left out: a row's q loaded where it is used 16 us of 26 at 1024 x 1024,
 // K = 4; reads of the columns beyond the tile under a lane condition, eight branches a row;
@@ -20,11 +20,11 @@
 //   2. g_i, p_i and the node sums of the tile; the tile's outer p_i to the neighbours;
 //   3. the neighbours' p_i, then the edge sums (d_a - d_b)^2, each edge with its upper or left end;
 //   4. the sums and the step (loop_sums, loop_step).
-// The exchanged rows lie in three sets used in turn.  A workgroup marks its places of the next
-// set empty while it publishes into this one: that set's last readers ended before they
-// published the sums of the iteration before, which this workgroup has read, and its marks are
-// complete (vmcnt) before it publishes this iteration's sums, which a reader needs before it
-// turns to that set.
+// The exchanged rows lie in four sets used in turn.  While a workgroup publishes into one, it marks
+// its places of the set after the next empty: that set's last readers ended before they published
+// the sums of two iterations before, which this workgroup has read.  The marks are complete
+// (vmcnt) before it publishes anything of the next iteration, and a reader turns to that set
+// only with that iteration's sums.
 // Every node's arithmetic is the image pass's; the sums differ in order only.
 #pragma once
 
@@ -33,7 +33,7 @@
 
 namespace pasc {
 
-constexpr int IMG_SETS = 3;
+constexpr int IMG_SETS = 4;
 
 struct ImgLoopArgs {
     ImgArgs p;           // buffers, descriptor, state, sizes (grp, part, counters not used)
@@ -238,9 +238,9 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
     bool fresh = first;  // gamma_0 stands
     int e = 0;
     for (; e < A.epochs; e++) {
-        double *ex = A.ex + (int64_t)NPART * slot_ld * e;
+        double *ex = A.ex + sum_words(nwg) * e;
         double *set = A.edges + (int64_t)(e % IMG_SETS) * nwg * L::EDGE;
-        double *next = A.edges + (int64_t)((e + 1) % IMG_SETS) * nwg * L::EDGE;
+        double *next = A.edges + (int64_t)((e + 2) % IMG_SETS) * nwg * L::EDGE;
         double *mine = set + (int64_t)wg * L::EDGE, *empty = next + (int64_t)wg * L::EDGE;
         double acc[NPART] = {0.0, 0.0, 0.0, 0.0, 0.0};
         // recomputed in every iteration: kept, the rows' conditions would spill
@@ -327,7 +327,9 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        // the tile's outer p_i to the neighbours, this workgroup's places of the next set empty
+        // the tile's outer p_i to the neighbours, this workgroup's places of the set after the next
+        // empty (last iteration's marks are complete)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         const double none = __builtin_bit_cast(double, PART_EMPTY);
         auto publish = [&](int off, int stride, const C(&v)[K]) {
 #pragma unroll
@@ -412,10 +414,9 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
                 for (int k = 0; k < K; k++) d[k] = dn[k];
             }
         }
-        // 4. the sums and the step; the marks in the next set are complete before the sums go out
+        // 4. the sums and the step
         if (!need_f) acc[3] = 0.0;
         loop_sums<NW>(sh, acc, cx.want_kkt, lane, wave);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (!QREG) fetch_q(y0);  // of the next iteration
         lds_barrier();
         if (wave == 0)
@@ -453,7 +454,7 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
         kkt = wave_max_all(kkt);
         if (lane == 0) sh.red[4][wave] = kkt;
         __syncthreads();
-        double *ex = A.ex + (int64_t)NPART * slot_ld * (e + 1);
+        double *ex = A.ex + sum_words(nwg) * (e + 1);
         if (wave == 0) {
             kkt = 0.0;
 #pragma unroll
