@@ -37,6 +37,7 @@ def _units():
         for rows in (1, 2, 4, 8):
             units.append((os.path.join(CSRC, "img_loop_inst.hip"), f"img_loop_{s}_{rows}.o",
                           [f"-DPASS_S={s}", f"-DLOOP_ROWS={rows}"]))
+        units.append((os.path.join(CSRC, "grid_loop_inst.hip"), f"grid_loop_{s}.o", [f"-DPASS_S={s}"]))
         units.append((os.path.join(CSRC, "grid_inst.hip"), f"grid_{s}.o", [f"-DPASS_S={s}"]))
         units.append((os.path.join(CSRC, "img_inst.hip"), f"img_{s}.o", [f"-DPASS_S={s}"]))
     units.append((os.path.join(CSRC, "engine.hip"), "engine.o", []))

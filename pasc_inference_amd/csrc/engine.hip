@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "img_kernels.h"
+#include "grid_loop.h"
 #include "img_loop.h"
 #include "loop_kernels.h"
 #include "project_kernels.h"
@@ -55,6 +56,8 @@ int launch_pass_img_double(int K, const ImgArgs &a, int grid, int pd, hipStream_
 PASC_IMG_LOOP(float, 1) PASC_IMG_LOOP(float, 2) PASC_IMG_LOOP(float, 4) PASC_IMG_LOOP(float, 8)
 PASC_IMG_LOOP(double, 1) PASC_IMG_LOOP(double, 2) PASC_IMG_LOOP(double, 4) PASC_IMG_LOOP(double, 8)
 #undef PASC_IMG_LOOP
+int launch_grid_loop_float(int K, const GridLoopArgs &a, int nwg, int npt, hipStream_t s);
+int launch_grid_loop_double(int K, const GridLoopArgs &a, int nwg, int npt, hipStream_t s);
 int launch_loop_1d_float_4_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
 int launch_loop_1d_float_8_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
 int launch_loop_1d_double_4_(int K, const LoopArgs &a, int nwg, int chunk, hipStream_t s);
@@ -630,11 +633,12 @@ static int img_data_terms(Engine &e, const void *x, S *q) {
     return PASC_OK;
 }
 
-// The persistent loop of a phase (loop_kernels.h, img_loop.h): how many workgroups of how many
-// waves with how many steps per lane or rows per wave, or nwg = 0 when the problem does not run it.
+// The persistent loop of a phase (loop_kernels.h, img_loop.h, grid_loop.h): how many workgroups of
+// how many waves with how many steps per lane, rows per wave or nodes per thread, or nwg = 0 when the problem does not run it.
 struct LoopPlan {
     int nwg = 0, nw = 0, chunk = 0, tpw = 0, ntiles = 0;
     int rows = 0, nct = 0;  // images: rows per wave, tiles across
+    int npt = 0, brick[3] = {0, 0, 0}, nbrick[3] = {0, 0, 0};  // grids: nodes per thread, bricks
     int64_t epoch_words = 0, edge_words = 0;
 };
 
@@ -691,13 +695,71 @@ static void img_loop_plan(const Engine &e, bool f64, int n_cu, LoopPlan &pl) {
     }
 }
 
-static LoopPlan loop_plan(const Engine &e, bool f64) {
+// T > 1 frames of an image on the implicit 4-neighbour grid: the bricks of the least cost, in units of
+// 0.1 us at FP64: 0.4 K us per wave's worth of nodes on a SIMD, 2 us for the sums of a full chip, 0.3
+// us per 512 nodes around the brick.  (3 frames of 9 x 9 in 1 / 4 / 16 / 243 bricks: 4.7 / 5.0 / 5.6 / 7.0
+// us per iteration; 20 of 20 x 20 in 4 / 16 / 64 / 250: 12.4 / 6.8 / 6.8 / 7.5.)
+static void find_bricks(const GraphGeo &g, int K, int64_t tile, int n_cu, int32_t (&brick)[3]) {
+    const int64_t W = g.width, H = g.R / W, most = (int64_t)4 * GRID_LOOP_NT * n_cu;
+    if (W > most || H > most || g.T > most || W * H > most || W * H * g.T > most) return;
+    auto cut = [](int64_t n, int64_t parts) { return (n + parts - 1) / parts; };
+    int64_t best = 0;
+    for (int64_t nx = 1; nx <= std::min<int64_t>(W, n_cu); nx++) {
+        const int64_t bx = cut(W, nx);
+        if (nx > 1 && bx == cut(W, nx - 1)) continue;
+        for (int64_t ny = 1; ny <= std::min<int64_t>(H, n_cu / nx); ny++) {
+            const int64_t by = cut(H, ny);
+            if (ny > 1 && by == cut(H, ny - 1)) continue;
+            for (int64_t nt = 1; nt <= std::min<int64_t>(g.T, n_cu / (nx * ny)); nt++) {
+                const int64_t bt = cut(g.T, nt), own = bx * by * bt;
+                const int64_t around = 2 * bx * by + 2 * (bx + by) * (bt + 2);
+                if (own > 4 * GRID_LOOP_NT || around > GRID_LOOP_HPT * GRID_LOOP_NT ||
+                    (bx + 2) * (by + 2) * (bt + 2) > tile)
+                    continue;
+                const int64_t cost = 4 * K * cut(own, 4 * WAVE) + 20 * nx * ny * nt / n_cu + 3 * around / 512;
+                if (brick[0] && cost >= best) continue;
+                best = cost;
+                brick[0] = (int32_t)bx;
+                brick[1] = (int32_t)by;
+                brick[2] = (int32_t)bt;
+            }
+        }
+    }
+}
+
+static void grid_loop_plan(Engine &e, bool f64, int n_cu, LoopPlan &pl) {
+    const GraphGeo &g = e.geo;
+    const int K = e.h_desc[0].K, KS = K >= 2 ? K - 1 : K;
+    if (g.T < 2 || g.width <= 0 || g.ptr || g.R % g.width != 0) return;
+    int32_t(&brick)[3] = e.brick[f64 ? 1 : 0];
+    if (!e.bricks_found[f64 ? 1 : 0])
+        find_bricks(g, K, f64 ? grid_loop_tile<double>(K) : grid_loop_tile<float>(K), n_cu, brick);
+    e.bricks_found[f64 ? 1 : 0] = true;
+    if (brick[0] == 0) return;
+    const int64_t dim[3] = {g.width, g.R / g.width, g.T};
+    int64_t own = 1;
+    pl.nwg = 1;
+    for (int i = 0; i < 3; i++) {
+        pl.brick[i] = brick[i];
+        pl.nbrick[i] = (int)((dim[i] + brick[i] - 1) / brick[i]);
+        pl.nwg *= pl.nbrick[i];
+        own *= brick[i];
+    }
+    pl.npt = own <= GRID_LOOP_NT ? 1 : own <= 2 * GRID_LOOP_NT ? 2 : 4;
+    pl.epoch_words = sum_words(pl.nwg);
+    pl.edge_words = (int64_t)IMG_SETS * pl.nwg * own * KS;
+}
+
+static LoopPlan loop_plan(Engine &e, bool f64) {
     LoopPlan pl;
     if (e.n_inst != 1 || e.profile || e.shape_pinned) return pl;
     const InstDesc &d = e.h_desc[0];
     const int n_cu = std::max(e.ctx->n_cu, 1);
-    if (engine_is_image(e)) img_loop_plan(e, f64, n_cu, pl);
-    if (e.stencil != STENCIL_TIME) return pl;
+    if (e.stencil != STENCIL_TIME) {
+        if (engine_is_image(e)) img_loop_plan(e, f64, n_cu, pl);
+        else grid_loop_plan(e, f64, n_cu, pl);
+        return pl;
+    }
     switch (d.K) {
 #define PASC_LK(KK)                                        \
     case KK:                                               \
@@ -741,7 +803,9 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
     const int K = e.h_desc[0].K;
     const int need_f = ph.sp.fx_identity ? 0 : 1;
     // a residual that no stop test reads is only reported: it is formed for the last iterate
-    const int kkt_last = !ph.sp.fp32_phase && ph.kkt_every <= 1 && !(ph.sp.stop_mask & PASC_STOP_KKT);
+    // (graph kernels: their residual is formed in every pass, whatever kkt_every)
+    const int kkt_last = !ph.sp.fp32_phase && (ph.kkt_every <= 1 || pl.npt > 0) &&
+                         !(ph.sp.stop_mask & PASC_STOP_KKT);
     if (img && !e.d_q[b]) HIP_TRY(hipMalloc(&e.d_q[b], (ph.f64 ? 8 : 4) * (size_t)e.state_elems));
     for (bool fresh = true; passes < max_passes; fresh = false) {
         const int n = std::min(epochs, max_passes - passes);
@@ -749,7 +813,26 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
         if ((rc = prepare(e, (uint64_t *)ex, sums + pl.edge_words))) return rc;
         flags[0] = 1;
         flags[1] = 0;
-        if (img) {
+        if (pl.npt > 0) {
+            GridLoopArgs a{};
+            a.p = GridArgs{g0, g1, g64 ? e.d_dir64[0] : e.d_dir[0], g64 ? e.d_dir64[1] : e.d_dir[1], x,
+                           e.d_desc, nullptr, nullptr, GroupView{}, e.geo};
+            a.state = e.d_state;
+            a.sp = ph.sp;
+            a.ex = (double *)ex;
+            a.edges = (double *)ex + sums;
+            a.out = e.h_state;
+            a.flags = flags;
+            a.bx = pl.brick[0];
+            a.by = pl.brick[1];
+            a.bt = pl.brick[2];
+            a.nx = pl.nbrick[0];
+            a.ny = pl.nbrick[1];
+            a.epochs = n;
+            a.kkt_last = kkt_last;
+            rc = ph.f64 ? launch_grid_loop_double(K, a, pl.nwg, pl.npt, s)
+                        : launch_grid_loop_float(K, a, pl.nwg, pl.npt, s);
+        } else if (img) {
             if (fresh) rc = ph.f64 ? img_data_terms<double>(e, x, (double *)e.d_q[1])
                                    : img_data_terms<float>(e, x, (float *)e.d_q[0]);
             if (rc) return rc;
