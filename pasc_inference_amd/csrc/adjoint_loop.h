@@ -5,7 +5,9 @@
 // took 55 us there, 26 + 20 us of it for the vectors at the rate of the last-level cache.  Here a
 // wave owns 64 x CH consecutive steps, r and p in registers and lambda in LDS, so a step costs
 // its arithmetic and two exchanges of one sum between the workgroups (exchange.h; see
-// loop_kernels.h for the scheme and the cooperative launch).  The neighbouring waves' edge values
+// loop_kernels.h for the scheme and the cooperative launch): 7.4 us, about 2 us of it each
+// exchange (10 us with the sums in one copy, barriers that waited for the edges' stores too and
+// lambda advanced before r'r was published).  The neighbouring waves' edge values
 // of p are not exchanged: each wave keeps copies and advances them with the edges of r, which
 // travel with r'r.
 // A lane holds up to 8 steps for K <= 4 (r, p and q: 48 doubles at K = 3 and 8 steps, within the
@@ -45,7 +47,7 @@ __host__ __device__ constexpr int64_t adj_open_words(int nwg) {
 }
 template <int K>
 __host__ __device__ constexpr int64_t adj_epoch_words(int nwg) {
-    return (int64_t)slot_stride(nwg) * 2 + (int64_t)nwg * 2 * K;
+    return (int64_t)slot_stride(nwg) * 2 * SUM_COPIES + (int64_t)nwg * 2 * K;
 }
 
 // P applied to the K values of one step (free set in the low K bits of fr)
@@ -88,6 +90,15 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
             }
         }
     };
+    // the sum of a CG step: in SUM_COPIES rows, each workgroup reading one (see exchange.h)
+    auto publish_step = [&](double *rows) {
+        lds_barrier();
+        if (wave == 0) {
+            const double s = wave_sum_all(lane < NW ? red[0][lane] : 0.0);
+            if (lane < SUM_COPIES) store_coherent(rows + (int64_t)lane * sld + wg, s);
+        }
+    };
+    const int64_t copy = (int64_t)(wg % SUM_COPIES) * sld;
     // the wave's edge steps of v to LDS and, at the workgroup's ends, to the exchange area
     auto put_edges = [&](int par, const double(&v)[K][CH], double *ex_edges) {
         if (lane == 0) {
@@ -209,7 +220,7 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
 
     for (int e = 0; e < A.epochs && !stop; e++) {
         double *ex = A.ex + adj_open_words<K>(nwg) + adj_epoch_words<K>(nwg) * e;
-        double *ex_edges = ex + 2 * (int64_t)sld;
+        double *ex_r = ex + SUM_COPIES * (int64_t)sld, *ex_edges = ex_r + SUM_COPIES * (int64_t)sld;
         const int par = e & 1;
         // q = P A p and p'q
         double q[K][CH], pq = 0.0;
@@ -242,35 +253,39 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
         }
         pq = wave_sum_all(pq);
         if (lane == 0) red[0][wave] = pq;
-        publish(ex, 1);
+        publish_step(ex);
         if (wave == 0) {
-            pq = await_sum(ex, nwg, lane, lost);
+            pq = await_sum(ex + copy, nwg, lane, lost);
             if (lane == 0) {
                 bc[0] = rr / pq;
                 bc[1] = pq > 0.0 ? 0.0 : 1.0;  // p in the null space of P A P: the system is solved
             }
         }
-        __syncthreads();
+        lds_barrier();
         const double step = bc[0];
         stop = bc[1] != 0.0;
         if (stop) break;
-        // lambda += step p, r -= step q, r'r
+        // r -= step q, r'r
         double rn = 0.0;
 #pragma unroll
         for (int k = 0; k < K; k++)
 #pragma unroll
             for (int c = 0; c < CH; c++) {
-                my_lam[k * LROW + c] += step * p[k][c];
                 r[k][c] -= step * q[k][c];
                 rn += r[k][c] * r[k][c];
             }
         put_edges(par ^ 1, r, ex_edges);
         rn = wave_sum_all(rn);
         if (lane == 0) red[0][wave] = rn;
-        publish(ex + sld, 1);
+        publish_step(ex_r);
+        // lambda += step p while the sums travel
+#pragma unroll
+        for (int k = 0; k < K; k++)
+#pragma unroll
+            for (int c = 0; c < CH; c++) my_lam[k * LROW + c] += step * p[k][c];
         if (wave == NW - 1) get_edges(par ^ 1, ex_edges);
         if (wave == 0) {
-            rn = await_sum(ex + sld, nwg, lane, lost);
+            rn = await_sum(ex_r + copy, nwg, lane, lost);
             const double b = rn / rr;
             rr = rn;
             it++;
@@ -280,7 +295,7 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
                 bc[1] = done ? 1.0 : 0.0;
             }
         }
-        __syncthreads();
+        lds_barrier();
         const double b = bc[0];
         stop = bc[1] != 0.0;
 #pragma unroll

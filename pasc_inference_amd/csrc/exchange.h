@@ -14,6 +14,12 @@ constexpr int64_t LOOP_EXCHANGE_BYTES = 16 << 20;  // exchange area of a launch 
 // workgroups' values as 512 contiguous bytes).
 __host__ __device__ constexpr int slot_stride(int nwg) { return (nwg + 15) / 16 * 16; }
 
+// Every workgroup publishes its sums SUM_COPIES times and reads one copy: the workgroups that meet
+// at one cache line, where they queue, are as many times fewer.  us per iteration with 1 / 2 / 4 / 8
+// copies: 250 x 150 image 6.4 / 5.6 / 5.4 / 5.3, 60 frames of 64 x 48 11.6 / 11.0 / 10.7 / 10.6,
+// 1024 x 1024 13.2 / 12.6 / 12.4 / 12.4, series of 2.5e5 steps 5.6 / 5.5 / 5.5 / 5.8.
+constexpr int SUM_COPIES = 4;
+
 // ---- wave-wide sums by lane swaps and DPP (VALU moves; no LDS round trips) -------------------
 template <int CTRL>
 __device__ __forceinline__ double dpp_from(double v) {

@@ -56,11 +56,6 @@ constexpr bool loop_has_chunk(bool f64, int K, int ch) {
     return f64 ? ch == 2 || (ch == 4 && K <= 4) : ch == 4;
 }
 
-// Every workgroup publishes its sums SUM_COPIES times and reads one copy: the workgroups that meet
-// at one cache line, where they queue, are as many times fewer.  us per iteration with 1 / 2 / 4 / 8
-// copies: 250 x 150 image 6.4 / 5.6 / 5.4 / 5.3, 60 frames of 64 x 48 11.6 / 11.0 / 10.7 / 10.6,
-// 1024 x 1024 13.2 / 12.6 / 12.4 / 12.4, series of 2.5e5 steps 5.6 / 5.5 / 5.5 / 5.8.
-constexpr int SUM_COPIES = 4;
 __host__ __device__ constexpr int64_t sum_words(int nwg) {
     return (int64_t)SUM_COPIES * NPART * slot_stride(nwg);
 }
