@@ -237,9 +237,9 @@ int engine_alloc(Engine &e, Ctx *ctx, int precision, int stencil, int32_t grid_w
     e.sh[1] = PassShape{256, 2, 0, 2048, 1};
     if (e.n_inst == 1 && stencil == STENCIL_TIME) {
         // One series beyond what the persistent loop holds: one-wave workgroups, the next tile
-        // staged.  us per pass at T = 1e7 against the shapes above: FP64 K = 2 / 3 / 4 58 / 93 /
-        // 136 (71 / 112 / 151), K = 8 (shorter chunk) 395 (443), FP32 41 / 53 / 76 / 244 (44 / 59
-        // / 82 / 273); at T = 2e6 24 / 32 / 41 / 100 (30 / 36 / 44 / 109).  The FP32 chunk stays 4:
+        // staged.  us per pass at T = 1e7 against the shapes above: FP64 K = 2 / 3 / 4 52 / 86 /
+        // 125 (71 / 112 / 151), K = 8 (shorter chunk) 388 (443), FP32 K = 3 / 4 49 / 69 (59 / 82).
+        // 2048 to 12288 slots differ by 2 %.  The FP32 chunk stays 4:
         // a thread's FP32 sums cover its chunk, so it fixes their rounding.
         const bool wide = descs[0].K > 4;
         e.sh[0] = PassShape{64, 4, 1, 4096, 1};
@@ -253,6 +253,9 @@ int engine_alloc(Engine &e, Ctx *ctx, int precision, int stencil, int32_t grid_w
     }
     int64_t se = 0;
     for (auto &d : descs) se = std::max(se, d.goff + (int64_t)d.K * d.ld);
+    int64_t touched = 0;
+    for (auto &d : descs) touched += 8 * d.ld * (2 * (int64_t)(d.K >= 2 ? d.K - 1 : d.K) + 1);
+    e.stores_nt = pass_stores_nt(touched);
     e.state_elems = round_up(std::max<int64_t>(se, 64), 64);
     const size_t es = precision == PASC_FP32_BULK ? 4 : 8;
     for (int b = 0; b < 2; b++) {
@@ -532,7 +535,7 @@ static int enqueue_iteration(Engine &e, const PhaseCfg &ph, const std::vector<in
             const void *bb = ph.f64 ? e.d_b64 : e.d_b32;
             PassArgs a{g0, g1, x, e.d_desc, e.d_state, e.d_part, gv, ph.kkt_every,
                        ph.sp.fx_identity ? 0 : 1, bb, ph.sp, fused ? e.d_done : nullptr,
-                       e.h_poll, e.d_dirty};
+                       e.h_poll, e.d_dirty, ph.f64 && e.stores_nt ? 1 : 0};
             const PassShape &sh = e.sh[ph.f64 ? 1 : 0];
             rc = launch_pass_1d(ph.f64, g.K, a, grids[gi], sh.block, sh.chunk, sh.prefetch, s);
         } else if (img) {

@@ -169,6 +169,7 @@ struct Engine {
     bool tiled_scan = false;             // a single problem's tile enumeration is on the device
     PassShape sh[2];                     // [0] FP32 phase of FP32-bulk, [1] every FP64 pass
     int32_t brick[2][3] = {};            // a grid's bricks in the persistent loop (0: none), by type,
+    bool stores_nt = false;              // FP64 1-D passes store gamma nontemporally
     bool bricks_found[2] = {};           //   found with the first solve
     bool shape_pinned = false;           // the caller pinned sh: the tiled passes run it
     int grid_cap = 0;                    // persistent grid cap (0: 32 blocks per CU)

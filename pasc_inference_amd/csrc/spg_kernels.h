@@ -43,7 +43,16 @@ struct PassArgs {
                         // the step
     int32_t *running;   // pinned host word: 0 once a single problem has stopped
     int32_t *dirty;     // set when an instance stops (the batch's tile scan rebuilds)
+    int32_t nt;         // FP64: nontemporal stores of gamma_i (see pass_stores_nt)
 };
+
+// FP64 passes store gamma_i nontemporally where what a pass touches (two sets of K - 1 rows and
+// the data) exceeds the last-level cache, and leave it there for the next pass where it fits.  us per
+// pass, nontemporal / plain: T = 1e7 (400 MB at K = 3, 560 at 4) 86 / 93 and 125 / 130; T = 1e7, K = 2
+// (240 MB) 60 / 52; T = 3e6 and 2e6, K = 3 39 / 34 and 31 / 27.  FP32 passes were slower with them at
+// T = 1e7 (49.5 -> 53.8 us).
+constexpr int64_t LAST_LEVEL_CACHE = int64_t(256) << 20;
+constexpr bool pass_stores_nt(int64_t bytes) { return bytes > LAST_LEVEL_CACHE; }
 
 template <int CH>
 constexpr int halo_threads() { return (3 + CH - 1) / CH; }
@@ -157,7 +166,7 @@ struct TileCtx {
     const uint8_t *heldout;
     C alpha, bscale, s_kkt, a_apply, b_apply, a_dir;
     C theta[K];
-    bool first, need_f, want_kkt;
+    bool first, need_f, want_kkt, nt;
 };
 
 template <typename S, typename C, int K>
@@ -185,6 +194,7 @@ __device__ __forceinline__ void make_tile_ctx(const PassArgs &A, const InstDesc 
     for (int k = 0; k < K; k++) c.theta[k] = uni(C(D.theta[k]));
     c.first = uni(st.first) != 0;
     c.need_f = A.need_f || c.first;
+    c.nt = A.nt != 0;
     const int it = uni(st.it);
     c.want_kkt = (it % (A.kkt_every > 0 ? A.kkt_every : 1)) == 0;
 }
@@ -240,6 +250,31 @@ __device__ __forceinline__ void stage_read(const S *stage, int r, C (&v)[CH]) {
 #pragma unroll
     for (int q = 0; q < CH / VW; q++) {
         const typename VT::type vec = *reinterpret_cast<const typename VT::type *>(row + q * VW);
+#pragma unroll
+        for (int i = 0; i < VW; i++) v[q * VW + i] = C(VT::get(vec, i));
+    }
+}
+
+// The same through an explicit LDS read and its wait: before a plain read of memory that
+// asynchronous copies write the compiler drains every outstanding vector memory operation, the
+// previous tile's stores included.
+template <typename S, typename C, int K, int CH, int NT>
+__device__ __forceinline__ void stage_read_now(const S *stage, int r, C (&v)[CH]) {
+    using VT = V16<S>;
+    constexpr int VW = VT::n, N = CH / VW;
+    static_assert(N == 1 || N == 2, "one or two vectors a row");
+    typedef float vec16 __attribute__((ext_vector_type(4)));
+    const S *row = stage + (size_t)r * Stage<S, K, CH, NT>::ROW + threadIdx.x * CH;
+    const uint32_t at = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) S *)row;
+    vec16 w[N];
+    if constexpr (N == 2)
+        asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:16\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(w[0]), "=&v"(w[N - 1]) : "v"(at) : "memory");
+    else
+        asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w[0]) : "v"(at) : "memory");
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        const typename VT::type vec = __builtin_bit_cast(typename VT::type, w[q]);
 #pragma unroll
         for (int i = 0; i < VW; i++) v[q * VW + i] = C(VT::get(vec, i));
     }
@@ -419,13 +454,15 @@ __device__ __forceinline__ void pass_levels(const TileCtx<S, C, K> &cx, int64_t 
     if (!owner) p = LevelSums<C>{};
 }
 
-// STAGED: the tile's gamma and data rows were copied into the LDS stage (interior tiles
-// only).  next: a callable run once every thread has taken the stage's rows into registers
+// STAGED: the tile's gamma and data rows were copied into the LDS stage (interior tiles of passes
+// after the first).  PLAIN: also no held-out steps and no explicit b, so that no load of device memory
+// stands in the tile's code (the compiler would wait for it, and for the last tile's stores, where
+// it is not even taken).  next: a callable run once every thread has taken the stage's rows into registers
 // (it issues the copies of the slot's next tile into the stage).
-template <typename S, typename C, int K, int CH, int NT, bool INT, bool STAGED, typename Next>
+template <typename S, typename C, int K, int CH, int NT, bool INT, bool STAGED, bool PLAIN, typename Next>
 __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chunk, C *lds_x,
                                              double (&acc)[NPART], const S *stage, Next next) {
-    static_assert(!STAGED || INT, "only interior tiles are staged");
+    static_assert((!STAGED || INT) && (!PLAIN || STAGED), "only interior tiles are staged");
     constexpr int HT = halo_threads<CH>();
     constexpr int TILE = tile_steps<NT, CH>();
     const int64_t T = cx.T;
@@ -441,7 +478,7 @@ __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chu
     // data term q = -b of every step of the chunk, formed once for the two levels that use it:
     // bscale*(x - theta_k)^2 (zero when held out or outside [0,T)), or read from an explicit b
     C Q[K][CH];
-    if (cx.br) {
+    if (!PLAIN && cx.br) {
 #pragma unroll
         for (int k = 0; k < K; k++) {
             load_chunk<S, C, CH, INT>(cx.br + k * ld, t0, T, ld, Q[k]);
@@ -450,7 +487,9 @@ __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chu
         }
     } else {
         C X[CH];
-        if (STAGED)
+        if (PLAIN)
+            stage_read_now<S, C, K, CH, NT>(stage, KS, X);
+        else if (STAGED)
             stage_read<S, C, K, CH, NT>(stage, KS, X);
         else
             load_chunk<S, C, CH, INT>(cx.xr, t0, T, ld, X);
@@ -460,7 +499,7 @@ __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chu
             const int64_t t = t0 + c;
             obs[c] = INT || (t >= 0 && t < T);
         }
-        if (cx.heldout) {
+        if (!PLAIN && cx.heldout) {
 #pragma unroll
             for (int c = 0; c < CH; c++)
                 if (obs[c]) obs[c] = cx.heldout[t0 + c] == 0;
@@ -470,14 +509,16 @@ __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chu
     C G[K][CH], G1[K][CH];
 #pragma unroll
     for (int k = 0; k < KS; k++) {
-        if (STAGED)
+        if (PLAIN)
+            stage_read_now<S, C, K, CH, NT>(stage, k, G[k]);
+        else if (STAGED)
             stage_read<S, C, K, CH, NT>(stage, k, G[k]);
         else
             load_chunk<S, C, CH, INT>(src + k * ld, t0, T, ld, G[k]);
     }
     if (KS < K) {
         // gamma_0 may lie off the simplex: its last row is read (first passes are never staged)
-        if (cx.first)
+        if (!STAGED && cx.first)
             load_chunk<S, C, CH, INT>(src + (K - 1) * ld, t0, T, ld, G[K - 1]);
         else
             rebuild_last_row<C, K, CH, INT>(t0, T, G);
@@ -497,30 +538,35 @@ __device__ __forceinline__ void pass_tile_1d(const TileCtx<S, C, K> &cx, int chu
         G1, p);
     if (owner) {
         // store gamma_i
-        using VT = V16<S>;
-        constexpr int VW = VT::n;
+        auto store = [&](auto nontemporal) {
+            using VT = V16<S>;
+            constexpr int VW = VT::n;
 #pragma unroll
-        for (int k = 0; k < KS; k++) {
+            for (int k = 0; k < KS; k++) {
 #pragma unroll
-            for (int q = 0; q < CH / VW; q++) {
-                const int64_t t = t0 + q * VW;
-                if (INT || t + VW <= T) {
-                    typename VT::type vec;
+                for (int q = 0; q < CH / VW; q++) {
+                    const int64_t t = t0 + q * VW;
+                    if (INT || t + VW <= T) {
+                        typename VT::type vec;
 #pragma unroll
-                    for (int i = 0; i < VW; i++) VT::set(vec, i, S(G1[k][q * VW + i]));
-                    // FP64 rows: nontemporal stores (95.8 -> 87.1 us per pass at
-                    // T = 1e7, K = 3); the FP32 pass was slower with them (49.5 -> 53.8 us)
-                    if constexpr (sizeof(S) == 8)
-                        store_nt(reinterpret_cast<typename VT::type *>(dst + k * ld + t), vec);
-                    else
-                        *reinterpret_cast<typename VT::type *>(dst + k * ld + t) = vec;
-                } else {
+                        for (int i = 0; i < VW; i++) VT::set(vec, i, S(G1[k][q * VW + i]));
+                        typename VT::type *to = reinterpret_cast<typename VT::type *>(dst + k * ld + t);
+                        if constexpr (decltype(nontemporal)::value)
+                            store_nt(to, vec);
+                        else
+                            *to = vec;
+                    } else {
 #pragma unroll
-                    for (int i = 0; i < VW; i++)
-                        if (t + i < T) dst[k * ld + t + i] = S(G1[k][q * VW + i]);
+                        for (int i = 0; i < VW; i++)
+                            if (t + i < T) dst[k * ld + t + i] = S(G1[k][q * VW + i]);
+                    }
                 }
             }
-        }
+        };
+        if (sizeof(S) == 8 && cx.nt)
+            store(std::true_type{});
+        else
+            store(std::false_type{});
     }
     const double dd = (double)p.dd;
     acc[0] += dd;
@@ -651,6 +697,7 @@ __global__ __launch_bounds__(NT) void spg_pass_1d(PassArgs A) {
         bool staged = false;  // the current tile's rows are in the stage
         // a first pass reads all K rows of gamma_0 and runs unstaged
         const bool can_stage = USE_STAGE && !cx.first;
+        const bool plain = !cx.br && !cx.heldout;
         if (can_stage && tile_is_interior<S, C, K, CH, NT>(first_tile, cx.T)) {
             stage_issue<S, C, K, CH, NT>(cx, first_tile, stage);
             __builtin_amdgcn_s_waitcnt(0);
@@ -666,15 +713,27 @@ __global__ __launch_bounds__(NT) void spg_pass_1d(PassArgs A) {
             auto issue = [&]() {
                 if (stage_next) stage_issue<S, C, K, CH, NT>(cx, nt, stage);
             };
-            if (USE_STAGE && staged)
-                pass_tile_1d<S, C, K, CH, NT, true, true>(cx, tile, lds_x, acc, stage, issue);
-            else if (tile_is_interior<S, C, K, CH, NT>(tile, cx.T))
-                pass_tile_1d<S, C, K, CH, NT, true, false>(cx, tile, lds_x, acc, stage, issue);
+            // The copies of the next tile must have arrived, the stores behind them need not: an
+            // interior tile ends with its KS * CH / VW stores, and vector memory operations complete
+            // in order, so the wait leaves that many outstanding.  With this and without the waits
+            // that PLAIN avoids, us per pass at T = 1e7: FP64 K = 3 / 4 93 / 136 -> 86 / 125, FP32
+            // 53 / 76 -> 49 / 70.
+            constexpr int STORES = stored_rows<K>() * (CH / V16<S>::n);
+            const bool interior = tile_is_interior<S, C, K, CH, NT>(tile, cx.T);
+            if (USE_STAGE && staged && plain)
+                pass_tile_1d<S, C, K, CH, NT, true, true, true>(cx, tile, lds_x, acc, stage, issue);
+            else if (USE_STAGE && staged)
+                pass_tile_1d<S, C, K, CH, NT, true, true, false>(cx, tile, lds_x, acc, stage, issue);
+            else if (interior)
+                pass_tile_1d<S, C, K, CH, NT, true, false, false>(cx, tile, lds_x, acc, stage, issue);
             else
-                pass_tile_1d<S, C, K, CH, NT, false, false>(cx, tile, lds_x, acc, stage, issue);
+                pass_tile_1d<S, C, K, CH, NT, false, false, false>(cx, tile, lds_x, acc, stage, issue);
             if (stage_next) {
-                __builtin_amdgcn_s_waitcnt(0);
-                __syncthreads();
+                if (interior)
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STORES) : "memory");
+                else
+                    __builtin_amdgcn_s_waitcnt(0);
+                lds_barrier();
             }
             staged = stage_next;
         }
