@@ -356,7 +356,7 @@ def run_graph_c5(args, ctx):
                 time_s=float(np.mean(times)), iterations=int(r.it), kkt=float(r.kkt),
                 us_per_iteration=float(np.mean(times)) / (r.it + 1) * 1e6,
                 label_accuracy=acc, pass_us=pass_s * 1e6, own_min_gbps=own / pass_s / 1e9,
-                kernels="spg_pass_img (one launch per iteration, step in its last workgroup)",
+                kernels="img_loop (time_s); spg_pass_img (pass_us: one launch per iteration)",
                 fp32_bulk=dict(time_s=float(np.mean(times32)), it_fp32=int(r32.it_fp32),
                                it_fp64=int(r32.it_fp64), kkt=float(r32.kkt),
                                pass_us_fp32=pass32_s * 1e6, pass_us_fp64=polish_s * 1e6,
