@@ -47,16 +47,18 @@ struct Lanes64 {
     }
 };
 
-constexpr double PROJ_LOW = -1e308;  // below any value; also what a lane without a value holds
+constexpr double PROJ_LOW = -1e308;  // what a place without a value holds: never above a threshold
 
-// Threshold of a block whose values fn(i), i < n, each lane of the group enumerates; false: the
-// block is feasible.  (Lanes past the block, and NaN, take no part: their values compare false.)
+// Threshold of a block whose values fn(i), i < nv <= n, each lane of the group enumerates; false:
+// the block is feasible.  Places from nv on hold PROJ_LOW.  They are told by their index: an
+// entry of the block may have that value, and is negative like any other.  In the search their
+// values, and NaN, compare false.
 template <typename G, typename F>
-__device__ __forceinline__ bool block_tau(int n, int K, F fn, double &tau) {
+__device__ __forceinline__ bool block_tau(int n, int nv, int K, F fn, double &tau) {
     double s = 0.0, mx = PROJ_LOW, neg = 0.0;
     for (int i = 0; i < n; i++) {
         const double v = fn(i);
-        if (v == PROJ_LOW) continue;
+        if (i >= nv) continue;
         s += v;
         neg += v < 0.0 ? 1.0 : 0.0;
         mx = v > mx ? v : mx;
@@ -94,14 +96,12 @@ __global__ __launch_bounds__(256) void project_group(S *x, int64_t nblocks, int 
     const int l = threadIdx.x & (LANES - 1);
     const bool in = b < nblocks;  // (every lane stays for the wave's ballots)
     S *xb = x + (in ? b : 0) * K;
+    const int nv = in ? (K - l + LANES - 1) / LANES : 0;
     double y[R];
 #pragma unroll
-    for (int i = 0; i < R; i++) {
-        const int k = l + i * LANES;
-        y[i] = in && k < K ? (double)xb[k] : PROJ_LOW;
-    }
+    for (int i = 0; i < R; i++) y[i] = i < nv ? (double)xb[l + i * LANES] : PROJ_LOW;
     double tau;
-    const bool project = block_tau<G>(R, K, [&](int i) { return y[i]; }, tau);
+    const bool project = block_tau<G>(R, nv, K, [&](int i) { return y[i]; }, tau);
     if (!in || !project) return;
 #pragma unroll
     for (int i = 0; i < R; i++) {
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256) void project_lane(S *x, int64_t nblocks, int K
 #pragma unroll
     for (int k = 0; k < KM; k++) y[k] = in && k < K ? (double)xb[k * ld] : PROJ_LOW;
     double tau;
-    const bool project = block_tau<Lanes1>(KM, K, [&](int i) { return y[i]; }, tau);
+    const bool project = block_tau<Lanes1>(KM, in ? K : 0, K, [&](int i) { return y[i]; }, tau);
     if (!in || !project) return;
 #pragma unroll
     for (int k = 0; k < KM; k++) {
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void project_lane_mem(S *x, int64_t nblocks, i
     S *xb = x + (in ? b : 0);
     double tau;
     const bool project =
-        block_tau<Lanes1>(K, K, [&](int k) { return in ? (double)xb[k * ld] : PROJ_LOW; }, tau);
+        block_tau<Lanes1>(K, in ? K : 0, K, [&](int k) { return in ? (double)xb[k * ld] : PROJ_LOW; }, tau);
     if (!in || !project) return;
     for (int k = 0; k < K; k++) {
         const double v = (double)xb[k * ld] - tau;
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void project_wave_mem(S *x, int64_t nblocks, i
     S *xb = x + b * K;
     double tau;
     const bool project = block_tau<Lanes64>(
-        (K + WAVE - 1) / WAVE, K,
+        (K + WAVE - 1) / WAVE, (K - lane + WAVE - 1) / WAVE, K,
         [&](int i) {
             const int k = lane + i * WAVE;
             return k < K ? (double)xb[k] : PROJ_LOW;
