@@ -465,6 +465,13 @@ int engine_set_gamma(Engine &e, int inst, const double *g, int layout) {
                           e.precision == PASC_FP32_BULK, d.T, d.ld, d.K);
 }
 
+// Waits for what a call queued on the caller's stream: the library's own stream orders what follows,
+// but a caller may go on with another stream as soon as the call is back.
+static int settle(const Ctx *ctx) {
+    if (!ctx->own_stream) HIP_TRY(hipStreamSynchronize((hipStream_t)ctx->stream));
+    return PASC_OK;
+}
+
 // Explicit linear term of one instance (the QP's b as the reference's QPData holds it): stored
 // k-major like gamma, FP64 plus an FP32 copy for the FP32 phase.  b_host == nullptr returns the
 // instance to the data term formed from x and theta.
@@ -487,6 +494,8 @@ int engine_set_linear_term(Engine &e, int inst, const double *b_host, int layout
         hipLaunchKernelGGL((convert_kernel<double, float>), dim3((unsigned)((n + 255) / 256)),
                            dim3(256), 0, S_(e), (const double *)b64, b32, n);
         HIP_TRY(hipGetLastError());
+        arc = settle(e.ctx);
+        if (arc) return arc;
     }
     d.b64 = b64;
     d.b32 = b32;
@@ -1397,9 +1406,7 @@ int rows_fill_uniform(Ctx *ctx, void *rows, bool f32, int64_t T, int64_t ld, int
         hipLaunchKernelGGL((fill_rows_kernel<double>), grid, dim3(256), 0, s, (double *)rows, T, ld,
                            K, 1.0 / K);
     HIP_TRY(hipGetLastError());
-    // the library's own stream orders what follows; a caller may take an external one away
-    if (!ctx->own_stream) HIP_TRY(hipStreamSynchronize(s));
-    return PASC_OK;
+    return settle(ctx);
 }
 
 int engine_fill_uniform(Engine &e) {
