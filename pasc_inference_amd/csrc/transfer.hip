@@ -16,14 +16,12 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
-#include <deque>
-#include <memory>
 #include <functional>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 #include "device_common.h"
+#include "team.h"
 
 namespace pasc {
 
@@ -119,86 +117,7 @@ struct SlotPool {
 
 static SlotPool *const g_pool = new SlotPool[POOL_DEVICES];
 
-// Helper threads of the host copies, parked between transfers; started when first needed, ended
-// with the process's last context.
-class Team {
-    struct Job {
-        const std::function<void()> *fn = nullptr;
-        int running = 0;
-        bool closed = false;
-    };
-    std::mutex mu;
-    std::condition_variable wake, done;
-    std::deque<std::shared_ptr<Job>> queue;
-    std::vector<std::thread> threads;
-    int users = 0;
-    bool stop = false;
-
-    void loop() {
-        std::unique_lock<std::mutex> lk(mu);
-        for (;;) {
-            wake.wait(lk, [&] { return stop || !queue.empty(); });
-            if (stop) return;
-            std::shared_ptr<Job> j = queue.front();
-            queue.pop_front();
-            if (j->closed) continue;
-            j->running++;
-            lk.unlock();
-            (*j->fn)();
-            lk.lock();
-            if (--j->running == 0) done.notify_all();
-        }
-    }
-
-  public:
-    static constexpr int MOST = SLOTS - 1;
-
-    static int helpers() {
-        return std::min(MOST, std::max(1, (int)std::thread::hardware_concurrency() / 2) - 1);
-    }
-    void open() {
-        std::lock_guard<std::mutex> lk(mu);
-        users++;
-    }
-    void close() {
-        std::vector<std::thread> gone;
-        {
-            std::lock_guard<std::mutex> lk(mu);
-            if (--users > 0) return;
-            stop = true;
-            gone.swap(threads);
-        }
-        wake.notify_all();
-        for (auto &t : gone) t.join();
-        std::lock_guard<std::mutex> lk(mu);
-        stop = false;
-    }
-    // fn on this thread and on up to n helpers; back when every helper that started has ended.
-    // fn must not throw.
-    void run(int n, const std::function<void()> &fn) {
-        std::shared_ptr<Job> job;
-        if (n > 0) {
-            try {
-                job = std::make_shared<Job>();
-                job->fn = &fn;
-                std::lock_guard<std::mutex> lk(mu);
-                while ((int)threads.size() < std::min(n, helpers()) && !stop)
-                    threads.emplace_back([this] { loop(); });
-                for (int i = 0; i < n; i++) queue.push_back(job);
-            } catch (const std::exception &) {
-                // fewer helpers: this thread does the rest
-            }
-            if (n == 1) wake.notify_one();
-            else wake.notify_all();
-        }
-        fn();
-        if (job) {
-            std::unique_lock<std::mutex> lk(mu);
-            job->closed = true;
-            done.wait(lk, [&] { return job->running == 0; });
-        }
-    }
-};
+static_assert(Team::MOST == SLOTS - 1, "a slot for the calling thread and one for every helper");
 
 // never destroyed: parked threads end with the process when a context is still open then
 static Team &g_team = *new Team;
