@@ -343,10 +343,11 @@ typedef struct {
                                 polish.block == 0 derives it from main (chunk / 2) */
 } pasc_launch_shape;
 
-/* Pin the launch shapes of later solves (the iterate is kept).  Without a pinned shape a 1-D
- * problem whose iterate and data fit on the chip (about 1.5 million steps at K = 3 in FP64, 3
- * million in the FP32 phase) runs its iterations in one persistent launch instead, which has no
- * shape to choose; a pinned shape is always run. */
+/* Pin the launch shapes of later solves (the iterate is kept).  Without a pinned shape a single
+ * problem whose iterate and data fit on the chip (a series of about 1.6 million steps at K = 3 in
+ * FP64, 3.1 million in the FP32 phase; an image of 1024 x 1024) runs its iterations in one
+ * persistent launch instead, which has no shape to choose; a pinned shape is always run, also by
+ * a batch of one instance. */
 int pasc_set_launch_shape(pasc_problem *p, const pasc_launch_shape *shape);
 
 /* ---- autotuner ----
@@ -356,7 +357,9 @@ int pasc_set_launch_shape(pasc_problem *p, const pasc_launch_shape *shape);
  * the FP64 polish are tuned separately.
  * The choice is cached per context.  With a non-NULL cache_path, a choice recorded there for
  * the same key by an earlier process is reused without timing, and every call appends its
- * choice to the file (one JSON object per line). */
+ * choice to the file (one JSON object per line).
+ * A tuned shape is the passes' shape; it pins nothing: a problem that fits on the chip still runs
+ * the persistent launch.  pasc_set_launch_shape with the returned shape pins it. */
 int pasc_autotune(pasc_problem *p, const char *cache_path, pasc_launch_shape *shape);
 /* the same for a batch (all instances share one shape per phase) */
 int pasc_batch_autotune(pasc_batch *b, const char *cache_path, pasc_launch_shape *shape);

@@ -1041,10 +1041,13 @@ static void shapes_of(const Engine &e, const pasc_launch_shape &sh, PassShape &s
     }
 }
 
+// The caller's shape, pinned: later solves run it, and no persistent loop.
 static int set_shape(Engine &e, const pasc_launch_shape *shape) {
     PassShape s32, s64;
     shapes_of(e, *shape, s32, s64);
-    return engine_set_shape(e, s32, s64);
+    const int rc = engine_set_shape(e, s32, s64);
+    if (rc == PASC_OK) e.shape_pinned = true;
+    return rc;
 }
 
 // Autotune with the per-context and on-file caches (one JSON object per line, last match wins).
@@ -1122,9 +1125,7 @@ int pasc_set_launch_shape(pasc_problem *p, const pasc_launch_shape *shape) {
     if (!p || !shape) return fail(PASC_ERR_ARG, "set_launch_shape: NULL argument");
     int rc = use_device(p->ctx);
     if (rc) return rc;
-    rc = set_shape(p->e, shape);
-    if (rc == PASC_OK) p->e.shape_pinned = true;
-    return rc;
+    return set_shape(p->e, shape);
 }
 
 int pasc_autotune(pasc_problem *p, const char *cache_path, pasc_launch_shape *shape) {
