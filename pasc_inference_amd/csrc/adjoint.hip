@@ -320,7 +320,7 @@ struct AdjResult {
 };
 
 // One problem on the 1-D graph whose CG vectors fit on chip: the persistent launch (adjoint_loop.h).
-// *ran = false when it does not qualify or the launch is refused.
+// *ran = false when it does not qualify, the launch is refused or its workgroups lost each other.
 template <int K, int CH, int NW>
 static bool launch_adj_loop(const AdjLoopArgs &a, int nwg, hipStream_t s) {
     const void *fn = reinterpret_cast<const void *>(adj_loop<K, CH, NW>);
@@ -378,6 +378,7 @@ static int run_adj_loop(Engine &e, const InstDesc &D, const double *gam, const u
     a.ex = ex;
     a.epochs = epochs;
     a.maxit = cg_maxit;
+    a.rereads = e.ctx->wait_limit;
     for (a.resume = 0;; a.resume = 1) {
         const int64_t words = ow + ew * epochs;
         hipLaunchKernelGGL(fill_u64, dim3((unsigned)std::min<int64_t>((words + 255) / 256, 1024)),
@@ -390,7 +391,7 @@ static int run_adj_loop(Engine &e, const InstDesc &D, const double *gam, const u
                                                      : launch_adj_loop<K, CH, 8>(a, nwg, s);
         if (!ok) return PASC_OK;
         HIP_TRY(hipStreamSynchronize(s));
-        if (a.flags[1]) return fail(PASC_ERR_HIP, "adjoint: the workgroups lost each other");
+        if (a.flags[1]) return PASC_OK;  // the workgroups lost each other: nothing of it is used
         if (!a.flags[0]) break;
     }
     res.loss = a.out[0];

@@ -151,6 +151,12 @@ int pasc_ctx_set_stream(pasc_ctx *ctx, void *stream) {
     return PASC_OK;
 }
 
+int pasc_ctx_set_wait_limit(pasc_ctx *ctx, int32_t rereads) {
+    if (!ctx || rereads < 0) return fail(PASC_ERR_ARG, "ctx_set_wait_limit: bad arguments");
+    ctx->c.wait_limit = rereads > 0 ? rereads : WAIT_LIMIT;
+    return PASC_OK;
+}
+
 int pasc_ctx_synchronize(pasc_ctx *ctx) {
     if (!ctx) return fail(PASC_ERR_ARG, "ctx is NULL");
     HIP_TRY(hipStreamSynchronize((hipStream_t)ctx->c.stream));

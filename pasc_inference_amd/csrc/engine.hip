@@ -784,9 +784,13 @@ static LoopPlan loop_plan(Engine &e, bool f64) {
     return pl;
 }
 
-// Runs a phase's passes in the persistent loop; *ran = false when the problem does not qualify or
-// the launch is refused (the tiled passes then go on from the state as it is).
-static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, bool *ran) {
+// Runs a phase's passes in the persistent loop; *ran = false when the problem does not qualify, the
+// launch is refused or its workgroups lost each other.  The tiled passes then go on from the
+// state as it is, in the last case from where the launch began: its gamma (and directions) lie
+// in the buffers the launch does not write, its state in *began, which becomes the state to start
+// from.
+static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, bool *ran,
+                    InstState *began) {
     *ran = false;
     const LoopPlan pl = loop_plan(e, ph.f64);
     if (pl.nwg == 0) return PASC_OK;
@@ -822,6 +826,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
     for (bool fresh = true; passes < max_passes; fresh = false) {
         const int n = std::min(epochs, max_passes - passes);
         const int64_t sums = pl.epoch_words * (n + 1);
+        *began = e.init_state ? *e.init_state : *e.h_state;
         if ((rc = prepare(e, (uint64_t *)ex, sums + pl.edge_words))) return rc;
         flags[0] = 1;
         flags[1] = 0;
@@ -842,6 +847,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
             a.ny = pl.nbrick[1];
             a.epochs = n;
             a.kkt_last = kkt_last;
+            a.rereads = e.ctx->wait_limit;
             rc = ph.f64 ? launch_grid_loop_double(K, a, pl.nwg, pl.npt, s)
                         : launch_grid_loop_float(K, a, pl.nwg, pl.npt, s);
         } else if (img) {
@@ -860,6 +866,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
             a.nct = pl.nct;
             a.epochs = n;
             a.kkt_last = kkt_last;
+            a.rereads = e.ctx->wait_limit;
             a.need_f = need_f;
 #define PASC_IL(R)                                                                  \
     case R:                                                                         \
@@ -886,6 +893,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
             a.tpw = pl.tpw;
             a.epochs = n;
             a.kkt_last = kkt_last;
+            a.rereads = e.ctx->wait_limit;
             const bool small = pl.nw == LOOP_WAVES_MIN;
             if (ph.f64)
                 rc = small ? launch_loop_1d_double_4_(K, a, pl.nwg, pl.chunk, s)
@@ -900,7 +908,10 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
         }
         HIP_TRY(hipEventRecord((hipEvent_t)e.ev_solve[1], s));
         HIP_TRY(hipStreamSynchronize(s));
-        if (flags[1]) return fail(PASC_ERR_HIP, "the workgroups of the persistent loop lost each other");
+        if (flags[1]) {
+            e.init_state = began;
+            return PASC_OK;
+        }
         passes += n;
         if (!flags[0]) break;
     }
@@ -911,9 +922,10 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
 static int run_phase(Engine &e, const PhaseCfg &ph, const pasc_spg_params &p, int max_passes) {
     hipStream_t s = S_(e);
     int passes = 0;
+    InstState began;  // alive until prepare() has taken it
     {
         bool ran;
-        int rc0 = run_loop(e, ph, passes, max_passes, &ran);
+        int rc0 = run_loop(e, ph, passes, max_passes, &ran, &began);
         e.looped = rc0 == PASC_OK && ran;
         if (rc0 || ran) return rc0;
     }

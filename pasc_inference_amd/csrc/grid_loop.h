@@ -35,6 +35,7 @@ struct GridLoopArgs {
     int32_t nx, ny;      // bricks across and down
     int32_t epochs;
     int32_t kkt_last;
+    int32_t rereads;  // as LoopArgs
 };
 
 // Nodes of a tile (the brick and the nodes around it) at most.  Also the distance of two components
@@ -78,6 +79,7 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
     double window = 0.0;
     if (wave == 0) loop_load_state(A.state[0], A.sp.m, lane, st, window);
     if (tid < 8 * NPART) sh.red[tid >> 3][tid & 7] = 0.0;
+    if (tid == 0) sh.parity = par0 ^ 1;
     for (int i = tid; i < (K + KS) * ts; i += NT) gam[i] = C(0);  // finite: it meets weight 0
     __syncthreads();
 
@@ -281,7 +283,7 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
                 for (int h = 0; h < HPT; h++)
 #pragma unroll
                     for (int k = 0; k < KS; k++) all = all && published(v[h][k]);
-            } while (!all && ++n < LOOP_SPIN_LIMIT);
+            } while (!all && ++n < A.rereads);
             if (!all) A.flags[1] = 1;
 #pragma unroll
             for (int h = 0; h < HPT; h++)
@@ -318,7 +320,7 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
         lds_barrier();
         if (wave == 0)
             loop_step(sh, want_kkt, alpha_d, (double)a_dir, sample_eps, ex, slot_ld, nwg, wg, lane, st,
-                      window, A.sp, A.flags);
+                      window, A.sp, A.rereads, A.flags);
         lds_barrier();
         beta = uni(C(sh.b_apply));
         a_dir = uni(C(sh.a_dir));
@@ -349,12 +351,12 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
             for (int w = 0; w < NW; w++) kkt = nan_max(kkt, sh.red[4][w]);
             if (lane == 0) store_coherent(ex + wg, kkt);
             if (wg == 0) {
-                for (int j = lane; j < nwg; j += WAVE) kkt = nan_max(kkt, await_value(ex + j, A.flags + 1));
+                for (int j = lane; j < nwg; j += WAVE) kkt = nan_max(kkt, await_value(ex + j, A.rereads, A.flags + 1));
                 st.kkt = wave_max_all(kkt);
             }
         }
     }
-    // gamma_i (K rows, the last as complete_last_row forms it) and d_i to the buffers its parity names
+    // gamma_i (K rows, the last as complete_last_row forms it) and d_i to the launch's other buffers
     const int par = uni(sh.parity);
     S *dst = reinterpret_cast<S *>(par ? A.p.gamma1 : A.p.gamma0) + goff;
     S *dout = reinterpret_cast<S *>(par ? A.p.dir1 : A.p.dir0) + goff;
@@ -371,6 +373,7 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
         for (int k = 0; k < KS; k++) dout[k * ld + gn[j]] = dir[k * ts + li[j]];
     }
     if (wg == 0 && wave == 0) {
+        st.parity = par;
         loop_put_state(A.state[0], A.sp.m, lane, st, window);
         loop_put_state(*A.out, A.sp.m, lane, st, window);
         if (lane == 0) A.flags[0] = st.active;

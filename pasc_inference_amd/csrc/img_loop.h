@@ -44,6 +44,7 @@ struct ImgLoopArgs {
     int32_t nct;         // tiles across the image
     int32_t epochs;
     int32_t kkt_last;    // as LoopArgs
+    int32_t rereads;     // as LoopArgs
     int32_t need_f;
 };
 
@@ -106,6 +107,7 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
     double window = 0.0;
     if (wave == 0) loop_load_state(A.p.state[0], A.p.sp.m, lane, st, window);
     if (threadIdx.x < 8 * NPART) sh.red[threadIdx.x >> 3][threadIdx.x & 7] = 0.0;
+    if (threadIdx.x == 0) sh.parity = A.p.state[0].parity ^ 1;
 
     // the halo node of this thread: side 0 above, 1 below, 2 left, 3 right; place `at` on the side
     const int u = threadIdx.x;
@@ -368,7 +370,7 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
                 for (int k = 0; k < K; k++) v[k] = load_coherent(src + k * src_ld);
 #pragma unroll
                 for (int k = 0; k < K; k++) all = all && published(v[k]);
-            } while (!all && ++n < LOOP_SPIN_LIMIT);
+            } while (!all && ++n < A.rereads);
             if (!all) A.flags[1] = 1;
 #pragma unroll
             for (int k = 0; k < K; k++) {
@@ -421,7 +423,7 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
         lds_barrier();
         if (wave == 0)
             loop_step(sh, cx.want_kkt, cx.alpha_d, cx.a_dir_d, sample_eps, ex, slot_ld, nwg, wg, lane, st,
-                      window, A.p.sp, A.flags);
+                      window, A.p.sp, A.rereads, A.flags);
         lds_barrier();
         cx.beta = uni(C(sh.b_apply));
         cx.a_dir = uni(C(sh.a_dir));
@@ -461,12 +463,12 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
             for (int w = 0; w < NW; w++) kkt = nan_max(kkt, sh.red[4][w]);
             if (lane == 0) store_coherent(ex + wg, kkt);
             if (wg == 0) {
-                for (int j = lane; j < nwg; j += WAVE) kkt = nan_max(kkt, await_value(ex + j, A.flags + 1));
+                for (int j = lane; j < nwg; j += WAVE) kkt = nan_max(kkt, await_value(ex + j, A.rereads, A.flags + 1));
                 st.kkt = wave_max_all(kkt);
             }
         }
     }
-    // gamma_i (K rows) and p_i to the buffers its parity names
+    // gamma_i (K rows) and p_i to the launch's other buffers
     const int par = uni(sh.parity);
     const int64_t goff = uni(A.p.desc[0].goff);
     S *dst = reinterpret_cast<S *>(par ? A.p.gamma1 : A.p.gamma0) + goff;
@@ -487,6 +489,7 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
         }
     }
     if (wg == 0 && wave == 0) {
+        st.parity = par;
         loop_put_state(A.p.state[0], A.p.sp.m, lane, st, window);
         loop_put_state(*A.out, A.p.sp.m, lane, st, window);
         if (lane == 0) A.flags[0] = st.active;

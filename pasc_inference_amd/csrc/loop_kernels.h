@@ -22,7 +22,10 @@
 // reader re-reads it until the value is there (settle_published), so no two locations need an
 // order between them, and nothing has to be reset inside the launch.  The workgroups must run
 // at the same time: the launch is cooperative (one workgroup per CU), which the runtime grants
-// only if they all fit.  Waits are bounded; a value that does not come makes the solve fail.
+// only if they all fit.  Waits are bounded: where a value does not come (work of another stream or
+// process keeps a workgroup off the chip) the launch is taken back and the phase goes on with the
+// tiled passes from where the launch began.  The launch therefore leaves its results in the
+// buffer it does not start from.
 #pragma once
 
 #include "exchange.h"
@@ -46,6 +49,7 @@ struct LoopArgs {
     int32_t epochs;      // iterations of this launch at most
     int32_t kkt_last;    // 1: the KKT residual is evaluated once, for the iterate that stopped
                          // (the area holds one more epoch for it)
+    int32_t rereads;     // re-reads of a value before it counts as lost
 };
 
 // Steps per lane.  FP64: 4, or 2 where 4 steps of K values in four arrays would spill (K >= 5)
@@ -131,7 +135,8 @@ __device__ __forceinline__ void loop_put_state(InstState &g, int m, int lane, co
 struct LoopShared {
     double red[NPART][8];  // [sum][wave]; waves from NW on stay 0
     double a_apply, b_apply, a_dir;
-    int32_t it, active, parity;
+    int32_t it, active;
+    int32_t parity;  // the buffer the launch ends in: the one it does not start from
 };
 
 // A wave's share of the iteration's sums dd, (sum of the edge terms), dd + off, f, residual: four
@@ -152,7 +157,7 @@ __device__ __forceinline__ void loop_sums(LoopShared &sh, double (&acc)[NPART], 
 __device__ __forceinline__ void loop_step(LoopShared &sh, bool want_kkt, double edge_scale,
                                           double a_dir, double sample_eps, double *ex, int slot_ld,
                                           int nwg, int wg, int lane, LoopState &st, double &window,
-                                          const StepParams &sp, int32_t *flags) {
+                                          const StepParams &sp, int32_t rereads, int32_t *flags) {
     // lane 8 q + w holds wave w's value q; three exchanges sum over w
     double v0 = lane < 8 * NPART ? sh.red[lane >> 3][lane & 7] : 0.0, v1 = v0;
     v0 += dpp_from<DPP_XOR1>(v0);
@@ -192,7 +197,7 @@ __device__ __forceinline__ void loop_step(LoopShared &sh, bool want_kkt, double 
             for (int b = 0; b < 4; b++)
 #pragma unroll
                 for (int q = 0; q < NPART; q++) all = all && published(w[b][q]);
-        } while (!all && ++n < LOOP_SPIN_LIMIT);
+        } while (!all && ++n < rereads);
         if (!all) {
             flags[1] = 1;
             w[0][0] = __builtin_nan("");
@@ -217,7 +222,6 @@ __device__ __forceinline__ void loop_step(LoopShared &sh, bool want_kkt, double 
         sh.a_dir = st.alpha_dir;
         sh.it = st.it;
         sh.active = st.active;
-        sh.parity = st.parity;
     }
 }
 
@@ -279,6 +283,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
     if (wave == 0) loop_load_state(A.p.state[0], A.p.sp.m, lane, st, window);
     const int slot_ld = slot_stride(nwg);
     if (threadIdx.x < 8 * NPART) sh.red[threadIdx.x >> 3][threadIdx.x & 7] = 0.0;
+    if (threadIdx.x == 0) sh.parity = A.p.state[0].parity ^ 1;
     // the series ends where no neighbouring workgroup is: zero halos there
     for (int i = threadIdx.x; i < 2 * 2 * EDGE; i += NW * WAVE) {
         const int par = i / (2 * EDGE), r = i - par * 2 * EDGE;
@@ -429,7 +434,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
         lds_barrier();
         if (wave == 0)
             loop_step(sh, cx.want_kkt, 2.0 * (double)cx.alpha, (double)cx.a_dir, sample_eps, ex, slot_ld,
-                      nwg, wg, lane, st, window, A.p.sp, A.flags);
+                      nwg, wg, lane, st, window, A.p.sp, A.rereads, A.flags);
         if (wave == NW - 1) {
             // the neighbouring workgroups' edges of this iteration
             for (int i = lane; i < 2 * EDGE; i += WAVE) {
@@ -438,7 +443,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
                 if (nb < 0 || nb >= nwg) continue;
                 const double *src = ex_edges + ((int64_t)nb * 2 + (side ^ 1)) * EDGE + r;
                 edge(par ^ 1, side == 0 ? -1 : ntl, side ^ 1)[r] =
-                    S(await_value(src, A.flags + 1));
+                    S(await_value(src, A.rereads, A.flags + 1));
             }
         }
         lds_barrier();
@@ -473,12 +478,12 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
             if (lane == 0) store_coherent(ex + wg, kkt);
             if (wg == 0) {
                 for (int j = lane; j < nwg; j += WAVE)
-                    kkt = nan_max(kkt, await_value(ex + j, A.flags + 1));
+                    kkt = nan_max(kkt, await_value(ex + j, A.rereads, A.flags + 1));
                 st.kkt = wave_max_all(kkt);
             }
         }
     }
-    // the iterate to the buffer its parity names: K rows, the last rebuilt as complete_last_row
+    // the iterate to the launch's other buffer: K rows, the last rebuilt as complete_last_row
     S *dst = reinterpret_cast<S *>(uni(sh.parity) ? A.p.gamma1 : A.p.gamma0) + uni(A.p.desc[0].goff);
     for (int lt = wave; lt < ntl; lt += NW) {
         const int64_t t0 = (int64_t)(tile0 + lt) * TILE - (int64_t)HT * CH + (int64_t)lane * CH;
@@ -517,6 +522,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
         }
     }
     if (wg == 0 && wave == 0) {
+        st.parity = uni(sh.parity);
         loop_put_state(A.p.state[0], A.p.sp.m, lane, st, window);
         loop_put_state(*A.out, A.p.sp.m, lane, st, window);
         if (lane == 0) {
