@@ -930,6 +930,8 @@ static int run_phase(Engine &e, const PhaseCfg &ph, const pasc_spg_params &p, in
         if (rc0 || ran) return rc0;
     }
     const bool runs = !e.init_state || e.init_state->active;
+    // the polish of an FP32 phase that failed: no pass would tell the host that nothing is active
+    if (e.n_inst == 1 && !runs) max_passes = 0;
     {
         const int rc0 = prepare(e, nullptr, 0);
         if (rc0) return rc0;
