@@ -259,7 +259,8 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
                 }
                 ddt += (double)d * (double)d;
                 const C r = tau - y[k];
-                off += (double)(r > C(0) ? r : C(0)) * (double)g0[k];
+                // y = tau = -inf (an overflow) gives NaN, which ends the solve, as in the graph kernels
+                off += (double)(r < C(0) ? C(0) : r) * (double)g0[k];
                 fq += ((double)g[k] + (double)q[j][k]) * (double)g0[k];
             }
             acc[2] += ddt + off;

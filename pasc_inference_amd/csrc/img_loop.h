@@ -418,6 +418,10 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
         }
         // 4. the sums and the step
         if (!need_f) acc[3] = 0.0;
+        // an overflow (of FP32: its f comes from the step, which would carry an infinity on) ends the
+        // solve as a NaN does; the image pass meets it as 0 * inf in its halo columns
+        acc[2] += 0.0 * acc[2];
+        acc[3] += 0.0 * acc[3];
         loop_sums<NW>(sh, acc, cx.want_kkt, lane, wave);
         if (!QREG) fetch_q(y0);  // of the next iteration
         lds_barrier();
