@@ -62,6 +62,7 @@ struct CgState {
 };
 constexpr int CG_POLL = 16;  // CG iterations launched between host reads of the stop flag
 constexpr int RNT = 1024;    // threads of the one-workgroup partial reductions
+constexpr size_t ADJ_KEEP_BYTES = (size_t)128 << 20;
 
 template <int NV>
 __device__ inline void block_sum(double (&v)[NV], double *lds, double *out) {
@@ -505,7 +506,11 @@ static int run_adj(Engine &e, const InstDesc &D, const uint8_t *mask, double cg_
         const int rc = run_adj_loop<K>(e, D, gam, mask, cg_tol, cg_maxit, res, &ran);
         if (rc || ran) return rc;
     }
-    return run_adj_kernels<K>(e, D, mask, cg_tol, cg_maxit, res);
+    const int rc = run_adj_kernels<K>(e, D, mask, cg_tol, cg_maxit, res);
+    // Six vectors (1.4 GB at T = 1e7, K = 3) are not kept with the problem between its adjoints; what
+    // the persistent launch needs at most (r, p and lambda of the series that fit on chip) is.
+    engine_trim_scratch(e, ADJ_KEEP_BYTES);
+    return rc;
 }
 
 int engine_adjoint(Engine &e, int inst, const uint8_t *mask_host, double cg_tol, int cg_maxit,

@@ -364,6 +364,13 @@ int engine_scratch(Engine &e, size_t bytes, void **p) {
     return PASC_OK;
 }
 
+void engine_trim_scratch(Engine &e, size_t keep) {
+    if (e.scratch_bytes <= keep) return;
+    (void)hipFree(e.d_scratch);
+    e.d_scratch = nullptr;
+    e.scratch_bytes = 0;
+}
+
 static int alloc_linear_term(Engine &e);
 
 int engine_set_graph(Engine &e, int64_t T, int64_t R, int32_t width, const int64_t *nbr_ptr,

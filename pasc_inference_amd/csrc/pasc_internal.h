@@ -220,6 +220,8 @@ int engine_update_desc(Engine &e);
 int engine_theta_update(Engine &e, int inst, double *theta_out);
 // the engine's scratch buffer, grown to `bytes` (any earlier content may be lost)
 int engine_scratch(Engine &e, size_t bytes, void **p);
+// gives a scratch buffer of more than `keep` bytes back (no work may be using it)
+void engine_trim_scratch(Engine &e, size_t keep);
 int engine_labels(Engine &e, int inst, int32_t *labels);
 int engine_abserr(Engine &e, int inst, const double *solution, double *abserr);
 int engine_adjoint(Engine &e, int inst, const uint8_t *mask, double cg_tol, int cg_maxit,
