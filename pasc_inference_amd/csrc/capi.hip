@@ -1184,6 +1184,7 @@ int pasc_batch_autotune(pasc_batch *b, const char *cache_path, pasc_launch_shape
     snprintf(key, sizeof(key), "%s/%sbatch%d/p%d/E2^%d", b->ctx->c.arch.c_str(), kind, b->e.n_inst,
              b->e.precision, (int)std::floor(std::log2((double)std::max<int64_t>(elems, 1))));
     rc = engine_fill_uniform(b->e);  // the scan starts from gamma0 = 1/K
+    if (rc == PASC_OK) rc = settle(&b->ctx->c);  // (with a cached shape nothing else waits for it)
     if (rc) return rc;
     return autotune_cached(b->e, b->ctx->c, key, elems, cache_path, shape);
 }

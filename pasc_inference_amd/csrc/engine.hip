@@ -474,7 +474,7 @@ int engine_set_gamma(Engine &e, int inst, const double *g, int layout) {
 
 // Waits for what a call queued on the caller's stream: the library's own stream orders what follows,
 // but a caller may go on with another stream as soon as the call is back.
-static int settle(const Ctx *ctx) {
+int settle(const Ctx *ctx) {
     if (!ctx->own_stream) HIP_TRY(hipStreamSynchronize((hipStream_t)ctx->stream));
     return PASC_OK;
 }

@@ -209,6 +209,8 @@ int engine_set_graph(Engine &e, int64_t T, int64_t R, int32_t width, const int64
 int engine_set_linear_term(Engine &e, int inst, const double *b_host, int layout);
 int engine_set_uniform(Engine &e, int inst);
 int engine_fill_uniform(Engine &e);
+// waits for what a call queued on a caller's stream (see engine.hip)
+int settle(const Ctx *ctx);
 int engine_set_gamma(Engine &e, int inst, const double *gamma_host, int layout);
 int engine_get_gamma(Engine &e, int inst, double *gamma_host, int layout);
 int engine_solve(Engine &e, const pasc_spg_params &p, pasc_spg_result *res_single,
