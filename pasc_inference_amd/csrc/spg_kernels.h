@@ -710,8 +710,13 @@ __global__ __launch_bounds__(NT) void spg_pass_1d(PassArgs A) {
             const int nt = tile + 1;
             const bool stage_next = can_stage && m + 1 < msub && (int64_t)nt * TILE < cx.T &&
                                     tile_is_interior<S, C, K, CH, NT>(nt, cx.T);
+            // (the barrier: no store of the tile may come to stand before the copies, which the counted
+            // wait below takes for older)
             auto issue = [&]() {
-                if (stage_next) stage_issue<S, C, K, CH, NT>(cx, nt, stage);
+                if (stage_next) {
+                    stage_issue<S, C, K, CH, NT>(cx, nt, stage);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             };
             // The copies of the next tile must have arrived, the stores behind them need not: an
             // interior tile ends with its KS * CH / VW stores, and vector memory operations complete
