@@ -293,12 +293,6 @@ static int sum_partials(hipStream_t s, const double *d_part, int blocks, int nv,
     return PASC_OK;
 }
 
-template <typename A, typename B>
-__global__ __launch_bounds__(256) void adj_convert(const A *src, B *dst, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = B(src[i]);
-}
-
 __global__ __launch_bounds__(256) void copy_bytes(const uint8_t *src, uint8_t *dst, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
         dst[i] = src[i];

@@ -190,11 +190,6 @@ __device__ inline double wave_max(double v) {
     }
     return v;
 }
-__device__ inline int wave_sum_i(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
-}
 
 // Block reduction of NPART partials (sum for the first 4, max for the last).  Thread 0 returns
 // the result in v.  lds must hold NPART * (NT/64) doubles.

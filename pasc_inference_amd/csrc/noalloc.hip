@@ -41,7 +41,9 @@ int noalloc_init(int device) {
     return PASC_OK;
 }
 
-// Largest number of steps the static scratch serves for K clusters and xdim channels.
+// Largest number of steps the call takes for K clusters and xdim channels: a row of partials per 256
+// steps, less one, in the scratch.  (The sums take at most READ_BLOCKS rows whatever the steps; the
+// limit stands as the interface states it.)
 int64_t noalloc_theta_max_T(int K, int xdim) {
     const int64_t nv = (int64_t)K * (1 + xdim);
     const int64_t blocks = (int64_t)NOALLOC_SCRATCH_DOUBLES / nv - 1;
@@ -58,9 +60,8 @@ int rows_theta_noalloc(Engine &e, const void *g, bool f32, const InstDesc &d, co
                                     "not set up (pasc_ctx_create does that)", device);
     if (d.T > noalloc_theta_max_T(d.K, d.xdim))
         return fail(PASC_ERR_ARG, "theta_update_noalloc: T*R = %lld exceeds %lld, the most the "
-                                  "static scratch (%zu doubles) serves at K = %d, xdim = %d",
-                    (long long)d.T, (long long)noalloc_theta_max_T(d.K, d.xdim),
-                    NOALLOC_SCRATCH_DOUBLES, d.K, d.xdim);
+                                  "call takes at K = %d, xdim = %d",
+                    (long long)d.T, (long long)noalloc_theta_max_T(d.K, d.xdim), d.K, d.xdim);
     static_assert(NOALLOC_SCRATCH_DOUBLES >= (size_t)READ_BLOCKS * PASC_MAX_K * 4, "the partials fit");
     return theta_from_rows(e, g, f32, d, x, g_scratch_ptr[device], theta_out);
 }
