@@ -174,11 +174,11 @@ int pasc_ctx_create(int device, pasc_ctx **out);
 int pasc_ctx_destroy(pasc_ctx *ctx);
 /* Use an external HIP stream (hipStream_t cast to void*), or NULL for the context's own. */
 int pasc_ctx_set_stream(pasc_ctx *ctx, void *stream);
-/* How long the workgroups of a persistent launch (a problem that fits on the chip) wait for one
- * another before the call goes on without it, in separate launches from where that launch began:
- * re-reads of about 1 us, default (and 0) 2^22.  The wait runs out when work of another stream or
- * process keeps part of the launch off the chip that long. */
-int pasc_ctx_set_wait_limit(pasc_ctx *ctx, int32_t rereads);
+/* The workgroups of a persistent launch (a problem that fits on the chip) wait about 4 s for one
+ * another.  When the wait runs out, because work of another stream or process keeps part of the
+ * launch off the chip, the launch is taken back: the call goes on in separate launches from where it
+ * began.  For tests: on != 0 takes every such launch back. */
+int pasc_ctx_set_take_back(pasc_ctx *ctx, int32_t on);
 int pasc_ctx_synchronize(pasc_ctx *ctx);
 
 /* ---- problem (TSData/QPData/GraphH1FEMModel) ---- */

@@ -105,7 +105,7 @@ _SIGS = {
     "pasc_ctx_create": ([C.c_int, C.POINTER(vp)], C.c_int),
     "pasc_ctx_destroy": ([vp], C.c_int),
     "pasc_ctx_set_stream": ([vp, vp], C.c_int),
-    "pasc_ctx_set_wait_limit": ([vp, C.c_int32], C.c_int),
+    "pasc_ctx_set_take_back": ([vp, C.c_int32], C.c_int),
     "pasc_ctx_synchronize": ([vp], C.c_int),
     "pasc_problem_create": ([vp, C.POINTER(ProblemDesc), C.POINTER(vp)], C.c_int),
     "pasc_problem_destroy": ([vp], C.c_int),

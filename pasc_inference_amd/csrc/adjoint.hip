@@ -373,7 +373,6 @@ static int run_adj_loop(Engine &e, const InstDesc &D, const double *gam, const u
     a.ex = ex;
     a.epochs = epochs;
     a.maxit = cg_maxit;
-    a.rereads = e.ctx->wait_limit;
     for (a.resume = 0;; a.resume = 1) {
         const int64_t words = ow + ew * epochs;
         hipLaunchKernelGGL(fill_u64, dim3((unsigned)std::min<int64_t>((words + 255) / 256, 1024)),
@@ -386,7 +385,7 @@ static int run_adj_loop(Engine &e, const InstDesc &D, const double *gam, const u
                                                      : launch_adj_loop<K, CH, 8>(a, nwg, s);
         if (!ok) return PASC_OK;
         HIP_TRY(hipStreamSynchronize(s));
-        if (a.flags[1]) return PASC_OK;  // the workgroups lost each other: nothing of it is used
+        if (a.flags[1] || e.ctx->take_back) return PASC_OK;  // the workgroups lost each other: nothing of it is used
         if (!a.flags[0]) break;
     }
     res.loss = a.out[0];

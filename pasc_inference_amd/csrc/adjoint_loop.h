@@ -37,7 +37,6 @@ struct AdjLoopArgs {
     int32_t epochs;         // CG steps of this launch at most
     int32_t maxit;
     int32_t resume;         // 1: r, p and lambda come from save
-    int32_t rereads;        // re-reads of a value before it counts as lost
 };
 
 constexpr int adj_chunk(int K) { return K <= 4 ? 8 : 4; }  // steps of a lane at most
@@ -125,7 +124,7 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
         const int nb = side == 0 ? wg - 1 : wg + 1;
         const double v = nb < 0 || nb >= nwg
                              ? 0.0
-                             : await_value(ex_edges + ((int64_t)nb * 2 + (side ^ 1)) * K + k, A.rereads, lost);
+                             : await_value(ex_edges + ((int64_t)nb * 2 + (side ^ 1)) * K + k, lost);
         redge[par][side == 0 ? 0 : NW + 1][side ^ 1][k] = v;
     };
 
@@ -207,11 +206,11 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
     const int maxit = A.maxit;
     bool done = false;
     if (wave == 0) {
-        loss = await_sum(open, nwg, lane, A.rereads, lost);
-        rr0 = await_sum(open + sld, nwg, lane, A.rereads, lost);
+        loss = await_sum(open, nwg, lane, lost);
+        rr0 = await_sum(open + sld, nwg, lane, lost);
 #pragma unroll
         for (int k = 0; k < K; k++)
-            direct[k] = await_sum(open + (int64_t)(2 + k) * sld, nwg, lane, A.rereads, lost);
+            direct[k] = await_sum(open + (int64_t)(2 + k) * sld, nwg, lane, lost);
         rr = A.resume ? A.save_rr[0] : rr0;
         it = A.resume ? (int)A.save_rr[1] : 0;
         done = !(it < maxit && rr > A.tol2 * rr0 && rr > 0.0);
@@ -257,7 +256,7 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
         if (lane == 0) red[0][wave] = pq;
         publish_step(ex);
         if (wave == 0) {
-            pq = await_sum(ex + copy, nwg, lane, A.rereads, lost);
+            pq = await_sum(ex + copy, nwg, lane, lost);
             if (lane == 0) {
                 bc[0] = rr / pq;
                 bc[1] = pq > 0.0 ? 0.0 : 1.0;  // p in the null space of P A P: the system is solved
@@ -287,7 +286,7 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
             for (int c = 0; c < CH; c++) my_lam[k * LROW + c] += step * p[k][c];
         if (wave == NW - 1) get_edges(par ^ 1, ex_edges);
         if (wave == 0) {
-            rn = await_sum(ex_r + copy, nwg, lane, A.rereads, lost);
+            rn = await_sum(ex_r + copy, nwg, lane, lost);
             const double b = rn / rr;
             rr = rn;
             it++;
@@ -359,12 +358,12 @@ __global__ __launch_bounds__(NW *WAVE) void adj_loop(AdjLoopArgs A) {
         }
         publish(close, 1 + K);
         if (wg == 0 && wave == 0) {
-            const double v0 = await_sum(close, nwg, lane, A.rereads, lost);
+            const double v0 = await_sum(close, nwg, lane, lost);
             double dth[K];
 #pragma unroll
             for (int k = 0; k < K; k++)
                 dth[k] = direct[k] +
-                         await_sum(close + (int64_t)(1 + k) * sld, nwg, lane, A.rereads, lost);
+                         await_sum(close + (int64_t)(1 + k) * sld, nwg, lane, lost);
             if (lane == 0) {
                 A.out[0] = loss;
                 A.out[1] = v0;

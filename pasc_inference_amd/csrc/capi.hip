@@ -151,9 +151,9 @@ int pasc_ctx_set_stream(pasc_ctx *ctx, void *stream) {
     return PASC_OK;
 }
 
-int pasc_ctx_set_wait_limit(pasc_ctx *ctx, int32_t rereads) {
-    if (!ctx || rereads < 0) return fail(PASC_ERR_ARG, "ctx_set_wait_limit: bad arguments");
-    ctx->c.wait_limit = rereads > 0 ? rereads : WAIT_LIMIT;
+int pasc_ctx_set_take_back(pasc_ctx *ctx, int32_t on) {
+    if (!ctx) return fail(PASC_ERR_ARG, "ctx is NULL");
+    ctx->c.take_back = on != 0;
     return PASC_OK;
 }
 

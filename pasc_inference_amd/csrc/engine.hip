@@ -854,7 +854,6 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
             a.ny = pl.nbrick[1];
             a.epochs = n;
             a.kkt_last = kkt_last;
-            a.rereads = e.ctx->wait_limit;
             rc = ph.f64 ? launch_grid_loop_double(K, a, pl.nwg, pl.npt, s)
                         : launch_grid_loop_float(K, a, pl.nwg, pl.npt, s);
         } else if (img) {
@@ -873,7 +872,6 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
             a.nct = pl.nct;
             a.epochs = n;
             a.kkt_last = kkt_last;
-            a.rereads = e.ctx->wait_limit;
             a.need_f = need_f;
 #define PASC_IL(R)                                                                  \
     case R:                                                                         \
@@ -900,7 +898,6 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
             a.tpw = pl.tpw;
             a.epochs = n;
             a.kkt_last = kkt_last;
-            a.rereads = e.ctx->wait_limit;
             const bool small = pl.nw == LOOP_WAVES_MIN;
             if (ph.f64)
                 rc = small ? launch_loop_1d_double_4_(K, a, pl.nwg, pl.chunk, s)
@@ -915,7 +912,7 @@ static int run_loop(Engine &e, const PhaseCfg &ph, int &passes, int max_passes, 
         }
         HIP_TRY(hipEventRecord((hipEvent_t)e.ev_solve[1], s));
         HIP_TRY(hipStreamSynchronize(s));
-        if (flags[1]) {
+        if (flags[1] || e.ctx->take_back) {
             e.init_state = began;
             return PASC_OK;
         }

@@ -6,6 +6,9 @@
 
 namespace pasc {
 
+// Re-reads (~1 us each) before a value counts as lost.  A constant: as a kernel argument it took a
+// scalar register that the adjoint's loop does not have (0.8 % of its call, 1.7 % kept in one).
+constexpr int LOOP_SPIN_LIMIT = 1 << 22;
 constexpr size_t LOOP_LDS_BYTES = 159 * 1024;      // dynamic LDS (160 KiB less the static part)
 constexpr int64_t LOOP_EXCHANGE_BYTES = 16 << 20;  // exchange area of a launch at most
 
@@ -84,19 +87,17 @@ __device__ __forceinline__ bool published(double v) {
     return __builtin_bit_cast(uint64_t, v) != PART_EMPTY;
 }
 
-// One value that another workgroup publishes at p; *lost is set when it does not come within
-// `limit` re-reads.
-__device__ __forceinline__ double await_value(const double *p, int32_t limit, int32_t *lost) {
+// One value that another workgroup publishes at p; *lost is set when it does not come.
+__device__ __forceinline__ double await_value(const double *p, int32_t *lost) {
     double v = load_coherent(p);
-    for (int n = 0; !published(v) && n < limit; n++) v = load_coherent(p);
+    for (int n = 0; !published(v) && n < LOOP_SPIN_LIMIT; n++) v = load_coherent(p);
     if (!published(v)) *lost = 1;
     return v;
 }
 
 // Sum of the n workgroups' values row[0 .. n), in index order per lane; called by a whole wave.
 // All values of a lane are re-read together until the last one is there.
-__device__ __forceinline__ double await_sum(const double *row, int n, int lane, int32_t limit,
-                                            int32_t *lost) {
+__device__ __forceinline__ double await_sum(const double *row, int n, int lane, int32_t *lost) {
     double s = 0.0;
     for (int j0 = lane; j0 < n; j0 += 4 * WAVE) {
         double w[4];
@@ -108,7 +109,7 @@ __device__ __forceinline__ double await_sum(const double *row, int n, int lane, 
             for (int b = 0; b < 4; b++) w[b] = j0 + b * WAVE < n ? load_coherent(row + j0 + b * WAVE) : 0.0;
 #pragma unroll
             for (int b = 0; b < 4; b++) all = all && published(w[b]);
-        } while (!all && ++spins < limit);
+        } while (!all && ++spins < LOOP_SPIN_LIMIT);
         if (!all) *lost = 1;
 #pragma unroll
         for (int b = 0; b < 4; b++) s += w[b];

@@ -35,7 +35,6 @@ struct GridLoopArgs {
     int32_t nx, ny;      // bricks across and down
     int32_t epochs;
     int32_t kkt_last;
-    int32_t rereads;  // as LoopArgs
 };
 
 // Nodes of a tile (the brick and the nodes around it) at most.  Also the distance of two components
@@ -284,7 +283,7 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
                 for (int h = 0; h < HPT; h++)
 #pragma unroll
                     for (int k = 0; k < KS; k++) all = all && published(v[h][k]);
-            } while (!all && ++n < A.rereads);
+            } while (!all && ++n < LOOP_SPIN_LIMIT);
             if (!all) A.flags[1] = 1;
 #pragma unroll
             for (int h = 0; h < HPT; h++)
@@ -321,7 +320,7 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
         lds_barrier();
         if (wave == 0)
             loop_step(sh, want_kkt, alpha_d, (double)a_dir, sample_eps, ex, slot_ld, nwg, wg, lane, st,
-                      window, A.sp, A.rereads, A.flags);
+                      window, A.sp, A.flags);
         lds_barrier();
         beta = uni(C(sh.b_apply));
         a_dir = uni(C(sh.a_dir));
@@ -352,7 +351,7 @@ __global__ __launch_bounds__(GRID_LOOP_NT) void grid_loop(GridLoopArgs A) {
             for (int w = 0; w < NW; w++) kkt = nan_max(kkt, sh.red[4][w]);
             if (lane == 0) store_coherent(ex + wg, kkt);
             if (wg == 0) {
-                for (int j = lane; j < nwg; j += WAVE) kkt = nan_max(kkt, await_value(ex + j, A.rereads, A.flags + 1));
+                for (int j = lane; j < nwg; j += WAVE) kkt = nan_max(kkt, await_value(ex + j, A.flags + 1));
                 st.kkt = wave_max_all(kkt);
             }
         }

@@ -44,7 +44,6 @@ struct ImgLoopArgs {
     int32_t nct;         // tiles across the image
     int32_t epochs;
     int32_t kkt_last;    // as LoopArgs
-    int32_t rereads;     // as LoopArgs
     int32_t need_f;
 };
 
@@ -370,7 +369,7 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
                 for (int k = 0; k < K; k++) v[k] = load_coherent(src + k * src_ld);
 #pragma unroll
                 for (int k = 0; k < K; k++) all = all && published(v[k]);
-            } while (!all && ++n < A.rereads);
+            } while (!all && ++n < LOOP_SPIN_LIMIT);
             if (!all) A.flags[1] = 1;
 #pragma unroll
             for (int k = 0; k < K; k++) {
@@ -427,7 +426,7 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
         lds_barrier();
         if (wave == 0)
             loop_step(sh, cx.want_kkt, cx.alpha_d, cx.a_dir_d, sample_eps, ex, slot_ld, nwg, wg, lane, st,
-                      window, A.p.sp, A.rereads, A.flags);
+                      window, A.p.sp, A.flags);
         lds_barrier();
         cx.beta = uni(C(sh.b_apply));
         cx.a_dir = uni(C(sh.a_dir));
@@ -467,7 +466,7 @@ __global__ __launch_bounds__(NW *WAVE) void img_loop(ImgLoopArgs A) {
             for (int w = 0; w < NW; w++) kkt = nan_max(kkt, sh.red[4][w]);
             if (lane == 0) store_coherent(ex + wg, kkt);
             if (wg == 0) {
-                for (int j = lane; j < nwg; j += WAVE) kkt = nan_max(kkt, await_value(ex + j, A.rereads, A.flags + 1));
+                for (int j = lane; j < nwg; j += WAVE) kkt = nan_max(kkt, await_value(ex + j, A.flags + 1));
                 st.kkt = wave_max_all(kkt);
             }
         }

@@ -49,7 +49,6 @@ struct LoopArgs {
     int32_t epochs;      // iterations of this launch at most
     int32_t kkt_last;    // 1: the KKT residual is evaluated once, for the iterate that stopped
                          // (the area holds one more epoch for it)
-    int32_t rereads;     // re-reads of a value before it counts as lost
 };
 
 // Steps per lane.  FP64: 4, or 2 where 4 steps of K values in four arrays would spill (K >= 5)
@@ -157,7 +156,7 @@ __device__ __forceinline__ void loop_sums(LoopShared &sh, double (&acc)[NPART], 
 __device__ __forceinline__ void loop_step(LoopShared &sh, bool want_kkt, double edge_scale,
                                           double a_dir, double sample_eps, double *ex, int slot_ld,
                                           int nwg, int wg, int lane, LoopState &st, double &window,
-                                          const StepParams &sp, int32_t rereads, int32_t *flags) {
+                                          const StepParams &sp, int32_t *flags) {
     // lane 8 q + w holds wave w's value q; three exchanges sum over w
     double v0 = lane < 8 * NPART ? sh.red[lane >> 3][lane & 7] : 0.0, v1 = v0;
     v0 += dpp_from<DPP_XOR1>(v0);
@@ -197,7 +196,7 @@ __device__ __forceinline__ void loop_step(LoopShared &sh, bool want_kkt, double 
             for (int b = 0; b < 4; b++)
 #pragma unroll
                 for (int q = 0; q < NPART; q++) all = all && published(w[b][q]);
-        } while (!all && ++n < rereads);
+        } while (!all && ++n < LOOP_SPIN_LIMIT);
         if (!all) {
             flags[1] = 1;
             w[0][0] = __builtin_nan("");
@@ -434,7 +433,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
         lds_barrier();
         if (wave == 0)
             loop_step(sh, cx.want_kkt, 2.0 * (double)cx.alpha, (double)cx.a_dir, sample_eps, ex, slot_ld,
-                      nwg, wg, lane, st, window, A.p.sp, A.rereads, A.flags);
+                      nwg, wg, lane, st, window, A.p.sp, A.flags);
         if (wave == NW - 1) {
             // the neighbouring workgroups' edges of this iteration
             for (int i = lane; i < 2 * EDGE; i += WAVE) {
@@ -443,7 +442,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
                 if (nb < 0 || nb >= nwg) continue;
                 const double *src = ex_edges + ((int64_t)nb * 2 + (side ^ 1)) * EDGE + r;
                 edge(par ^ 1, side == 0 ? -1 : ntl, side ^ 1)[r] =
-                    S(await_value(src, A.rereads, A.flags + 1));
+                    S(await_value(src, A.flags + 1));
             }
         }
         lds_barrier();
@@ -478,7 +477,7 @@ __global__ __launch_bounds__(NW *WAVE) void spg_loop_1d(LoopArgs A) {
             if (lane == 0) store_coherent(ex + wg, kkt);
             if (wg == 0) {
                 for (int j = lane; j < nwg; j += WAVE)
-                    kkt = nan_max(kkt, await_value(ex + j, A.rereads, A.flags + 1));
+                    kkt = nan_max(kkt, await_value(ex + j, A.flags + 1));
                 st.kkt = wave_max_all(kkt);
             }
         }

@@ -180,15 +180,12 @@ struct Engine {
     int prof_n[2] = {0, 0};              // passes launched per phase
 };
 
-// Re-reads (~1 us each) of a value awaited from another workgroup before it counts as lost.
-constexpr int32_t WAIT_LIMIT = 1 << 22;
-
 struct Ctx {
     int device = 0;
     void *stream = nullptr;     // hipStream_t
     bool own_stream = false;
     int n_cu = 0;
-    int32_t wait_limit = WAIT_LIMIT;  // of the persistent loops
+    bool take_back = false;     // every persistent launch counts as lost (tests)
     std::string arch;
     // autotune cache: key -> launch shapes of the two phases
     std::vector<std::pair<std::string, pasc_launch_shape>> tune;

@@ -1,6 +1,6 @@
-"""A persistent launch whose workgroups do not all run at once (forced here by a wait limit of one
-re-read) is taken back: the call goes on in separate launches from where the launch began and
-gives what those give by themselves (profiling on), bit for bit."""
+"""A persistent launch whose workgroups lost each other (here: every launch counts as such) is taken
+back: the call goes on in separate launches from where the launch began and gives what those
+give by themselves (profiling on), bit for bit."""
 import numpy as np
 import pytest
 
@@ -46,9 +46,9 @@ def test_lost_launch_is_taken_back(kind, prec):
         P.set_profiling(True)
         passes = solve()
         P.set_profiling(False)
-        capi.check(capi.lib().pasc_ctx_set_wait_limit(c.h, 1))
+        capi.check(capi.lib().pasc_ctx_set_take_back(c.h, 1))
         lost = [solve(), solve()]
-        capi.check(capi.lib().pasc_ctx_set_wait_limit(c.h, 0))
+        capi.check(capi.lib().pasc_ctx_set_take_back(c.h, 0))
         again = solve()
         P.close()
     assert not np.array_equal(loop[0], passes[0])  # else the comparison below says nothing
@@ -66,9 +66,9 @@ def test_lost_adjoint_is_taken_back():
         P.set_gamma_uniform()
         P.gamma_solve(maxit=3000, stop_mask=capi.STOP_KKT, kkt_tol=1e-10)
         out = {}
-        for name, limit, profile in (("loop", 0, False), ("kernels", 0, True), ("lost", 1, False)):
+        for name, on, profile in (("loop", 0, False), ("kernels", 0, True), ("lost", 1, False)):
             print(name, flush=True)
-            capi.check(capi.lib().pasc_ctx_set_wait_limit(c.h, limit))
+            capi.check(capi.lib().pasc_ctx_set_take_back(c.h, on))
             P.set_profiling(profile)
             loss, dle, dth, it = P.adjoint(mask, cg_tol=1e-10, cg_maxit=2000)
             out[name] = np.concatenate([[loss, dle, it], np.ravel(dth)])
