@@ -9,7 +9,8 @@
 // when one host thread did the layout around a pageable copy; in 4 MiB pieces over 8 threads it
 // takes 5 ms, of which the link needs 4.3.  One thread would be bound by its page faults and
 // copies (23 ms).  Up to one piece, a single kernel moves the whole transfer and the threads share
-// the host copy (1.4 MB into fresh pages: 150 us by one thread, 75 by several).
+// the host copy (1.4 MB into fresh pages: 150 us by one thread, 75 by several).  Rows of up to 1 MiB
+// go by the copy engine (small_transfer).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -247,8 +248,86 @@ int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t to
 
 static unsigned piece_blocks(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 1024); }
 
+// Transfers of up to 1 MiB of rows: the rows as they lie by the copy engine, the change of layout and
+// type on this thread.  us of a whole call with fresh pages, FP64, K = 3, interleaved, up / down: 24 KB
+// 10.7 / 10.8 (17.9 / 17.4 through a kernel, its event and a parked thread), 240 KB 16.7 / 21.4 (29 /
+// 30), 1 MB 44 / 50 (60 / 65); 1.2 MB through the kernel 62 / 65.
+constexpr size_t SMALL_BYTES = (size_t)1 << 20;
+
+// rows of T values to and from the interleaved order (K known: the rows are walked together)
+template <int K, typename S>
+static void weave(const S *rows, int64_t T, int64_t ld, double *host) {
+    for (int64_t t = 0; t < T; t++)
+        for (int k = 0; k < K; k++) host[t * K + k] = (double)rows[k * ld + t];
+}
+template <int K, typename S>
+static void unweave(const double *host, int64_t T, int64_t ld, S *rows) {
+    for (int64_t t = 0; t < T; t++)
+        for (int k = 0; k < K; k++) rows[k * ld + t] = S(host[t * K + k]);
+}
+
+template <typename S>
+static void rows_to_boundary(const S *rows, int64_t T, int64_t ld, int K, double *host, bool interleaved) {
+    switch (interleaved ? K : 1) {
+        case 2: return weave<2>(rows, T, ld, host);
+        case 3: return weave<3>(rows, T, ld, host);
+        case 4: return weave<4>(rows, T, ld, host);
+        case 5: return weave<5>(rows, T, ld, host);
+        case 6: return weave<6>(rows, T, ld, host);
+        case 7: return weave<7>(rows, T, ld, host);
+        case 8: return weave<8>(rows, T, ld, host);
+    }
+    for (int k = 0; k < K; k++) std::copy(rows + k * ld, rows + k * ld + T, host + k * T);
+}
+
+template <typename S>
+static void boundary_to_rows(const double *host, int64_t T, int64_t ld, int K, S *rows, bool interleaved) {
+    for (int k = 0; k < K; k++) std::fill(rows + k * ld + T, rows + (k + 1) * ld, S(0));  // as allocated
+    switch (interleaved ? K : 1) {
+        case 2: return unweave<2>(host, T, ld, rows);
+        case 3: return unweave<3>(host, T, ld, rows);
+        case 4: return unweave<4>(host, T, ld, rows);
+        case 5: return unweave<5>(host, T, ld, rows);
+        case 6: return unweave<6>(host, T, ld, rows);
+        case 7: return unweave<7>(host, T, ld, rows);
+        case 8: return unweave<8>(host, T, ld, rows);
+    }
+    for (int k = 0; k < K; k++)
+        for (int64_t t = 0; t < T; t++) rows[k * ld + t] = S(host[k * T + t]);
+}
+static_assert(PASC_MAX_K == 8, "a case for every K");
+
+static int small_transfer(Ctx *ctx, bool to_host, void *rows, bool f32, int64_t T, int64_t ld, int K,
+                          double *host, bool interleaved) {
+    const size_t bytes = (f32 ? 4 : 8) * (size_t)ld * K;
+    SlotPool &pool = g_pool[ctx->device];
+    hipStream_t stream = (hipStream_t)ctx->stream;
+    Slot s;
+    hipError_t e = pool.take(true, s);
+    if (e == hipSuccess) {
+        if (!to_host) {
+            if (f32) boundary_to_rows(host, T, ld, K, (float *)s.p, interleaved);
+            else boundary_to_rows(host, T, ld, K, s.p, interleaved);
+        }
+        e = hipMemcpyAsync(to_host ? (void *)s.p : rows, to_host ? rows : (void *)s.p, bytes,
+                           to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(stream);
+        if (e == hipSuccess && to_host) {
+            if (f32) rows_to_boundary((const float *)s.p, T, ld, K, host, interleaved);
+            else rows_to_boundary((const double *)s.p, T, ld, K, host, interleaved);
+        }
+        pool.give(s);
+    }
+    if (e != hipSuccess)
+        return fail(PASC_ERR_HIP, "%s transfer: %s", to_host ? "device to host" : "host to device",
+                    hipGetErrorString(e));
+    return PASC_OK;
+}
+
 int rows_to_host(Ctx *ctx, const void *rows, bool f32, int64_t T, int64_t ld, int K, double *host,
                  bool interleaved) {
+    if (sizeof(double) * (size_t)ld * K <= SMALL_BYTES)
+        return small_transfer(ctx, true, const_cast<void *>(rows), f32, T, ld, K, host, interleaved);
     const int il = interleaved ? 1 : 0;
     return staged_transfer(
         ctx, true, host, sizeof(double), T * K, [=](hipStream_t s, int64_t i0, int64_t n, void *p) {
@@ -263,6 +342,8 @@ int rows_to_host(Ctx *ctx, const void *rows, bool f32, int64_t T, int64_t ld, in
 
 int rows_from_host(Ctx *ctx, const double *host, bool interleaved, void *rows, bool f32,
                    int64_t T, int64_t ld, int K) {
+    if (sizeof(double) * (size_t)ld * K <= SMALL_BYTES)
+        return small_transfer(ctx, false, rows, f32, T, ld, K, const_cast<double *>(host), interleaved);
     const int il = interleaved ? 1 : 0;
     return staged_transfer(
         ctx, false, const_cast<double *>(host), sizeof(double), T * K,
