@@ -1710,8 +1710,14 @@ int kernel_matvec(Ctx *ctx, const void *x, void *y, int64_t T, int64_t R, int K,
     const int64_t n = T * R;
     if (n == 0) return PASC_OK;
     dim3 grid((unsigned)((n + 255) / 256), (unsigned)K);
-    // the image kernel's columns are 64 lanes wide: narrower images run the general walk
-    const bool image = T == 1 && grid_width >= 48 && !nbr_ptr_dev && R / grid_width < (int64_t)65535 * 4 * MV_ROWS;
+    // The image kernel's columns are 64 lanes wide and a thread walks MV_ROWS rows: the general walk
+    // runs narrower images and those too small to fill the chip so (0.8 million values, over the
+    // share of the lanes that have a column).  us, general / image, FP64: 300 x 300, K = 3 13.1 / 14.2;
+    // 640 x 300, K = 3 14.5 / 14.8; 1000 x 300, K = 3 15.5 / 15.1; 130 x 1000, K = 8 16.0 / 17.3;
+    // 1000 x 1000, K = 1 / 3 15.7 / 15.1 and 28.5 / 20.3.
+    const int64_t lanes = grid_width > 0 ? ((int64_t)grid_width + 63) / 64 * 64 : 1;
+    const bool image = T == 1 && grid_width >= 48 && !nbr_ptr_dev &&
+                       R / grid_width < (int64_t)65535 * 4 * MV_ROWS && n * K >= 800000 * lanes / grid_width;
     if (image && K <= 65535) {
         const int32_t H = (int32_t)(R / grid_width);
         grid = dim3((unsigned)((grid_width + 63) / 64), (unsigned)((H + 4 * MV_ROWS - 1) / (4 * MV_ROWS)),
