@@ -62,10 +62,10 @@ struct CgState {
 };
 constexpr int CG_POLL = 16;  // CG iterations launched between host reads of the stop flag
 constexpr int RNT = 1024;    // threads of the one-workgroup partial reductions
-constexpr size_t ADJ_KEEP_BYTES = (size_t)128 << 20;
+constexpr size_t ADJ_KEEP_BYTES = (size_t)1 << 30;
 
 template <int NV>
-__device__ inline void block_sum(double (&v)[NV], double *lds, double *out) {
+__device__ inline void block_sum(double (&v)[NV], double *lds, double *out, int block) {
     const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
 #pragma unroll
     for (int i = 0; i < NV; i++) v[i] = wave_sum(v[i]);
@@ -500,8 +500,9 @@ static int run_adj(Engine &e, const InstDesc &D, const uint8_t *mask, double cg_
         if (rc || ran) return rc;
     }
     const int rc = run_adj_kernels<K>(e, D, mask, cg_tol, cg_maxit, res);
-    // Six vectors (1.4 GB at T = 1e7, K = 3) are not kept with the problem between its adjoints; what
-    // the persistent launch needs at most (r, p and lambda of the series that fit on chip) is.
+    // Six vectors of a large problem (1.4 GB at T = 1e7, K = 3) are not kept with it between its
+    // adjoints; up to 1 GiB they are, since a new allocation costs 0.5 - 0.9 ms (3.8 -> 4.4 ms for
+    // T = 3e6, K = 3 and 20 steps, 12.3 -> 13.2 for T = 1e7).
     engine_trim_scratch(e, ADJ_KEEP_BYTES);
     return rc;
 }
