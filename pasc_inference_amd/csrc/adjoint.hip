@@ -78,7 +78,7 @@ __device__ inline void block_sum(double (&v)[NV], double *lds, double *out, int 
         for (int i = 0; i < NV; i++) {
             double s = 0.0;
             for (int q = 0; q < ANT / WAVE; q++) s += lds[q * NV + i];
-            out[(int64_t)blockIdx.x * NV + i] = s;
+            out[(int64_t)block * NV + i] = s;
         }
     }
 }
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(ANT) void adj_init(AdjArgs a, double *r, double *pa
             v[1] += dj[k] * dj[k];
         }
     }
-    block_sum<NV>(v, lds, part);
+    block_sum<NV>(v, lds, part, blockIdx.x);
 }
 
 // Sum of part[0 .. blocks) in a fixed order (thread i adds blocks i, i + RNT, ..., then the
@@ -184,6 +184,15 @@ __global__ __launch_bounds__(RNT) void adj_cg_rr(const double *part, int blocks,
 // The search direction p = r + b pold of this step (b = 0 on the first, where pold = r), written
 // to pnew, and q = P A P p (p in range(P)); partial p'q.  pnew and pold are two buffers, since
 // the neighbours' pold are read while other workgroups write.
+//
+// The K components of a neighbour are read together.  On videos the frames before and after are
+// then fetched by all eight L2s (40 frames of 100 x 100, K = 3, 20 steps: 1.41 ms, 1.60 with one
+// component after the other before, against 1.21 here), unless each XCD has a band of its own
+// (xcd_tile).  That pays while a component's three frames of r and p leave room in an L2 of 4 MB:
+// ms without / with bands at K = 2 / 4, frames of 30,000 nodes 2.6 / 4.5 against 1.7 / 3.7, of 48,000
+// 5.2 / 9.0 against 4.2 / 9.2, of 90,000 2.0 / 3.5 against 2.6 / 4.0.  Images have rows in their
+// place: 1024 x 1024, K = 4 2.0 / 1.7, never slower.
+constexpr int64_t BAND_FRAME = 40960;
 template <int K>
 __global__ __launch_bounds__(ANT) void adj_matvec(AdjArgs a, const double *r, const double *pold,
                                                   double *pnew, double *q, double *part,
@@ -191,7 +200,9 @@ __global__ __launch_bounds__(ANT) void adj_matvec(AdjArgs a, const double *r, co
     __shared__ double lds[ANT / WAVE];
     if (cs->done) return;
     const double b = cs->b;
-    const int64_t t = (int64_t)blockIdx.x * ANT + threadIdx.x;
+    const bool bands = a.G.R > 1 && (a.G.T == 1 || a.G.R <= BAND_FRAME);
+    const int block = bands ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+    const int64_t t = (int64_t)block * ANT + threadIdx.x;
     double v[1] = {0.0};
     if (t < a.T) {
         double w[K], pn[K];
@@ -218,7 +229,7 @@ __global__ __launch_bounds__(ANT) void adj_matvec(AdjArgs a, const double *r, co
             v[0] += pn[k] * w[k];
         }
     }
-    block_sum<1>(v, lds, part);
+    block_sum<1>(v, lds, part, block);
 }
 
 // lam += s p; r -= s q with s the step; partial r'r
@@ -241,7 +252,7 @@ __global__ __launch_bounds__(ANT) void adj_axpy(AdjArgs a, const CgState *cs, co
             v[0] += rn * rn;
         }
     }
-    block_sum<1>(v, lds, part);
+    block_sum<1>(v, lds, part, blockIdx.x);
 }
 
 // partials: [0] lambda' A gamma, [1 + 3 k + c] sum_{n with data} lambda_kn 2 (x_nc - theta_kc) bscale
@@ -279,7 +290,7 @@ __global__ __launch_bounds__(ANT) void adj_final(AdjArgs a, const double *lam, d
             }
         }
     }
-    block_sum<NV>(v, lds, part);
+    block_sum<NV>(v, lds, part, blockIdx.x);
 }
 
 static int sum_partials(hipStream_t s, const double *d_part, int blocks, int nv,
