@@ -262,6 +262,10 @@ using PieceLaunch = std::function<void(struct ihipStream_t *, int64_t, int64_t, 
 int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t total,
                     const PieceLaunch &launch);
 
+// `bytes` of host input (4 MiB at most) copied to a pinned piece by this thread; launch(p) enqueues
+// the kernels that read it; returns when they are done
+int with_input(Ctx *ctx, const void *host, size_t bytes, const std::function<void(const void *)> &launch);
+
 // elements of one piece of such a transfer (the last one may be shorter)
 int64_t staged_piece(size_t esize, int64_t total);
 

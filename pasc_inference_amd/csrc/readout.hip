@@ -245,7 +245,10 @@ int engine_eval_raw(Engine &e, int inst, double *fx, double *kkt, double *nb2) {
 }
 
 // ---- |sum_k theta_k gamma_k - solution|_1: the solution's pieces are read where they are staged,
-// each piece leaving one row of partials ----
+// each piece leaving one row of partials.  Up to ABS_ONE_WAIT steps this thread copies the solution
+// and waits once, for everything.  us of a call, so / staged: T = 1000 18.5 / 31, 40,000 27 / 52, 1e5
+// 46 / 71, 2e5 either 90 ----
+constexpr int64_t ABS_ONE_WAIT = 160000;
 template <typename S>
 __global__ __launch_bounds__(RNTH) void abserr_sums(const S *gam, InstDesc D, const double *sol,
                                                     int64_t t0, int64_t n, double *part) {
@@ -261,8 +264,33 @@ __global__ __launch_bounds__(RNTH) void abserr_sums(const S *gam, InstDesc D, co
 
 int rows_abserr(Engine &e, const void *g, bool f32, const InstDesc &d, const double *solution,
                 double *abserr) {
-    // one row of ABS_BLOCKS partials per piece of the solution
     constexpr int ABS_BLOCKS = 64;
+    hipStream_t s = (hipStream_t)e.ctx->stream;
+    double *tot = reinterpret_cast<double *>(e.h_state);
+    auto finish = [=](const double *part, int rows) {
+        hipLaunchKernelGGL(finish_sums, dim3(1), dim3(FINISH_WAVES * WAVE), 0, s, part, rows * ABS_BLOCKS,
+                           1, -1, tot);
+    };
+    auto sums = [=, &d](const void *sol, int64_t t0, int64_t n, double *row) {
+        if (f32)
+            hipLaunchKernelGGL(abserr_sums<float>, dim3(ABS_BLOCKS), dim3(RNTH), 0, s, (const float *)g, d,
+                               (const double *)sol, t0, n, row);
+        else
+            hipLaunchKernelGGL(abserr_sums<double>, dim3(ABS_BLOCKS), dim3(RNTH), 0, s, (const double *)g,
+                               d, (const double *)sol, t0, n, row);
+    };
+    if (d.T <= ABS_ONE_WAIT) {
+        void *part;
+        int rc = engine_scratch(e, sizeof(double) * ABS_BLOCKS, &part);
+        if (rc == PASC_OK)
+            rc = with_input(e.ctx, solution, sizeof(double) * (size_t)d.T, [&](const void *p) {
+                sums(p, 0, d.T, (double *)part);
+                finish((const double *)part, 1);
+            });
+        if (rc == PASC_OK) *abserr = tot[0];
+        return rc;
+    }
+    // one row of ABS_BLOCKS partials per piece of the solution
     const int64_t piece = staged_piece(sizeof(double), d.T);
     const int64_t rows = (d.T + piece - 1) / piece;
     void *buf;
@@ -270,20 +298,11 @@ int rows_abserr(Engine &e, const void *g, bool f32, const InstDesc &d, const dou
     if (rc) return rc;
     double *part = (double *)buf;
     rc = staged_transfer(e.ctx, false, const_cast<double *>(solution), sizeof(double), d.T,
-                         [=, &d](hipStream_t s, int64_t t0, int64_t n, void *p) {
-                             double *row = part + t0 / piece * ABS_BLOCKS;
-                             if (f32)
-                                 hipLaunchKernelGGL(abserr_sums<float>, dim3(ABS_BLOCKS), dim3(RNTH), 0,
-                                                    s, (const float *)g, d, (const double *)p, t0, n, row);
-                             else
-                                 hipLaunchKernelGGL(abserr_sums<double>, dim3(ABS_BLOCKS), dim3(RNTH), 0,
-                                                    s, (const double *)g, d, (const double *)p, t0, n, row);
+                         [=](hipStream_t, int64_t t0, int64_t n, void *p) {
+                             sums(p, t0, n, part + t0 / piece * ABS_BLOCKS);
                          });
     if (rc) return rc;
-    hipStream_t s = (hipStream_t)e.ctx->stream;
-    double *tot = reinterpret_cast<double *>(e.h_state);
-    hipLaunchKernelGGL(finish_sums, dim3(1), dim3(FINISH_WAVES * WAVE), 0, s, (const double *)part,
-                       (int)(rows * ABS_BLOCKS), 1, -1, tot);
+    finish(part, (int)rows);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
     *abserr = tot[0];

@@ -9,7 +9,7 @@
 // when one host thread did the layout around a pageable copy; in 4 MiB pieces over 8 threads it
 // takes 5 ms, of which the link needs 4.3.  One thread would be bound by its page faults and
 // copies (23 ms).  Up to one piece, a single kernel moves the whole transfer and the threads share
-// the host copy (1.4 MB into fresh pages: 150 us by one thread, 75 by several).  Rows of up to 1 MiB
+// the host copy (1.4 MB into fresh pages: 150 us by one thread, 75 by several).  A few rows
 // go by the copy engine (small_transfer).
 #include <hip/hip_runtime.h>
 
@@ -216,6 +216,22 @@ struct Transfer {
     }
 };
 
+int with_input(Ctx *ctx, const void *host, size_t bytes, const std::function<void(const void *)> &launch) {
+    if (bytes > SLOT_BYTES) return fail(PASC_ERR_ARG, "with_input: %zu bytes", bytes);
+    SlotPool &pool = g_pool[ctx->device];
+    Slot s;
+    hipError_t e = pool.take(true, s);
+    if (e == hipSuccess) {
+        std::memcpy(s.p, host, bytes);
+        launch(s.p);
+        e = hipGetLastError();
+        const hipError_t w = hipStreamSynchronize((hipStream_t)ctx->stream);
+        if (e == hipSuccess) e = w;
+        pool.give(s);
+    }
+    return e == hipSuccess ? PASC_OK : fail(PASC_ERR_HIP, "host to device: %s", hipGetErrorString(e));
+}
+
 // Whole slots, or an eighth of a transfer that would fill only a few.
 int64_t staged_piece(size_t esize, int64_t total) {
     const int64_t slot = (int64_t)(SLOT_BYTES / esize);
@@ -248,11 +264,12 @@ int staged_transfer(Ctx *ctx, bool to_host, void *host, size_t esize, int64_t to
 
 static unsigned piece_blocks(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 1024); }
 
-// Transfers of up to 1 MiB of rows: the rows as they lie by the copy engine, the change of layout and
-// type on this thread.  us of a whole call with fresh pages, FP64, K = 3, interleaved, up / down: 24 KB
-// 10.7 / 10.8 (17.9 / 17.4 through a kernel, its event and a parked thread), 240 KB 16.7 / 21.4 (29 /
-// 30), 1 MB 44 / 50 (60 / 65); 1.2 MB through the kernel 62 / 65.
-constexpr size_t SMALL_BYTES = (size_t)1 << 20;
+// Transfers of a few rows: the rows as they lie by the copy engine, the change of layout and type on
+// this thread.  us of a whole call, FP64, K = 3, interleaved, against a kernel, its event and parked
+// threads: up 24 KB 10.7 / 17.9, 240 KB 16.7 / 29, 1 MB 44 / 60; down into pages of an earlier call
+// 10.8 / 17.4, 21.4 / 30, 50 / 65.  Down into fresh pages the threads share the page faults: 240 KB
+// 41 / 47 - 66, 375 KB 66 / 75, 470 KB 83 / 85 (one row after another 96 / 86), 940 KB 167 / 153.
+constexpr size_t SMALL_UP = (size_t)1 << 20, SMALL_DOWN = (size_t)400 << 10;
 
 // rows of T values to and from the interleaved order (K known: the rows are walked together)
 template <int K, typename S>
@@ -326,7 +343,7 @@ static int small_transfer(Ctx *ctx, bool to_host, void *rows, bool f32, int64_t 
 
 int rows_to_host(Ctx *ctx, const void *rows, bool f32, int64_t T, int64_t ld, int K, double *host,
                  bool interleaved) {
-    if (sizeof(double) * (size_t)ld * K <= SMALL_BYTES)
+    if (sizeof(double) * (size_t)ld * K <= SMALL_DOWN)
         return small_transfer(ctx, true, const_cast<void *>(rows), f32, T, ld, K, host, interleaved);
     const int il = interleaved ? 1 : 0;
     return staged_transfer(
@@ -342,7 +359,7 @@ int rows_to_host(Ctx *ctx, const void *rows, bool f32, int64_t T, int64_t ld, in
 
 int rows_from_host(Ctx *ctx, const double *host, bool interleaved, void *rows, bool f32,
                    int64_t T, int64_t ld, int K) {
-    if (sizeof(double) * (size_t)ld * K <= SMALL_BYTES)
+    if (sizeof(double) * (size_t)ld * K <= SMALL_UP)
         return small_transfer(ctx, false, rows, f32, T, ld, K, const_cast<double *>(host), interleaved);
     const int il = interleaved ? 1 : 0;
     return staged_transfer(
