@@ -3,10 +3,11 @@
 //
 // The graph kernels take three launches per iteration and gather gamma_{i-1} and d_{i-1} of 14
 // neighbours per node through branches and 64-bit index arithmetic: 36 us on 60 frames of
-// 64 x 48, K = 3, FP64 (here 10.7), 60 on 100 frames of 64 x 64 (14.1).  Here a workgroup owns a
-// brick of bx x by x bt nodes; gamma and d of the brick and of the nodes around it lie in LDS, q and
-// the node's place in registers, up to NPT nodes a thread.  What is left at 60 frames, us: node pass 2.2,
-// edges 0.9, gamma 0.6 (LDS reads and FP64 issue), exchange of d 2, sums and step 4.  An iteration
+// 64 x 48, K = 3, FP64 (here 9.3 in a long launch), 60 on 100 frames of 64 x 64 (12.5).  Here a
+// workgroup owns a brick of bx x by x bt nodes; gamma and d of the brick and of the nodes around it
+// lie in LDS, q and the node's place in registers, up to NPT nodes a thread.  What is left at 60
+// frames, us: node pass 2.2, edges 0.9, gamma 0.6 (LDS reads and FP64 issue), exchange of d 2, sums
+// and step 4.  An iteration
 //   1. advances gamma on the brick and around it, gamma_i = gamma_{i-1} + beta d_{i-1};
 //   2. forms g_i and d_i of the brick and publishes d_i of its outer nodes;
 //   3. takes the d_i around it from the bricks that own them (sets and marks as in img_loop.h) and

@@ -8,7 +8,7 @@
 // the adjacent lanes, rows above and below from registers or, between waves, LDS; no node is
 // computed twice.  us per iteration, image pass / here (FP64): 250 x 150, K = 2 13.4 / 5.3;
 // 512 x 512, K = 3 16.4 / 7.9; 1024 x 1024, K = 2 / 3 / 4 19.7 / 23.7 / 29.5 against 9.7 / 12.1 /
-// 15.5 (FP32, K = 4: 25 / 9.2); 300 x 200, K = 8 36 / 8.8.  Issue bounds the large ones (270 - 370
+// 15.5 (FP32, K = 4: 25 / 12.4); 300 x 200, K = 8 36 / 8.8.  Issue bounds the large ones (270 - 370
 // instructions a row, two waves per SIMD), the two exchanges (~2 us each) the small ones.
 // What the layout costs when left out: a row's q loaded where it is used 16 us of 26 at 1024 x 1024,
 // K = 4; reads of the columns beyond the tile under a lane condition, eight branches a row;
